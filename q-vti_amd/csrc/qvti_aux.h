@@ -83,27 +83,39 @@ static __global__ __launch_bounds__(256) void k_probe(const float* f, long long 
 
 // Q coefficients (cuviscoelas_3D.cu:195-205) in FP64, rounded to FP32.
 // set: 0 P (vp, gp), 1 S (vs, gs), 2 H (vp*sqrt(1+2eps), gp), 3 D (v_delta, gp).
-// The tau terms act on dv = v - v_prev, so they carry the 1/dt of the
-// reference's (V - V_prev)/dt.
+// The reference's five terms act on A1 v, v, A3 v, A1 dv and dv, dv = v -
+// v_prev (the tau terms carry the 1/dt of its (V - V_prev)/dt).  With c =
+// v cos(pi g/2), M = rho c^2 they are
+//   o0 = -rho c g w0, o1 = M, o2 = rho c^3 g / w0, o3 = rho c g pi / dt,
+//   o4 = M g^2 pi / (w0 dt).
+// o3 / o0 = -pi / (w0 dt) = kappa is one constant of the run, and A1 is
+// linear, so with the field w = alpha (v + kappa dv)
+//   o0 A1 v + o3 A1 dv = (o0 / alpha) A1 w,
+//   o1 v + o4 dv       = (o1 - o4 / kappa) v + (o4 / (alpha kappa)) w,
+// o4 / kappa = -M g^2: four terms per moduli set instead of five, exactly,
+// and A1 acts on w alone.  alpha and the length scale L of A1 = 1/(L |k|) and
+// A3 = L |k| are powers of two (they only shift exponents) that keep w and
+// A3 v below v up to five times the dominant frequency: v, whose coefficient
+// is the largest by far, then takes no rounding from the field that shares a
+// complex transform with it, and the others' coefficients are of order g.
+//   o[0] = L o0 / alpha (A1 w), o[1] = M (1 + g^2) (v),
+//   o[2] = o2 / L (A3 v),       o[3] = -M g^2 / alpha (w)
 // media (qvti_set_media, the reference's media_type, viscoelas_3D.cpp:57-60):
-// 0 viscoelastic (as above); 1 dispersion only (tau terms dropped); 2
-// lossless (gamma = 0); 3 Q-compensating (tau terms negated: the amplitude
-// loss becomes a gain of the same size, the dispersion is kept).
-__device__ __forceinline__ void q_coeffs(double rho, double v, double g, double w0, double dt, int media, double* o)
+// 0 viscoelastic (as above); 1 dispersion only (tau terms dropped: kappa = 0,
+// w = v, no fourth term); 2 lossless (gamma = 0); 3 Q-compensating (tau terms
+// negated: the amplitude loss becomes a gain of the same size, the dispersion
+// is kept; kappa changes sign, the four coefficients do not).
+__device__ __forceinline__ void q_coeffs(double rho, double v, double g, double w0, double alpha, double L, int media,
+                                         double* o)
 {
     const double pi = 3.1415926;
     if (media == 2) g = 0.0;
     const double c = v * cos(g * pi / 2.0);
-    o[0] = -rho * c * g * w0;
-    o[1] = rho * (c * c);
-    o[2] = rho * pow(c, 3.0) * g / w0;
-    o[3] = rho * c * g * pi / dt;
-    o[4] = rho * (c * c) * (g * g) * pi / w0 / dt;
-    if (media == 1) o[3] = o[4] = 0.0;
-    if (media == 3) {
-        o[3] = -o[3];
-        o[4] = -o[4];
-    }
+    const double M = rho * (c * c), Mg2 = media == 1 ? 0.0 : M * (g * g);
+    o[0] = -rho * c * g * w0 * (L / alpha);
+    o[1] = M + Mg2;
+    o[2] = rho * pow(c, 3.0) * g / w0 / L;
+    o[3] = -Mg2 / alpha;
 }
 
 // (blocked field groups and coefficient group sizes: qvti_layout.h)
@@ -111,34 +123,34 @@ __device__ __forceinline__ void q_coeffs(double rho, double v, double g, double 
 struct CoefArgs {
     long long N;
     int vti, media;
-    double w0, dt;
+    double w0, alpha, L;
     const float *vp, *gp, *vs, *gs, *rho, *eps, *del;
-    float* g1;  // blocked [N/64][15][64]: P, S (S-bar filled by k_averages)
-    float* g2;  // blocked [N/64][10][64]: H, D (VTI only)
+    float* g1;  // blocked [N/64][kG1][64]: P, S (S-bar filled by k_averages)
+    float* g2;  // blocked [N/64][kG2][64]: H, D (VTI only)
 };
 
 static __global__ __launch_bounds__(256) void k_coefficients(CoefArgs a)
 {
     for (long long ip = (long long)blockIdx.x * 256 + threadIdx.x; ip < a.N; ip += (long long)gridDim.x * 256) {
-        double o[5];
+        double o[kFam];
         const double r = a.rho[ip];
-        q_coeffs(r, a.vp[ip], a.gp[ip], a.w0, a.dt, a.media, o);
-        for (int j = 0; j < 5; ++j) a.g1[blk_index(ip, kG1, j)] = (float)o[j];
-        q_coeffs(r, a.vs[ip], a.gs[ip], a.w0, a.dt, a.media, o);
-        for (int j = 0; j < 5; ++j) a.g1[blk_index(ip, kG1, 5 + j)] = (float)o[j];
+        q_coeffs(r, a.vp[ip], a.gp[ip], a.w0, a.alpha, a.L, a.media, o);
+        for (int j = 0; j < kFam; ++j) a.g1[blk_index(ip, kG1, j)] = (float)o[j];
+        q_coeffs(r, a.vs[ip], a.gs[ip], a.w0, a.alpha, a.L, a.media, o);
+        for (int j = 0; j < kFam; ++j) a.g1[blk_index(ip, kG1, kFam + j)] = (float)o[j];
         if (a.vti) {
             const double e = a.eps[ip], dl = a.del[ip], vp = a.vp[ip], vs = a.vs[ip];
             const double vh = e == 0.0 ? vp : vp * sqrt(1.0 + 2.0 * e);
-            q_coeffs(r, vh, a.gp[ip], a.w0, a.dt, a.media, o);
-            for (int j = 0; j < 5; ++j) a.g2[blk_index(ip, kG2, j)] = (float)o[j];
+            q_coeffs(r, vh, a.gp[ip], a.w0, a.alpha, a.L, a.media, o);
+            for (int j = 0; j < kFam; ++j) a.g2[blk_index(ip, kG2, j)] = (float)o[j];
             double vd = vp;
             if (dl != 0.0) {
                 const double c33 = r * vp * vp, c44 = r * vs * vs;
                 const double prod = (c33 - c44) * (c33 * (1.0 + 2.0 * dl) - c44);
                 vd = sqrt((sqrt(prod > 0.0 ? prod : 0.0) + c44) / r);
             }
-            q_coeffs(r, vd, a.gp[ip], a.w0, a.dt, a.media, o);
-            for (int j = 0; j < 5; ++j) a.g2[blk_index(ip, kG2, 5 + j)] = (float)o[j];
+            q_coeffs(r, vd, a.gp[ip], a.w0, a.alpha, a.L, a.media, o);
+            for (int j = 0; j < kFam; ++j) a.g2[blk_index(ip, kG2, kFam + j)] = (float)o[j];
         }
     }
 }
@@ -149,7 +161,7 @@ struct AvgArgs {
     int nx, ny, nz;
     long long sx, sy, N;
     float dt;
-    float* g1;       // coefficient group 1: reads S (fields 5-9), writes S-bar (10-14)
+    float* g1;       // coefficient group 1: reads S (fields 4-7), writes S-bar (8-11)
     const float* rho;
     float* buoy;     // [3][N]
 };
@@ -161,15 +173,15 @@ static __global__ __launch_bounds__(256) void k_averages(AvgArgs a)
         const int iy = (int)((ip - (long long)ix * a.sx) / a.sy);
         const int iz = (int)(ip - (long long)ix * a.sx - (long long)iy * a.sy);
         const bool in = ix < a.nx - 1 && iy < a.ny - 1 && iz < a.nz - 1;
-        for (int j = 0; j < 5; ++j) {
-            auto c = [&](long long q) { return a.g1[blk_index(q, kG1, 5 + j)]; };
+        for (int j = 0; j < kFam; ++j) {
+            auto c = [&](long long q) { return a.g1[blk_index(q, kG1, kFam + j)]; };
             float v = 0.f;
             if (in) {
                 const float s8 = c(ip) + c(ip + 1) + c(ip + a.sy) + c(ip + 1 + a.sy) + c(ip + a.sx) + c(ip + a.sx + 1)
                                + c(ip + a.sx + a.sy) + c(ip + a.sx + 1 + a.sy);
                 v = 0.125f * s8;
             }
-            a.g1[blk_index(ip, kG1, 10 + j)] = v;
+            a.g1[blk_index(ip, kG1, 2 * kFam + j)] = v;
         }
         // rho + rho' is an FP32 sum in the reference, the rest FP64
         const float r = a.rho[ip];

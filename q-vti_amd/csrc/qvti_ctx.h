@@ -38,12 +38,15 @@ struct qvti_ctx {
     const LenOps* ops[3] = {nullptr, nullptr, nullptr};  // kernels of the x, y, z lengths
     int split[3] = {0, 0, 0};                            // their split variants (len_ops)
     // model
-    float* coef = nullptr;  // blocked coefficient groups G1 (15 fields) then G2 (10, VTI)
+    float* coef = nullptr;  // blocked coefficient groups G1 (12 fields) then G2 (8, VTI)
     float* buoy = nullptr;  // [3][N]
     bool has_model = false;
     int media = 0;  // QVTI_MEDIA_*: applied by the next qvti_set_model
+    double alpha = 1.0, kappa = 0.0;  // w = alpha (v + kappa dv) of the current model's medium (q_coeffs)
+    double L = 1.0;                   // length scale of A1 and A3
+    float* d_wab = nullptr;           // {alpha, alpha kappa} on the device
     // state, field-major [field][shot][N]
-    float *v = nullptr, *sig = nullptr, *dv = nullptr, *H = nullptr, *bufA = nullptr, *bufB = nullptr;
+    float *v = nullptr, *sig = nullptr, *w = nullptr, *H = nullptr, *bufA = nullptr, *bufB = nullptr;
     float *phiv[3] = {nullptr, nullptr, nullptr}, *phis[3] = {nullptr, nullptr, nullptr};
     long long slab[3] = {0, 0, 0};
     int nphis[3] = {5, 5, 4};
@@ -102,7 +105,7 @@ struct qvti_ctx {
     // opt-in k-space correction / wavenumber filter (off: the reference scheme)
     bool ks = false;
     float ks_vref = 0.f, ks_fcut = 0.f, ks_vmax = 0.f, ks_taper = 0.f;
-    float* H2 = nullptr;  // [A2 v x,y,z][A2 dv x,y,z], allocated on first use
+    float* H2 = nullptr;  // [A2 v x,y,z][A2 w x,y,z], allocated on first use
     long long bytes = 0;
     std::vector<void*> allocs;
 };

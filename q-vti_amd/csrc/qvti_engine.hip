@@ -190,7 +190,11 @@ static void release(qvti_ctx* c)
 }
 
 // ------------------------------------------------------- sizes / memory --
-static long long state_fields() { return 3 + 6 + 3 + 9 + 15 + 15; }
+// Fields per shot of each scratch buffer (bufA, bufB): the 12 derivatives of
+// the stress family along x and y; the spectra they held before take 8 and
+// 6 (12 in k-space mode).
+constexpr int kBufFields = 3 * kFam;
+static long long state_fields() { return 3 + 6 + 3 + 6 + kBufFields + kBufFields; }
 
 extern "C" long long qvti_estimate_bytes(const qvti_grid* g, int max_shots)
 {
@@ -198,7 +202,7 @@ extern "C" long long qvti_estimate_bytes(const qvti_grid* g, int max_shots)
     const long long N = (long long)g->nx * g->ny * g->nz;
     const long long p2 = 2LL * g->pml;
     const long long slabs = 8LL * (p2 * g->ny * g->nz + (long long)g->nx * p2 * g->nz) + 7LL * g->nx * g->ny * p2;
-    const long long model = (g->vti ? 20 : 10) + 5 + 3;
+    const long long model = kG1 + (g->vti ? kG2 : 0) + 3;
     return 4LL * (N * (state_fields() * max_shots + model) + slabs * max_shots) + (64LL << 20);
 }
 
@@ -280,6 +284,9 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
         c->snap_hi[a] = dims[a] - g->pml;
     }
     c->nrows = (long long)g->nx * g->ny;
+    // 1 / |k| of five times the dominant frequency at 3000 m/s, as a power of
+    // two: A3 v = L |k| v stays below v, with which it shares a transform
+    c->L = exp2(round(log2(3000.0 / (5.0 * 2.0 * M_PI * (double)g->f0))));
     // When a z row does not end on a 128-byte line, neighbouring row tiles
     // and neighbouring planes share lines (and 64-cell blocks): run 8 row
     // tiles and 2 planes per XCD so those are fetched once.  Measured at
@@ -326,15 +333,16 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
     rc = rc ? rc : dalloc(c, (void**)&c->buoy, sizeof(float) * 3 * N);
     rc = rc ? rc : dalloc(c, (void**)&c->v, sizeof(float) * 3 * S * N);
     rc = rc ? rc : dalloc(c, (void**)&c->sig, sizeof(float) * 6 * S * N);
-    rc = rc ? rc : dalloc(c, (void**)&c->dv, sizeof(float) * 3 * S * N);
-    rc = rc ? rc : dalloc(c, (void**)&c->H, sizeof(float) * 9 * S * N);
-    rc = rc ? rc : dalloc(c, (void**)&c->bufA, sizeof(float) * 15 * S * Nb);
-    rc = rc ? rc : dalloc(c, (void**)&c->bufB, sizeof(float) * 15 * S * Nb);
+    rc = rc ? rc : dalloc(c, (void**)&c->w, sizeof(float) * 3 * S * N);
+    rc = rc ? rc : dalloc(c, (void**)&c->H, sizeof(float) * 6 * S * N);
+    rc = rc ? rc : dalloc(c, (void**)&c->bufA, sizeof(float) * kBufFields * S * Nb);
+    rc = rc ? rc : dalloc(c, (void**)&c->bufB, sizeof(float) * kBufFields * S * Nb);
     for (int a = 0; a < 3 && !rc; ++a) {
         rc = dalloc(c, (void**)&c->phiv[a], sizeof(float) * 3 * S * c->slab[a]);
         rc = rc ? rc : dalloc(c, (void**)&c->phis[a], sizeof(float) * c->nphis[a] * S * c->slab[a]);
     }
     rc = rc ? rc : dalloc(c, (void**)&c->d_it, sizeof(int));
+    rc = rc ? rc : dalloc(c, (void**)&c->d_wab, 2 * sizeof(float));
     rc = rc ? rc : dalloc(c, (void**)&c->d_probe, sizeof(int));
     rc = rc ? rc : dalloc(c, (void**)&c->d_src_kind, sizeof(int) * S);
     rc = rc ? rc : dalloc(c, (void**)&c->d_src_ip, sizeof(long long) * S);
@@ -374,7 +382,7 @@ static int build_launch_config(qvti_ctx* c)
 
     float* acc[3] = {fld(c->bufA, 0, c), fld(c->bufA, 1, c), fld(c->bufA, 2, c)};
     float* vv[3] = {fld(c->v, 0, c), fld(c->v, 1, c), fld(c->v, 2, c)};
-    float* dvv[3] = {fld(c->dv, 0, c), fld(c->dv, 1, c), fld(c->dv, 2, c)};
+    float* ww[3] = {fld(c->w, 0, c), fld(c->w, 1, c), fld(c->w, 2, c)};
     // sig order: pxx pyy pzz pxy pxz pyz
     float* sg[6];
     for (int k = 0; k < 6; ++k) sg[k] = fld(c->sig, k, c);
@@ -422,16 +430,11 @@ static int build_launch_config(qvti_ctx* c)
     vy.job[2] = job(pyz, acc[2], acc[2], nullptr, 0, 0);
     for (int k = 0; k < 3; ++k) vy.job[k].phi = c->phiv[1] + (long long)k * c->S * c->slab[1];
 
-    // ---- 3-D transform buffers: P_c = FFT(v_c + i dv_c) (bufB as complex),
-    // Q1_c, Q3_c (bufA as complex)
+    // ---- 3-D transform buffers: P (bufB as complex), Q1, Q3 (bufA as complex)
     float2* P[3];
-    float2* Q1[3];
-    float2* Q3[3];
-    for (int k = 0; k < 3; ++k) {
-        P[k] = reinterpret_cast<float2*>(fld(c->bufB, 2 * k, c));
-        Q1[k] = reinterpret_cast<float2*>(fld(c->bufA, 2 * k, c));
-        Q3[k] = reinterpret_cast<float2*>(fld(c->bufA, 6 + 2 * k, c));
-    }
+    float2* Q[4];
+    for (int k = 0; k < 3; ++k) P[k] = reinterpret_cast<float2*>(fld(c->bufB, 2 * k, c));
+    for (int k = 0; k < 4; ++k) Q[k] = reinterpret_cast<float2*>(fld(c->bufA, 2 * k, c));
     // ---- velocity z + update + forward z-FFT: pxz (D+) -> vx, pyz (D+) -> vy, pzz (D-, half) -> vz
     VelZArgs& vz = c->a_vz;
     vz.nx = nx; vz.ny = ny; vz.nz = nz; vz.pml = g.pml;
@@ -445,11 +448,12 @@ static int build_launch_config(qvti_ctx* c)
     for (int k = 0; k < 3; ++k) {
         vz.acc[k] = acc[k];
         vz.v[k] = vv[k];
-        vz.dv[k] = dvv[k];
+        vz.w[k] = ww[k];
         vz.P[k] = P[k];
         vz.buoy[k] = c->buoy + (long long)k * N;
         vz.phi[k] = c->phiv[2] + (long long)k * c->S * c->slab[2];
     }
+    vz.wab = c->d_wab;
     vz.src_kind = c->d_src_kind;
     vz.src_ip = c->d_src_ip;
     vz.rik = nullptr;  // set at begin
@@ -459,14 +463,12 @@ static int build_launch_config(qvti_ctx* c)
     vz.nshots = 1;
     c->g_zr = c->g_vz;
 
-    // H: [A1 v x,y,z][A1 dv x,y,z][A3 v x,y,z]
-    float* H1v[3];
-    float* H1dv[3];
+    // H: [A1 w x,y,z][A3 v x,y,z]
+    float* H1w[3];
     float* H3v[3];
     for (int k = 0; k < 3; ++k) {
-        H1v[k] = fld(c->H, k, c);
-        H1dv[k] = fld(c->H, 3 + k, c);
-        H3v[k] = fld(c->H, 6 + k, c);
+        H1w[k] = fld(c->H, k, c);
+        H3v[k] = fld(c->H, 3 + k, c);
     }
     CStridedArgs& yf = c->a_yf;
     yf.nz = nz; yf.sx = sx; yf.sy = sy;
@@ -487,24 +489,25 @@ static int build_launch_config(qvti_ctx* c)
     xp.tw = X.tw;
     xp.kfx = X.kf; xp.kfy = Y.kf; xp.kfz = Z.kf;
     xp.invN = 1.0 / (double)N;
+    xp.invN1 = xp.invN / c->L;
+    xp.invN3 = xp.invN * c->L;
     xp.ncomp = 3;
-    // P0 = F(vx + i vy), P1 = F(dvx + i dvy), P2 = F(vz + i dvz): A1 on all
-    // three, |k| on P0 and P2 (A3 vx + i A3 vy, A3 vz + i unused)
-    for (int k = 0; k < 3; ++k) { xp.P[k] = P[k]; xp.Q1[k] = Q1[k]; }
-    xp.Q3[0] = Q3[0];
-    xp.Q3[1] = nullptr;
-    xp.Q3[2] = Q3[1];
+    // P0 = F(wx + i wy), P1 = F(wz + i vz), P2 = F(vx + i vy): A1 on P0 and
+    // P1, A3 on P1 and P2 (A1 wz + i unused, unused + i A3 vz)
+    for (int k = 0; k < 3; ++k) xp.P[k] = P[k];
+    xp.Q1[0] = Q[0]; xp.Q1[1] = Q[1]; xp.Q1[2] = nullptr;
+    xp.Q3[0] = nullptr; xp.Q3[1] = Q[2]; xp.Q3[2] = Q[3];
     // k-space mode: A2 F P_c -> Q2_c in bufB fields 6-11 (free once the
     // x-pass has read P; the y-derivatives overwrite them after z_inv)
     float2* Q2[3] = {nullptr, nullptr, nullptr};
     float* H2v[3] = {nullptr, nullptr, nullptr};
-    float* H2dv[3] = {nullptr, nullptr, nullptr};
+    float* H2w[3] = {nullptr, nullptr, nullptr};
     xp.ks_vh = xp.ks_k0 = xp.ks_kc = xp.ks_pw = 0.f;
     if (c->ks) {
         for (int k = 0; k < 3; ++k) {
             Q2[k] = reinterpret_cast<float2*>(fld(c->bufB, 6 + 2 * k, c));
             H2v[k] = fld(c->H2, k, c);
-            H2dv[k] = fld(c->H2, 3 + k, c);
+            H2w[k] = fld(c->H2, 3 + k, c);
             xp.Q2[k] = Q2[k];
         }
         xp.ks_vh = (float)(0.5 * (double)c->ks_vref * (double)g.dt);
@@ -519,13 +522,11 @@ static int build_launch_config(qvti_ctx* c)
 
     CStridedArgs& yi = c->a_yi;
     yi = yf;
-    yi.nfields = 5;
-    for (int k = 0; k < 3; ++k) yi.f[k] = Q1[k];
-    yi.f[3] = Q3[0];
-    yi.f[4] = Q3[1];
+    yi.nfields = 4;
+    for (int k = 0; k < 4; ++k) yi.f[k] = Q[k];
     if (c->ks) {
-        yi.nfields = 8;
-        for (int k = 0; k < 3; ++k) yi.f[5 + k] = Q2[k];
+        yi.nfields = 7;
+        for (int k = 0; k < 3; ++k) yi.f[4 + k] = Q2[k];
     }
 
     ZRowsArgs& zi = c->a_zi;
@@ -534,56 +535,58 @@ static int build_launch_config(qvti_ctx* c)
     zi.tw = Z.tw;
     zi.mode = 1;
     zi.dir = 1;
-    zi.nfields = 5;
-    zi.cin[0] = Q1[0]; zi.re_out[0] = H1v[0]; zi.im_out[0] = H1v[1];    // A1 vx, A1 vy
-    zi.cin[1] = Q1[1]; zi.re_out[1] = H1dv[0]; zi.im_out[1] = H1dv[1];  // A1 dvx, A1 dvy
-    zi.cin[2] = Q1[2]; zi.re_out[2] = H1v[2]; zi.im_out[2] = H1dv[2];   // A1 vz, A1 dvz
-    zi.cin[3] = Q3[0]; zi.re_out[3] = H3v[0]; zi.im_out[3] = H3v[1];    // A3 vx, A3 vy
-    zi.cin[4] = Q3[1]; zi.re_out[4] = H3v[2]; zi.im_out[4] = nullptr;   // A3 vz
+    zi.nfields = 4;
+    for (int k = 0; k < 4; ++k) zi.cin[k] = Q[k];
+    zi.re_out[0] = H1w[0]; zi.im_out[0] = H1w[1];  // A1 wx, A1 wy
+    zi.re_out[1] = H1w[2]; zi.im_out[1] = nullptr; // A1 wz
+    zi.re_out[2] = nullptr; zi.im_out[2] = H3v[2]; // A3 vz
+    zi.re_out[3] = H3v[0]; zi.im_out[3] = H3v[1];  // A3 vx, A3 vy
     if (c->ks) {
-        zi.nfields = 8;
-        zi.cin[5] = Q2[0]; zi.re_out[5] = H2v[0]; zi.im_out[5] = H2v[1];    // A2 vx, A2 vy
-        zi.cin[6] = Q2[1]; zi.re_out[6] = H2dv[0]; zi.im_out[6] = H2dv[1];  // A2 dvx, A2 dvy
-        zi.cin[7] = Q2[2]; zi.re_out[7] = H2v[2]; zi.im_out[7] = H2dv[2];   // A2 vz, A2 dvz
+        zi.nfields = 7;
+        zi.cin[4] = Q2[0]; zi.re_out[4] = H2w[0]; zi.im_out[4] = H2w[1];  // A2 wx, A2 wy
+        zi.cin[5] = Q2[1]; zi.re_out[5] = H2w[2]; zi.im_out[5] = H2v[2];  // A2 wz, A2 vz
+        zi.cin[6] = Q2[2]; zi.re_out[6] = H2v[0]; zi.im_out[6] = H2v[1];  // A2 vx, A2 vy
     }
 
-    // ---- stress x / y derivatives of the 15 family fields
-    const float* fam[3][5];
+    // ---- stress x / y derivatives of the 12 family fields
+    const float* fam[3][kFam];
     for (int k = 0; k < 3; ++k) {
-        fam[k][0] = H1v[k]; fam[k][1] = vv[k]; fam[k][2] = H3v[k]; fam[k][3] = H1dv[k]; fam[k][4] = dvv[k];
-        if (c->ks) { fam[k][1] = H2v[k]; fam[k][4] = H2dv[k]; }
+        fam[k][0] = H1w[k]; fam[k][1] = vv[k]; fam[k][2] = H3v[k]; fam[k][3] = ww[k];
+        if (c->ks) { fam[k][1] = H2v[k]; fam[k][3] = H2w[k]; }
     }
-    // x/y derivatives of the stress step: blocked groups of 15 fields per
-    // shot in bufA (x) and bufB (y); job k writes field k of the group
-    float* DX[15];
-    float* DY[15];
-    // x-derivatives: three blocked groups of 5 (ex, gx, hx), each [shot][N/64][5][64];
-    // y-derivatives: one blocked group of 15
-    for (int k = 0; k < 15; ++k) {
-        DX[k] = c->bufA + (long long)(k / 5) * 5 * c->S * c->Nb + (long long)(k % 5) * kBlk;
+    // x/y derivatives of the stress step: blocked groups in bufA (x) and bufB
+    // (y); job k writes field k of the group.
+    // x-derivatives: three blocked groups of 4 (ex, gx, hx), each [shot][N/64][4][64];
+    // y-derivatives: one blocked group of 12
+    float* DX[3 * kFam];
+    float* DY[3 * kFam];
+    for (int k = 0; k < 3 * kFam; ++k) {
+        DX[k] = c->bufA + (long long)(k / kFam) * kFam * c->S * c->Nb + (long long)(k % kFam) * kBlk;
         DY[k] = c->bufB + (long long)k * kBlk;
     }
     StridedArgs& sxa = c->a_sx;
     strided_common(sxa, 0, Px);
     sxa.mode = MODE_STORE;
-    sxa.njobs = 15;
-    sxa.bnf = 5;
+    sxa.njobs = 3 * kFam;
+    sxa.bnf = kFam;
     sxa.blk_stride = c->Nb;
-    for (int j = 0; j < 5; ++j) {
-        sxa.job[j] = job(fam[0][j], DX[j], nullptr, nullptr, 0, 0);          // ex: dx vx-family, D+
-        sxa.job[5 + j] = job(fam[2][j], DX[5 + j], nullptr, nullptr, 1, 0);   // gx: dx vz-family, D-
-        sxa.job[10 + j] = job(fam[1][j], DX[10 + j], nullptr, nullptr, 1, 0); // hx: dx vy-family, D-
+    for (int j = 0; j < kFam; ++j) {
+        const int g = kFam + j, h = 2 * kFam + j;
+        sxa.job[j] = job(fam[0][j], DX[j], nullptr, nullptr, 0, 0);  // ex: dx vx-family, D+
+        sxa.job[g] = job(fam[2][j], DX[g], nullptr, nullptr, 1, 0);  // gx: dx vz-family, D-
+        sxa.job[h] = job(fam[1][j], DX[h], nullptr, nullptr, 1, 0);  // hx: dx vy-family, D-
     }
     StridedArgs& sya = c->a_sy;
     strided_common(sya, 1, Py);
     sya.mode = MODE_STORE;
-    sya.njobs = 15;
-    sya.bnf = kG1;
+    sya.njobs = 3 * kFam;
+    sya.bnf = 3 * kFam;
     sya.blk_stride = c->Nb;
-    for (int j = 0; j < 5; ++j) {
-        sya.job[j] = job(fam[1][j], DY[j], nullptr, nullptr, 0, 0);          // ey: dy vy-family, D+
-        sya.job[5 + j] = job(fam[2][j], DY[5 + j], nullptr, nullptr, 1, 0);   // gy: dy vz-family, D-
-        sya.job[10 + j] = job(fam[0][j], DY[10 + j], nullptr, nullptr, 1, 0); // hy: dy vx-family, D-
+    for (int j = 0; j < kFam; ++j) {
+        const int g = kFam + j, h = 2 * kFam + j;
+        sya.job[j] = job(fam[1][j], DY[j], nullptr, nullptr, 0, 0);  // ey: dy vy-family, D+
+        sya.job[g] = job(fam[2][j], DY[g], nullptr, nullptr, 1, 0);  // gy: dy vz-family, D-
+        sya.job[h] = job(fam[0][j], DY[h], nullptr, nullptr, 1, 0);  // hy: dy vx-family, D-
     }
 
     // ---- stress z + update
@@ -598,9 +601,9 @@ static int build_launch_config(qvti_ctx* c)
     sz.pay = Y.a; sz.pby = Y.b; sz.payh = Y.ah; sz.pbyh = Y.bh;
     sz.paz = Z.a; sz.pbz = Z.b; sz.pazh = Z.ah; sz.pbzh = Z.bh;
     for (int k = 0; k < 3; ++k)
-        for (int j = 0; j < 5; ++j) sz.fam[k][j] = fam[k][j];
+        for (int j = 0; j < kFam; ++j) sz.fam[k][j] = fam[k][j];
     sz.dxb = c->bufA;
-    sz.dx_group = 5LL * c->S * c->Nb;
+    sz.dx_group = (long long)kFam * c->S * c->Nb;
     sz.blk_stride = c->Nb;
     sz.dyb = c->bufB;
     sz.g1 = c->coef;
@@ -642,13 +645,28 @@ extern "C" int qvti_set_model(qvti_ctx* c, const float* velp, const float* gama_
     HIPCHK(hipSetDevice(c->device));
     const long long N = c->N;
     const size_t B = sizeof(float) * N;
-    // The model is staged in the spectral scratch buffer (15 fields per shot,
+    // The model is staged in the spectral scratch buffer (kBufFields per shot,
     // free between runs and ordered on the context's stream), so setting a
     // model allocates nothing and never waits for other contexts' work.
     float* tmp = c->bufA;
     const int nin = c->g.vti ? 7 : 5;
     const float* srcs[7] = {velp, gama_p, vels, gama_s, rho, eps, delta};
+    // w = alpha (v + kappa dv), kappa dv being pi f / f_ref times v at the
+    // frequency f (w0 = 2 pi f_ref).  alpha scales w to the size of v at 5 f0,
+    // the top of a pulse's spectrum: in the transforms that carry both, the
+    // rounding of w then stays below that of v, and w itself enters the
+    // stresses with the small Q coefficients only (measured, 160x160x128,
+    // k-space mode, records against FP64: 3.2e-7 with alpha set at f0)
+    c->kappa = c->media == QVTI_MEDIA_DISPERSION || c->media == QVTI_MEDIA_LOSSLESS
+                   ? 0.0
+                   : -kRefPi / ((double)c->g.w0 * (double)c->g.dt);
+    if (c->media == QVTI_MEDIA_QCOMP) c->kappa = -c->kappa;
+    const double tilt = c->kappa == 0.0 ? 0.0 : 5.0 * 2.0 * M_PI * M_PI * (double)c->g.f0 / (double)c->g.w0;
+    c->alpha = exp2(-round(log2(sqrt(1.0 + tilt * tilt))));
+    const float wab[2] = {(float)c->alpha, (float)(c->alpha * c->kappa)};
     int rc = QVTI_OK;
+    if (hipMemcpyAsync(c->d_wab, wab, sizeof wab, hipMemcpyHostToDevice, c->stream) != hipSuccess)
+        rc = qvti_fail(QVTI_E_DEVICE, "model upload failed");
     for (int k = 0; k < nin && !rc; ++k)
         if (hipMemcpyAsync(tmp + k * N, srcs[k], B, hipMemcpyHostToDevice, c->stream) != hipSuccess)
             rc = qvti_fail(QVTI_E_DEVICE, "model upload failed");
@@ -658,7 +676,8 @@ extern "C" int qvti_set_model(qvti_ctx* c, const float* velp, const float* gama_
         ca.vti = c->g.vti;
         ca.media = c->media;
         ca.w0 = (double)c->g.w0;
-        ca.dt = (double)c->g.dt;
+        ca.alpha = c->alpha;
+        ca.L = c->L;
         ca.vp = tmp; ca.gp = tmp + N; ca.vs = tmp + 2 * N; ca.gs = tmp + 3 * N; ca.rho = tmp + 4 * N;
         ca.eps = c->g.vti ? tmp + 5 * N : nullptr;
         ca.del = c->g.vti ? tmp + 6 * N : nullptr;
@@ -797,8 +816,8 @@ static int class_fields(const qvti_ctx* c, int cls)
 {
     switch (cls) {
     case KC_VEL_X: case KC_VEL_Y: case KC_Y_FWD: case KC_XPASS: return 3;
-    case KC_Y_INV: return c->a_yi.nfields;  // 5, or 8 in k-space mode
-    case KC_STR_X: case KC_STR_Y: return 15;
+    case KC_Y_INV: return c->a_yi.nfields;  // 4, or 7 in k-space mode
+    case KC_STR_X: case KC_STR_Y: return 3 * kFam;
     default: return 1;
     }
 }
@@ -1124,7 +1143,7 @@ extern "C" int qvti_finish(qvti_ctx* c, float* rec_vx, float* rec_vy, float* rec
 // ------------------------------------------------------ checkpoint ------
 // Image of a run in progress: header, then for shots [0, nshots) the fields
 // that carry from one step to the next (v, sig, the C-PML slabs), the records
-// gathered so far and the snapshots taken so far.  dv, the spectral buffers
+// gathered so far and the snapshots taken so far.  w, the spectral buffers
 // and the derivative buffers are rebuilt inside every step.
 namespace {
 struct CkptHeader {
@@ -1713,21 +1732,21 @@ extern "C" int qvti_kernel_bytes(qvti_ctx* c, int max_classes, double* bytes)
     const double N = (double)c->N * std::max(1, c->nshots), f = 4.0 * N;
     const double slab = (double)std::max(1, c->nshots) * 4.0;
     const double sx = c->slab[0] * slab, sy = c->slab[1] * slab, sz = c->slab[2] * slab;
-    const int ncoef = c->g.vti ? 25 : 15;
+    const int ncoef = kG1 + (c->g.vti ? kG2 : 0);
     double b[KC_COUNT] = {};
     b[KC_TICK] = 8;
     b[KC_VEL_X] = 6 * f + 3 * 2 * sx;
     b[KC_VEL_Y] = 9 * f + 3 * 2 * sy;
-    b[KC_VEL_Z] = (3 + 3 + 3 + 3 + 3 + 6) * f + 3.0 * 4 * c->N + 3 * 2 * sz;  // sig, acc, v r/w, dv, P, buoy
+    b[KC_VEL_Z] = (3 + 3 + 3 + 3 + 3 + 6) * f + 3.0 * 4 * c->N + 3 * 2 * sz;  // sig, acc, v r/w, w, P, buoy
     b[KC_Y_FWD] = 12 * f;
     // k-space mode: three more complex spectra through the x-pass, y-inverse
     // and z-inverse, six more real fields out
-    b[KC_XPASS] = 6 * f + (c->ks ? 16 : 10) * f;
-    b[KC_Y_INV] = (c->ks ? 32 : 20) * f;
-    b[KC_Z_INV] = c->ks ? 16 * f + 15 * f : 10 * f + 9 * f;
-    b[KC_STR_X] = 30 * f;
-    b[KC_STR_Y] = 30 * f;
-    b[KC_STR_Z] = (15 + 30 + 12) * f + ncoef * 4.0 * c->N + 2 * (5 * sx + 5 * sy + 4 * sz);
+    b[KC_XPASS] = 6 * f + (c->ks ? 14 : 8) * f;
+    b[KC_Y_INV] = (c->ks ? 28 : 16) * f;
+    b[KC_Z_INV] = c->ks ? 14 * f + 12 * f : 8 * f + 6 * f;
+    b[KC_STR_X] = 24 * f;
+    b[KC_STR_Y] = 24 * f;
+    b[KC_STR_Z] = (12 + 24 + 12) * f + ncoef * 4.0 * c->N + 2 * (5 * sx + 5 * sy + 4 * sz);
     b[KC_RECORD] = 6.0 * 4 * c->total_rec;
     const int n = std::min(max_classes, (int)KC_COUNT);
     for (int k = 0; k < n; ++k) bytes[k] = b[k];

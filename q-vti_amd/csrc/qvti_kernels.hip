@@ -38,7 +38,7 @@ void l_zrows(dim3 grid, hipStream_t st, const ZRowsArgs& a)
 template <class G, bool VTI>
 void l_stress_z(dim3 grid, hipStream_t st, const StressZArgs& a)
 {
-    hipLaunchKernelGGL((k2_stress_z<G, VTI>), grid, dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL((k2_stress_z<G, VTI>), grid, dim3(StressTile<G>::T), 0, st, a);
 }
 template <class G>
 void l_deriv_rows(dim3 grid, hipStream_t st, const RowDerivArgs& a)

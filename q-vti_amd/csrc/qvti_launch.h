@@ -24,7 +24,7 @@ struct LenOps {
     void (*deriv[3][3])(dim3 grid, hipStream_t st, const StridedArgs& a);  // [MODE_*]
     void (*cfft[2][3])(dim3 grid, hipStream_t st, const CStridedArgs& a);  // [0 forward, 1 inverse]
     void (*xpass[2][3])(dim3 grid, hipStream_t st, const XPassArgs& a);    // [k-space mode off, on]
-    // row (z) kernels, 256 threads
+    // row (z) kernels, 256 threads (stress_z: StressTile)
     void (*vel_z[2])(dim3 grid, hipStream_t st, const VelZArgs& a);  // [without, with extra point sources]
     void (*zrows)(dim3 grid, hipStream_t st, const ZRowsArgs& a);
     void (*stress_z[2])(dim3 grid, hipStream_t st, const StressZArgs& a);  // [isotropic, VTI]

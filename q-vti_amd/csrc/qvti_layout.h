@@ -19,7 +19,11 @@ __host__ __device__ __forceinline__ long long blk_index(long long ip, int nf, in
 {
     return ((ip >> 6) * nf + f) * kBlk + (ip & 63);
 }
-// coefficient groups: G1 = {P 0-4, S 5-9, S-bar 10-14}, G2 = {H 0-4, D 5-9} (VTI)
-constexpr int kG1 = 15, kG2 = 10;
+// Stress family: per velocity component the four fields {A1 w, A2 v, A3 v,
+// A2 w} whose derivatives the stress update weighs with the Q coefficients
+// (k_coefficients in qvti_aux.h).
+constexpr int kFam = 4;
+// coefficient groups: G1 = {P 0-3, S 4-7, S-bar 8-11}, G2 = {H 0-3, D 4-7} (VTI)
+constexpr int kG1 = 3 * kFam, kG2 = 2 * kFam;
 
 }  // namespace qvti

@@ -6,7 +6,7 @@
 // Per step (reference loop: cuviscoelas_3D.cu:1255-1605):
 //   velocity half-step   k2_deriv_strided(x, VEL_FIRST; advances the step counter)
 //                        -> k2_deriv_strided(y, VEL_ACC)
-//                        -> k2_vel_z (z-derivatives, velocity update, forward z-FFT of v + i dv)
+//                        -> k2_vel_z (z-derivatives, velocity update, forward z-FFTs of v and w)
 //   stress half-step     k2_cfft_strided(y, fwd) -> k2_xpass -> k2_cfft_strided(y, inv)
 //                        -> k2_zrows (inverse z) -> k2_deriv_strided(x, STORE) -> k2_deriv_strided(y, STORE)
 //                        -> k2_stress_z (z-derivatives, stress update, source injection)
@@ -22,13 +22,16 @@
 //    derivatives and the A2 = 1 stress terms) is a 1-D transform along that
 //    axis: the other two axes' forward and inverse transforms cancel;
 //  * A_j D_a V = D_a (A_j V): the 45 stress terms are 1-D derivatives of the
-//    15 fields {A1 v, v, A3 v, A1 dv, dv} per component, with dv = v - v_prev
-//    in real space (v_prev: the previous step's pre-injection velocity) and
-//    the 1/dt of the time difference folded into the tau coefficients, so
-//    only A1 (v + i dv) and A3 v need the full 3-D transform.  v and dv are
-//    packed together because their magnitudes are comparable (|dv| ~ w dt |v|);
-//    packing v with dv/dt instead lets the FP32 rounding of the larger part
-//    swamp the smaller one.
+//    12 fields {A1 w, v, A3 v, w} per component, w = alpha (v + kappa dv) with
+//    dv = v - v_prev in real space (v_prev: the previous step's pre-injection
+//    velocity): the coefficients of A1 v and A1 dv are in one ratio kappa
+//    everywhere (q_coeffs in qvti_aux.h), so only A1 w and A3 v need the full
+//    3-D transform - three forward and four inverse complex transforms.  With
+//    five fields {A1 v, v, A3 v, A1 dv, dv} per component it was three and
+//    five, and 248 floats per cell and step through HBM instead of 211 (VTI).
+//    Fields that share a complex transform are scaled (alpha and the length
+//    scale of A1 and A3, powers of two) so that the FP32 rounding of one does
+//    not swamp the other where it matters (q_coeffs).
 #pragma once
 #include "qvti_fft2l.h"
 #include "qvti_layout.h"
@@ -151,7 +154,7 @@ struct StridedArgs {
     long long blk_stride;
     // step counter advanced by this launch (the first kernel of a step), or null
     int* tick;
-    DJob job[15];
+    DJob job[3 * kFam];
 };
 
 template <class G, int MODE>
@@ -299,7 +302,8 @@ void k2_deriv_strided(StridedArgs a)
 // Velocity update (cuviscoelas_3D.cu:1018-1101) fused with the z-derivatives
 // and with the first (z) pass of the stress step's 3-D transform:
 //   v += b * (acc_xy + dz sigma + phi_z);  dv = v_new - v_old + src_prev;
-//   P0 = FFT_z(vx + i vy), P1 = FFT_z(dvx + i dvy), P2 = FFT_z(vz + i dvz)
+//   w = alpha v + (alpha kappa) dv;
+//   P0 = FFT_z(wx + i wy), P1 = FFT_z(wz + i vz), P2 = FFT_z(vx + i vy)
 // dv is the change since the previous step's pre-injection velocity (the
 // reference's V - V_prev, cuviscoelas_3D.cu:517-522, 1124-1131, without 1/dt).
 // Tile: G::P rows (z-pencils).
@@ -315,7 +319,8 @@ struct VelZArgs {
     const float *pxz, *pyz, *pzz;
     const float* acc[3];
     float* v[3];
-    float* dv[3];
+    float* w[3];
+    const float* wab;  // {alpha, alpha kappa}
     float2* P[3];
     const float* buoy[3];
     float* phi[3];  // z-slab: phi_pxz_z (node), phi_pyz_z (node), phi_pzz_z (half)
@@ -333,14 +338,14 @@ struct VelZArgs {
 // Velocity update of one component on the thread's level-1 elements of one
 // row (iz = j + N2*j1), from its z-derivative d (real or imaginary part):
 // C-PML memory variable on the z-slab, v += b * (acc + dz + phi), dv = v_new
-// - v_old (+ the previous step's source at the injection cell).  Writes v and
-// dv (rows with rowdom / ok1 only), returns (v_new, dv).  The pointers are
-// row bases (v, dv, acc, bu: the row; ph: the row's z-slab of 2*pml values)
+// - v_old (+ the previous step's source at the injection cell), w = wa v +
+// wb dv.  Writes v and w (rows with rowdom / ok1 only), returns (v_new, w).
+// The pointers are row bases (v, w, acc, bu: the row; ph: the row's z-slab of 2*pml values)
 // and never alias, which lets the compiler issue the loads of later elements
 // before the stores of earlier ones.
 template <class G, bool INJ>
 __device__ __forceinline__ void vz_component(float2 (&out)[G::N1], const float2 (&d)[G::N1], const bool imag,
-                                             float* __restrict__ v, float* __restrict__ dv,
+                                             float* __restrict__ v, float* __restrict__ w, const float wa, const float wb,
                                              const float* __restrict__ acc, const float* __restrict__ bu,
                                              float* __restrict__ ph, const float* __restrict__ pa,
                                              const float* __restrict__ pb, const int j, const int pml,
@@ -374,7 +379,7 @@ __device__ __forceinline__ void vz_component(float2 (&out)[G::N1], const float2 
         float dvv = vnew - vold;
         if (iz == src_iz) dvv += sprev;
         if constexpr (INJ) dvv += inj[iz];
-        out[j1] = make_float2(vnew, dvv);
+        out[j1] = make_float2(vnew, wa * vnew + wb * dvv);
     }
 #pragma unroll
     for (int jc = 0; jc < CH; ++jc) {
@@ -383,7 +388,7 @@ __device__ __forceinline__ void vz_component(float2 (&out)[G::N1], const float2 
         const bool upd = rowdom && iz < n - 1;
         if (upd && (iz < pml || iz >= n - pml)) ph[iz < pml ? iz : iz - (n - 2 * pml)] = qn[jc];
         if (upd) v[iz] = out[j1].x;
-        if (ok1) dv[iz] = out[j1].y;
+        if (ok1) w[iz] = out[j1].y;
     }
     asm volatile("" ::: "memory");  // the next chunk's loads stay after this chunk
     }
@@ -442,6 +447,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
     const int kind = a.src_kind[shot];
     const long long sip = a.src_ip[shot];
     const float sprev = it > 0 ? a.rik[it - 1] : 0.f;
+    const float wa = a.wab[0], wb = a.wab[1];
     const int ix = (int)(r1 / a.ny), iy = (int)(r1 - (long long)ix * a.ny);
     const bool rowdom = ok1 && ix < a.nx - 1 && iy < a.ny - 1;
     const long long slab_row = (long long)shot * a.slab_stride + r1 * 2 * a.pml;
@@ -451,7 +457,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
         const long long rb = ubase + lrow1;  // row base of this thread's row in the shot's fields
         const int src_iz = (kind == c && sip >= r1 * n && sip < (r1 + 1) * n) ? (int)(sip - r1 * n) : -1;
         const bool h = c == 2;
-        vz_component<G, INJ>(out, d, imag, a.v[c] + rb, a.dv[c] + rb, a.acc[c] + rb,
+        vz_component<G, INJ>(out, d, imag, a.v[c] + rb, a.w[c] + rb, wa, wb, a.acc[c] + rb,
                         a.buoy[c] + (rb - (long long)shot * a.shot_stride),
                         a.phi[c] + (ok1 ? slab_row : (long long)shot * a.slab_stride),
                         h ? a.pah : a.pa, h ? a.pbh : a.pb, j, a.pml, a.dt, rowdom, ok1, src_iz, sprev,
@@ -471,15 +477,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
         }
     };
 
-    // Packing of the stress step's transforms: P0 = F(vx + i vy),
-    // P1 = F(dvx + i dvy), P2 = F(vz + i dvz).  The |k| operator is then
-    // needed on P0 and P2 only (A3 acts on v, not on dv).
+    // Packing of the stress step's transforms: P0 = F(wx + i wy),
+    // P1 = F(wz + i vz), P2 = F(vx + i vy).  A1 is needed on P0 and P1, A3 on
+    // P1 and P2.
     {
         float2 d[G::N1];
         deriv(a.pxz, a.pyz, a.symp, d);  // dz pxz (vx) + i dz pyz (vy), D+
         float2 u[G::N1];
         update(u, d, 0, false);
-        // park (vx, dvx) in this thread's own pencil slots while vy is updated
+        // park (vx, wx) in this thread's own pencil slots while vy is updated
         __syncthreads();  // every thread has read the pencil buffer (inv_lb)
         if (act1) {  // (threads past the last pencil own no slots)
 #pragma unroll
@@ -490,18 +496,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
 #pragma unroll
         for (int j1 = 0; j1 < G::N1; ++j1) {
             const float2 ux = act1 ? pen1[j + G::N2 * j1] : make_float2(0.f, 0.f);
-            x0[j1] = make_float2(ux.x, u[j1].x);
-            x1[j1] = make_float2(ux.y, u[j1].y);
+            x0[j1] = make_float2(ux.y, u[j1].y);
+            x1[j1] = make_float2(ux.x, u[j1].x);
         }
         fft_store(x0, a.P[0]);
-        fft_store(x1, a.P[1]);
+        fft_store(x1, a.P[2]);
     }
     {
         float2 d[G::N1];
         deriv(a.pzz, nullptr, a.symm, d);  // dz pzz (vz), D-
         float2 x2[G::N1];
         update(x2, d, 2, false);
-        fft_store(x2, a.P[2]);
+#pragma unroll
+        for (int j1 = 0; j1 < G::N1; ++j1) x2[j1] = make_float2(x2[j1].y, x2[j1].x);
+        fft_store(x2, a.P[1]);
     }
 }
 
@@ -578,7 +586,7 @@ __global__ __launch_bounds__(G::T) void k2_cfft_strided(CStridedArgs a)
 
 // ------------------------------------------------------------------------
 // x-pass of the 3-D transform: forward x-FFT of P (already z- and
-// y-transformed), multiply by |k|^-1 / N and |k| / N (|k|^2 = kx^2+ky^2+kz^2
+// y-transformed), multiply by A1 = |k|^-1 / L and A3 = L |k| over N (|k|^2 = kx^2+ky^2+kz^2
 // from the folded 1-D |K| tables, evaluated in FP64 and rounded once,
 // cuviscoelas_3D.cu:72, 188-190; the DC symbol of |k|^-1 is 0 because every
 // use is followed by a derivative that vanishes there), inverse x-FFT,
@@ -599,11 +607,11 @@ struct XPassArgs {
     long long shot_stride;
     const float2* tw;
     const float *kfx, *kfy, *kfz;
-    double invN;
+    double invN, invN1, invN3;  // 1/N, 1/(N L), L/N
     int ncomp;
     const float2* P[3];
-    float2* Q1[3];
-    float2* Q3[3];
+    float2* Q1[3];           // null: A1 P_c is not used
+    float2* Q3[3];           // null: A3 P_c is not used
     float2* Q2[3];           // KS only
     float ks_vh;             // vref dt / 2 (0: no sinc^2 factor)
     float ks_k0, ks_kc;      // taper start and cut-off (kc = 0: no filter)
@@ -661,7 +669,6 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
         __syncthreads();
         float2 b[G::N2];
         if (act2) fwd_l2<G>(b, pen, jj);
-        const int nops = a.Q3[comp] ? 2 : 1;  // |k| (op 1) only where its output is used
         int jl = jj;  // opaque copy: the |k| symbols are computed here, not hoisted and held
         asm volatile("" : "+v"(jl));
         if (KS && act2) {
@@ -677,8 +684,8 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
         // ops: 0 A1 -> Q1, 1 A3 -> Q3 (where used), 2 A2 -> Q2 (KS only)
 #pragma unroll
         for (int op = 0; op < (KS ? 3 : 2); ++op) {
-            if (!KS && op >= nops) break;
-            if (KS && op == 1 && nops < 2) continue;
+            float2* const q = op == 0 ? a.Q1[comp] : (op == 1 ? a.Q3[comp] : a.Q2[comp]);
+            if (!q) continue;  // uniform: this product is not used
             __syncthreads();
             if (act2) {
                 float2 c[G::N2];
@@ -693,7 +700,7 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
                     double y = __builtin_amdgcn_rsqf((float)k2s);
                     y = fma(y, fma(-0.5 * k2s * y, y, 0.5), y);
                     const double s = KS && op == 2 ? a.invN  // A2 = 1 (F already applied)
-                                                   : (op == 0 ? a.invN * y : a.invN * (k2s * y));
+                                                   : (op == 0 ? a.invN1 * y : a.invN3 * (k2s * y));
                     float fs = (float)s;
                     // k = 0 only at element 0 (k2 = 0, jl = 0), where the
                     // estimate is inf and y NaN: both symbols are 0 there,
@@ -707,7 +714,7 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
             if (act1) {
                 float2 d[G::N1];
                 inv_lb<G>(d, pen, jj);
-                float2* const dst = (op == 0 ? a.Q1[comp] : (op == 1 ? a.Q3[comp] : a.Q2[comp])) + tbase;
+                float2* const dst = q + tbase;
 #pragma unroll
                 for (int j1 = 0; j1 < G::N1; ++j1) (dst + (long long)(G::N2 * j1) * sxi)[voff] = d[j1];
             }
@@ -717,7 +724,7 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
 
 // ------------------------------------------------------------------------
 // z-direction complex transforms on rows.
-//  mode 1 (inverse, stress step end): re_out + i im_out = IFFT_z(cin)   (im_out may be null)
+//  mode 1 (inverse, stress step end): re_out + i im_out = IFFT_z(cin)   (either may be null)
 //  mode 2 (plain, standalone transforms): cout = FFT_z^DIR(cin), in place allowed
 struct ZRowsArgs {
     long long nrows;
@@ -780,11 +787,11 @@ __global__ __launch_bounds__(kThreads) void k2_zrows(ZRowsArgs a)
 #pragma unroll
                     for (int j1 = 0; j1 < G::N1; ++j1) dst[j + G::N2 * j1] = d[j1];
                 } else {
-                    float* re = a.re_out[f] + soff + r1 * n;
+                    float* re = a.re_out[f] ? a.re_out[f] + soff + r1 * n : nullptr;
                     float* im = a.im_out[f] ? a.im_out[f] + soff + r1 * n : nullptr;
 #pragma unroll
                     for (int j1 = 0; j1 < G::N1; ++j1) {
-                        re[j + G::N2 * j1] = d[j1].x;
+                        if (re) re[j + G::N2 * j1] = d[j1].x;
                         if (im) im[j + G::N2 * j1] = d[j1].y;
                     }
                 }
@@ -852,11 +859,11 @@ __global__ __launch_bounds__(kThreads) void k2_deriv_rows(RowDerivArgs a)
 
 // ------------------------------------------------------------------------
 // Stress update (cuviscoelas_3D.cu:800-1015, generalised to VTI moduli) fused
-// with the z-derivatives of the 15 family fields, the stress C-PML memory
+// with the z-derivatives of the 12 family fields, the stress C-PML memory
 // variables on the face slabs, and the source injection
-// (cuviscoelas_3D.cu:771-777).  Tile: R = G::P/8 rows; 8 complex pencils per
-// row carry the 15 fields (two per pencil, same z-symbol); their derivatives
-// are staged in LDS, then every thread updates R*nz/256 cells.
+// (cuviscoelas_3D.cu:771-777).  Tile: R rows (StressTile); 6 complex pencils
+// per row carry the 12 fields (two per pencil, same z-symbol); their
+// derivatives are staged in LDS, then every thread updates R*nz/T cells.
 struct StressZArgs {
     int nx, ny, nz, pml;
     int ntiles, nshots, run;  // grid: tile_shot()
@@ -868,14 +875,15 @@ struct StressZArgs {
     const float *pax, *pbx, *paxh, *pbxh;
     const float *pay, *pby, *payh, *pbyh;
     const float *paz, *pbz, *pazh, *pbzh;
-    // [component][A1 v, A2 v, A3 v, A1 dv, A2 dv]; A2 = 1 (the fields v and
-    // dv themselves) unless the k-space correction is on
-    const float* fam[3][5];
+    // [component][A1 w, A2 v, A3 v, A2 w]; A2 = 1 (the fields v and w
+    // themselves) unless the k-space correction is on
+    const float* fam[3][kFam];
     float* vel[3];  // vx vy vz: force sources are added here
-    // x- and y-derivatives, blocked groups of 15 per shot:
-    //   dxb: three groups of 5, dx_group floats apart: ex (dx vx-family),
-    //        gx (dx vz-family), hx (dx vy-family), each [shot][N/64][5][64]
-    //   dyb: ey 0-4 (dy vy-family), gy 5-9 (dy vz-family), hy 10-14 (dy vx-family)
+    // x- and y-derivatives in blocked groups:
+    //   dxb: three groups of 4, dx_group floats apart: ex (dx vx-family),
+    //        gx (dx vz-family), hx (dx vy-family), each [shot][N/64][4][64]
+    //   dyb: one group of 12 per shot: ey 0-3 (dy vy-family), gy 4-7 (dy
+    //        vz-family), hy 8-11 (dy vx-family)
     const float *dxb, *dyb;
     long long dx_group;
     long long blk_stride;  // per-shot field length of the blocked groups (N rounded up to 64)
@@ -891,33 +899,33 @@ struct StressZArgs {
     const int* it;
 };
 
-// Rows of the stress update's workgroup tile: 8 pencils (kinds) per row.  One
-// pass of G::P pencils gives P/8 rows; where that leaves a third or more of
-// the pencil slots unused (P = 12..15) and 2P/8 rows still fit 54 KB of LDS
-// (3 workgroups per CU), the first transform level takes two passes over
-// 2P/8 rows instead (n = 200 = 10 x 20: 3 rows instead of 1).
+// Workgroup tile of the stress update: R rows of 6 pencils on T threads (both
+// transform levels take one pass: 6 R NMAX <= T).
+//  * rows that end on a 128-byte line: T = 192 or 256, whichever leaves fewer
+//    threads idle in the transforms (256 = 16 x 16: 12 pencils on 192 threads;
+//    at 256^3 1001 us against 1081 us on 384 and 1269 us on 512 threads: more,
+//    smaller workgroups overlap their load and transform phases better);
+//  * long rows that end mid-line share their last line and 64-cell block with
+//    the next tile, so fewer, larger tiles: T = 512 (400x400x200: 4 rows,
+//    1980 us, against 2211 us with 2 rows on 256 threads).
 template <class G>
 struct StressTile {
-    static constexpr int P1 = kThreads / G::N2, P2 = kThreads / G::N1;  // pencils per pass of each level
-    static constexpr int R2 = 2 * G::P / 8;
-    static constexpr bool kWide = G::P / 8 == 1 && G::P >= 12 && 8L * (8 * R2 * G::PS + G::TWN) <= 54L * 1024 &&
-                                  8 * R2 <= P2;
-    static constexpr int R = kWide ? R2 : G::P / 8;
-    static constexpr int RD1 = (8 * R + P1 - 1) / P1;  // passes of the first level
-    static_assert(8 * R <= P2, "the second level takes one pass");
+    static constexpr int R256 = 256 / (6 * G::NMAX), R192 = 192 / (6 * G::NMAX);
+    static constexpr int T = G::N % 32 != 0 && G::N >= 128 ? 512 : (4 * R192 >= 3 * R256 ? 192 : 256);
+    static constexpr int R = T / (6 * G::NMAX);
+    static constexpr int NP = 6 * R;  // pencils
 };
 
 // pencil kind -> (component, family member of the real part, of the imaginary part)
 // staging field index = 2*kind (+1 for the imaginary part)
-//   0: A1 vx + i A1 dvx (D-)   1: A1 vy + i A1 dvy (D-)   2: A1 vz + i A1 dvz (D+)
-//   3: vx + i dvx (D-)         4: vy + i dvy (D-)         5: vz + i dvz (D+)
-//   6: A3 vx + i A3 vy (D-)    7: A3 vz (D+)
+//   c     (0-2): A1 w_c + i A2 w_c    3 + c (3-5): A2 v_c + i A3 v_c
+// (c = 2: D+, else D-)
 template <class G, bool VTI>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_STRESSZ_WAVES))) void k2_stress_z(
+__global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_eu(QVTI_STRESSZ_WAVES))) void k2_stress_z(
     StressZArgs a)
 {
     using T = StressTile<G>;
-    constexpr int R = T::R, NP = 8 * R;
+    constexpr int R = T::R, NP = T::NP;
     constexpr int n = G::N;
     static_assert(R >= 1, "tile too small");
     static_assert(G::PS >= n + 1, "staging must fit in the pencil buffer");
@@ -926,77 +934,56 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_S
     const TileShot ts = tile_shot(a.ntiles, a.nshots, a.run);
     if (ts.tile < 0) return;  // padding workgroup (whole workgroup, before any barrier)
     const int tid = threadIdx.x, shot = ts.shot;
-    // level 1: N2 lanes per pencil, T::P1 pencils per pass; level 2: N1 lanes
-    // per pencil, all NP pencils in one pass
-    const int j = tid % G::N2, u1 = tid / G::N2;
+    // level 1: N2 lanes per pencil; level 2: N1 lanes per pencil
+    const int j = tid % G::N2, q1 = tid / G::N2;
     const int k1 = tid % G::N1, q2 = tid / G::N1;
-    const bool act2 = q2 < NP;
+    const bool act1 = q1 < NP, act2 = q2 < NP;
     const long long r0 = (long long)ts.tile * R;
     const long long soff = (long long)shot * a.shot_stride;
+    float2* pen1 = lds + q1 * G::PS;
     float2* pen2 = lds + q2 * G::PS;
-    load_twiddles<G>(tws, a.tw);
+    for (int t = tid; t < G::TWN; t += T::T) twiddle_entry<G>(tws, a.tw, t);
     __syncthreads();
-    float2 d[T::RD1][G::N1];
     {
+        const int kind1 = q1 % 6, rr1 = q1 / 6;
+        if (act1) {
+            const long long row1 = r0 + rr1;
+            const bool ok1 = row1 < a.nrows;
+            const int c = kind1 < 3 ? kind1 : kind1 - 3;
+            const float* fre = a.fam[c][kind1 < 3 ? 0 : 1];
+            const float* fim = a.fam[c][kind1 < 3 ? 3 : 2];
+            float2 v[G::N1];
 #pragma unroll
-        for (int r = 0; r < T::RD1; ++r) {
-            const int q1 = u1 + r * T::P1;
-            if (u1 < T::P1 && q1 < NP) {
-                const long long row1 = r0 + q1 / 8;
-                const bool ok1 = row1 < a.nrows;
-                const float* fre;
-                const float* fim;
-                switch (q1 % 8) {
-                case 0: fre = a.fam[0][0]; fim = a.fam[0][3]; break;
-                case 1: fre = a.fam[1][0]; fim = a.fam[1][3]; break;
-                case 2: fre = a.fam[2][0]; fim = a.fam[2][3]; break;
-                case 3: fre = a.fam[0][1]; fim = a.fam[0][4]; break;
-                case 4: fre = a.fam[1][1]; fim = a.fam[1][4]; break;
-                case 5: fre = a.fam[2][1]; fim = a.fam[2][4]; break;
-                case 6: fre = a.fam[0][2]; fim = a.fam[1][2]; break;
-                default: fre = a.fam[2][2]; fim = nullptr; break;
-                }
-                float2 v[G::N1];
-#pragma unroll
-                for (int j1 = 0; j1 < G::N1; ++j1) {
-                    const long long g = soff + row1 * n + j1 * G::N2 + j;
-                    v[j1] = ok1 ? make_float2(fre[g], fim ? fim[g] : 0.f) : make_float2(0.f, 0.f);
-                }
-                fwd_l1<G>(v, lds + q1 * G::PS, tws, j);
+            for (int j1 = 0; j1 < G::N1; ++j1) {
+                const long long g = soff + row1 * n + j1 * G::N2 + j;
+                v[j1] = ok1 ? make_float2(fre[g], fim[g]) : make_float2(0.f, 0.f);
             }
+            fwd_l1<G>(v, pen1, tws, j);
         }
         __syncthreads();
         float2 b[G::N2];
         if (act2) {
             fwd_l2<G>(b, pen2, k1);
-            const int k2kind = q2 % 8;
-            const float2* S = (k2kind == 2 || k2kind == 5 || k2kind == 7) ? a.symp : a.symm;
+            const int kind2 = q2 % 6;
+            const float2* S = kind2 == 2 || kind2 == 5 ? a.symp : a.symm;
 #pragma unroll
             for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = c_mul(b[k2], S[k1 + G::N1 * k2]);
         }
         __syncthreads();
         if (act2) inv_la<G>(b, pen2, tws + G::T2OFF, k1);
         __syncthreads();
-#pragma unroll
-        for (int r = 0; r < T::RD1; ++r) {
-            const int q1 = u1 + r * T::P1;
-            if (u1 < T::P1 && q1 < NP) inv_lb<G>(d[r], lds + q1 * G::PS, j);
-        }
+        float2 d[G::N1];
+        if (act1) inv_lb<G>(d, pen1, j);
         __syncthreads();
         // stage: st[field][rr][iz] with rows padded to n + 1 floats (odd), so
         // the rows written by one wave fall in different banks, field = 2*kind + part
         float* st = reinterpret_cast<float*>(lds);
+        if (act1) {
 #pragma unroll
-        for (int r = 0; r < T::RD1; ++r) {
-            const int q1 = u1 + r * T::P1;
-            if (u1 < T::P1 && q1 < NP) {
-                const int kind = q1 % 8, rr = q1 / 8;
-#pragma unroll
-                for (int j1 = 0; j1 < G::N1; ++j1) {
-                    const int iz = j + G::N2 * j1;
-                    st[((2 * kind) * R + rr) * (n + 1) + iz] = d[r][j1].x;
-                    st[((2 * kind + 1) * R + rr) * (n + 1) + iz] = d[r][j1].y;
-                }
+            for (int j1 = 0; j1 < G::N1; ++j1) {
+                const int iz = j + G::N2 * j1;
+                st[((2 * kind1) * R + rr1) * (n + 1) + iz] = d[j1].x;
+                st[((2 * kind1 + 1) * R + rr1) * (n + 1) + iz] = d[j1].y;
             }
         }
         __syncthreads();
@@ -1010,13 +997,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_S
     // uniform block bases; per-cell offsets below are unsigned 32-bit
     const long long cbase = r0 * n;          // flat index of the tile's first cell
     const long long fbase = soff + cbase;    // per-shot natural fields
-    const float* __restrict__ dxs = a.dxb + (long long)shot * 5 * a.blk_stride;
-    const float* __restrict__ dys = a.dyb + (long long)shot * kG1 * a.blk_stride;
+    constexpr int kDY = 3 * kFam;  // y-derivatives per cell
+    const float* __restrict__ dxs = a.dxb + (long long)shot * kFam * a.blk_stride;
+    const float* __restrict__ dys = a.dyb + (long long)shot * kDY * a.blk_stride;
     constexpr bool vti = VTI;  // G2 (H, D sets) present: a compile-time choice keeps the loads branch-free
     const long long sxb = (long long)shot * a.slabx_stride, syb = (long long)shot * a.slaby_stride,
                     szb = (long long)shot * a.slabz_stride;
 #pragma unroll 1
-    for (int cell = tid; cell < R * n; cell += kThreads) {
+    for (int cell = tid; cell < R * n; cell += T::T) {
         const int rr = cell / n, iz = cell - rr * n;
         const long long row = r0 + rr;
         if (row >= a.nrows) continue;
@@ -1024,31 +1012,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_S
         const unsigned o = (unsigned)cell;  // == rr * n + iz
         auto S = [&](int f) { return st[(f * R + rr) * (n + 1) + iz]; };
         if (ix < a.nx - 1 && iy < a.ny - 1 && iz < n - 1) {
-            // staging fields of the family members j = 0..4 (A1 v, v, A3 v, A1 dv, dv)
-            const int fz[5] = {4, 10, 14, 5, 11};   // vz family (D+): normal dz vz
-            const int fgx[5] = {0, 6, 12, 1, 7};    // vx family (D-): dz vx for pxz
-            const int fhy[5] = {2, 8, 13, 3, 9};    // vy family (D-): dz vy for pyz
+            // staging fields of the family members (A1 w, v, A3 v, w)
+            const int fz[kFam] = {4, 10, 11, 5};   // vz family (D+): normal dz vz
+            const int fgx[kFam] = {0, 6, 7, 1};    // vx family (D-): dz vx for pxz
+            const int fhy[kFam] = {2, 8, 9, 3};    // vy family (D-): dz vy for pyz
             // blocked addresses of the cell: one pointer per group, the
             // fields at immediate offsets f*64 floats
             const unsigned ip = (unsigned)cbase + o;
-            const unsigned q15 = (ip >> 6) * (kBlk * kG1) + (ip & 63u);
-            const float* __restrict__ dxp = dxs + ((ip >> 6) * (kBlk * 5) + (ip & 63u));
-            const float* __restrict__ dyp = dys + q15;
-            const float* __restrict__ g1p = a.g1 + q15;
-            const float* __restrict__ g2p = vti ? a.g2 + ((ip >> 6) * (kBlk * kG2) + (ip & 63u)) : nullptr;
+            const unsigned blk = ip >> 6, in = ip & 63u;
+            const float* __restrict__ dxp = dxs + (blk * (kBlk * kFam) + in);
+            const float* __restrict__ dyp = dys + (blk * (kBlk * kDY) + in);
+            const float* __restrict__ g1p = a.g1 + (blk * (kBlk * kG1) + in);
+            const float* __restrict__ g2p = vti ? a.g2 + (blk * (kBlk * kG2) + in) : nullptr;
             float A[14];
 #pragma unroll
             for (int k = 0; k < 14; ++k) A[k] = 0.f;
 #pragma unroll
-            for (int jf = 0; jf < 5; ++jf) {
+            for (int jf = 0; jf < kFam; ++jf) {
                 const float ez = S(fz[jf]), gz = S(fgx[jf]), hz = S(fhy[jf]);
                 const float ex = dxp[jf * kBlk], gx = dxp[a.dx_group + jf * kBlk], hx = dxp[2 * a.dx_group + jf * kBlk];
-                const float ey = dyp[jf * kBlk], gy = dyp[(5 + jf) * kBlk], hy = dyp[(10 + jf) * kBlk];
-                const float c33 = g1p[jf * kBlk], cs = g1p[(5 + jf) * kBlk], csb = g1p[(10 + jf) * kBlk];
+                const float ey = dyp[jf * kBlk], gy = dyp[(kFam + jf) * kBlk], hy = dyp[(2 * kFam + jf) * kBlk];
+                const float c33 = g1p[jf * kBlk], cs = g1p[(kFam + jf) * kBlk], csb = g1p[(2 * kFam + jf) * kBlk];
                 float c11 = c33, c13 = c33;
                 if (vti) {
                     c11 = g2p[jf * kBlk];
-                    c13 = g2p[(5 + jf) * kBlk];
+                    c13 = g2p[(kFam + jf) * kBlk];
                 }
                 const float c12 = c11 - 2 * cs, c13d = c13 - 2 * cs;
                 A[0] += c11 * ex;   // s11x

@@ -1,0 +1,56 @@
+"""GPU: the four-field stress family {A1 w, v, A3 v, w}, w = alpha (v + kappa
+dv), against the FP64 oracle, which evaluates the scheme's five terms per
+moduli set.  kappa and alpha depend on the Q reference frequency and the
+medium, and the stress update's tile (rows per workgroup) on the row length.
+
+The bound is that of the other step cases (1e-5 relative L2): FP32 rounding
+per step is about 1e-7 and the runs take at most 20 steps.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+import qvti
+from cases import rel_l2, small_case
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+# row lengths of every tile shape (192, 256 and 512 threads; 1 to 10 rows),
+# with row counts that leave a remainder; reference frequencies below, at and
+# above the source's, so that w is dominated by dv, balanced, or close to v
+CASES = [
+    # nx, ny, nz, vti, media, w0 / (2 pi f0)
+    (18, 30, 16, True, qvti.MEDIA_VISCO, 1.0),
+    (16, 18, 64, False, qvti.MEDIA_VISCO, 0.05),
+    (20, 18, 96, True, qvti.MEDIA_VISCO, 20.0),
+    (18, 18, 128, True, qvti.MEDIA_QCOMP, 0.3),
+    (18, 16, 150, False, qvti.MEDIA_DISPERSION, 1.0),
+    (16, 18, 200, True, qvti.MEDIA_VISCO, 3.0),
+    (16, 20, 256, False, qvti.MEDIA_LOSSLESS, 1.0),
+    (18, 16, 324, True, qvti.MEDIA_QCOMP, 1.0),
+    (16, 16, 400, True, qvti.MEDIA_VISCO, 0.5),
+    (18, 16, 512, False, qvti.MEDIA_VISCO, 1.0),
+]
+
+
+@pytest.mark.parametrize("nx,ny,nz,vti,media,ratio", CASES)
+def test_stress_family_matches_the_oracle(nx, ny, nz, vti, media, ratio):
+    shot, model = small_case(nx, ny, nz, 4, 12 if nx * ny * nz > 50000 else 20, O.SRC_FX, vti, seed=nz)
+    shot["w0"] = float(np.float32(shot["w0"] * ratio))
+    ref = O.run(shot, model, "f64", state=True, media=media)
+    with qvti.Engine(nx, ny, nz, shot["pml"], shot["dx"], shot["dy"], shot["dz"], shot["dt"], shot["f0"], shot["w0"],
+                     vti=vti) as e:
+        e.set_media(media)
+        e.set_model_dict(model)
+        e.begin(shot["nt"], shot["rik"], [qvti.make_shot(shot["src_kind"], (shot["sx"], shot["sy"], shot["sz"]),
+                                                         shot["rx"], shot["ry"], shot["rz"])])
+        e.step(shot["nt"])
+        e.finish()
+        st = e.state()
+    errs = [rel_l2(st[k], ref["state"][k]) for k in range(9)]
+    print("%dx%dx%d media %d w0 ratio %g: state vs FP64 oracle %.2e, per field max %.2e"
+          % (nx, ny, nz, media, ratio, rel_l2(st, ref["state"]), max(errs)))
+    assert rel_l2(st[:3], ref["state"][:3]) < TOL
+    assert rel_l2(st[3:], ref["state"][3:]) < TOL

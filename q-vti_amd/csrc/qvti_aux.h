@@ -100,6 +100,12 @@ static __global__ __launch_bounds__(256) void k_probe(const float* f, long long 
 // complex transform with it, and the others' coefficients are of order g.
 //   o[0] = L o0 / alpha (A1 w), o[1] = M (1 + g^2) (v),
 //   o[2] = o2 / L (A3 v),       o[3] = -M g^2 / alpha (w)
+// o2 and o3 follow from o0, o1 and one field r = alpha / (rho w0^2 L^2):
+//   o3 = -o0^2 r,  o2 = -o0 r M,  M = o1 + alpha o3
+// (set_coeffs).  The stress update forms them per cell in FP32, so that it
+// reads 13 coefficient fields instead of 20 (VTI; 9 instead of 12 isotropic).
+// Their rounding (about 2^-23 relative) enters the stresses times g, of order
+// 1e-2, so below that of o1 v.
 // media (qvti_set_media, the reference's media_type, viscoelas_3D.cpp:57-60):
 // 0 viscoelastic (as above); 1 dispersion only (tau terms dropped: kappa = 0,
 // w = v, no fourth term); 2 lossless (gamma = 0); 3 Q-compensating (tau terms
@@ -118,6 +124,18 @@ __device__ __forceinline__ void q_coeffs(double rho, double v, double g, double 
     o[3] = -Mg2 / alpha;
 }
 
+// The four coefficients of one moduli set in the stress update from its
+// stored o0, o1 and the cell's r; s4 = 0 where the medium has no tau terms
+// (dispersion only), else 1.
+__device__ __forceinline__ void set_coeffs(float (&o)[kFam], float o0, float o1, float r, float alpha, float s4)
+{
+    const float t = o0 * r;
+    o[0] = o0;
+    o[1] = o1;
+    o[3] = -s4 * (o0 * t);
+    o[2] = -t * (o1 + alpha * o[3]);
+}
+
 // (blocked field groups and coefficient group sizes: qvti_layout.h)
 
 struct CoefArgs {
@@ -125,8 +143,9 @@ struct CoefArgs {
     int vti, media;
     double w0, alpha, L;
     const float *vp, *gp, *vs, *gs, *rho, *eps, *del;
-    float* g1;  // blocked [N/64][kG1][64]: P, S (S-bar filled by k_averages)
-    float* g2;  // blocked [N/64][kG2][64]: H, D (VTI only)
+    float* g1;  // blocked [N/64][kG1][64]
+    float* g2;  // blocked [N/64][kG2][64] (VTI only)
+    float* s;   // [kFam][N]: the S set, averaged by k_averages
 };
 
 static __global__ __launch_bounds__(256) void k_coefficients(CoefArgs a)
@@ -135,14 +154,17 @@ static __global__ __launch_bounds__(256) void k_coefficients(CoefArgs a)
         double o[kFam];
         const double r = a.rho[ip];
         q_coeffs(r, a.vp[ip], a.gp[ip], a.w0, a.alpha, a.L, a.media, o);
-        for (int j = 0; j < kFam; ++j) a.g1[blk_index(ip, kG1, j)] = (float)o[j];
+        for (int j = 0; j < 2; ++j) a.g1[blk_index(ip, kG1, j)] = (float)o[j];
         q_coeffs(r, a.vs[ip], a.gs[ip], a.w0, a.alpha, a.L, a.media, o);
-        for (int j = 0; j < kFam; ++j) a.g1[blk_index(ip, kG1, kFam + j)] = (float)o[j];
+        for (int j = 0; j < 2; ++j) a.g1[blk_index(ip, kG1, 2 + j)] = (float)o[j];
+        for (int j = 0; j < kFam; ++j) a.s[j * a.N + ip] = (float)o[j];
+        // (rho = 0: every coefficient is 0)
+        a.g1[blk_index(ip, kG1, 4)] = r != 0.0 ? (float)(a.alpha / (r * (a.w0 * a.w0) * (a.L * a.L))) : 0.f;
         if (a.vti) {
             const double e = a.eps[ip], dl = a.del[ip], vp = a.vp[ip], vs = a.vs[ip];
             const double vh = e == 0.0 ? vp : vp * sqrt(1.0 + 2.0 * e);
             q_coeffs(r, vh, a.gp[ip], a.w0, a.alpha, a.L, a.media, o);
-            for (int j = 0; j < kFam; ++j) a.g2[blk_index(ip, kG2, j)] = (float)o[j];
+            for (int j = 0; j < 2; ++j) a.g2[blk_index(ip, kG2, j)] = (float)o[j];
             double vd = vp;
             if (dl != 0.0) {
                 const double c33 = r * vp * vp, c44 = r * vs * vs;
@@ -150,7 +172,7 @@ static __global__ __launch_bounds__(256) void k_coefficients(CoefArgs a)
                 vd = sqrt((sqrt(prod > 0.0 ? prod : 0.0) + c44) / r);
             }
             q_coeffs(r, vd, a.gp[ip], a.w0, a.alpha, a.L, a.media, o);
-            for (int j = 0; j < kFam; ++j) a.g2[blk_index(ip, kG2, kFam + j)] = (float)o[j];
+            for (int j = 0; j < 2; ++j) a.g2[blk_index(ip, kG2, 2 + j)] = (float)o[j];
         }
     }
 }
@@ -161,7 +183,8 @@ struct AvgArgs {
     int nx, ny, nz;
     long long sx, sy, N;
     float dt;
-    float* g1;       // coefficient group 1: reads S (fields 4-7), writes S-bar (8-11)
+    const float* s;  // [kFam][N]: the S set
+    float* gs;       // blocked [N/64][kGS][64]: S-bar
     const float* rho;
     float* buoy;     // [3][N]
 };
@@ -174,14 +197,15 @@ static __global__ __launch_bounds__(256) void k_averages(AvgArgs a)
         const int iz = (int)(ip - (long long)ix * a.sx - (long long)iy * a.sy);
         const bool in = ix < a.nx - 1 && iy < a.ny - 1 && iz < a.nz - 1;
         for (int j = 0; j < kFam; ++j) {
-            auto c = [&](long long q) { return a.g1[blk_index(q, kG1, kFam + j)]; };
+            const float* c_ = a.s + j * a.N;
+            auto c = [&](long long q) { return c_[q]; };
             float v = 0.f;
             if (in) {
                 const float s8 = c(ip) + c(ip + 1) + c(ip + a.sy) + c(ip + 1 + a.sy) + c(ip + a.sx) + c(ip + a.sx + 1)
                                + c(ip + a.sx + a.sy) + c(ip + a.sx + 1 + a.sy);
                 v = 0.125f * s8;
             }
-            a.g1[blk_index(ip, kG1, 2 * kFam + j)] = v;
+            a.gs[blk_index(ip, kGS, j)] = v;
         }
         // rho + rho' is an FP32 sum in the reference, the rest FP64
         const float r = a.rho[ip];

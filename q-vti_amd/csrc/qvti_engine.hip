@@ -202,7 +202,7 @@ extern "C" long long qvti_estimate_bytes(const qvti_grid* g, int max_shots)
     const long long N = (long long)g->nx * g->ny * g->nz;
     const long long p2 = 2LL * g->pml;
     const long long slabs = 8LL * (p2 * g->ny * g->nz + (long long)g->nx * p2 * g->nz) + 7LL * g->nx * g->ny * p2;
-    const long long model = kG1 + (g->vti ? kG2 : 0) + 3;
+    const long long model = kG1 + kGS + (g->vti ? kG2 : 0) + 3;
     return 4LL * (N * (state_fields() * max_shots + model) + slabs * max_shots) + (64LL << 20);
 }
 
@@ -329,7 +329,7 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
     c->slab[1] = (long long)g->nx * p2 * g->nz;
     c->slab[2] = (long long)g->nx * g->ny * p2;
     const long long Nb = c->Nb;
-    rc = rc ? rc : dalloc(c, (void**)&c->coef, sizeof(float) * (kG1 + (g->vti ? kG2 : 0)) * Nb);
+    rc = rc ? rc : dalloc(c, (void**)&c->coef, sizeof(float) * (kG1 + kGS + (g->vti ? kG2 : 0)) * Nb);
     rc = rc ? rc : dalloc(c, (void**)&c->buoy, sizeof(float) * 3 * N);
     rc = rc ? rc : dalloc(c, (void**)&c->v, sizeof(float) * 3 * S * N);
     rc = rc ? rc : dalloc(c, (void**)&c->sig, sizeof(float) * 6 * S * N);
@@ -342,7 +342,7 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
         rc = rc ? rc : dalloc(c, (void**)&c->phis[a], sizeof(float) * c->nphis[a] * S * c->slab[a]);
     }
     rc = rc ? rc : dalloc(c, (void**)&c->d_it, sizeof(int));
-    rc = rc ? rc : dalloc(c, (void**)&c->d_wab, 2 * sizeof(float));
+    rc = rc ? rc : dalloc(c, (void**)&c->d_wab, 3 * sizeof(float));
     rc = rc ? rc : dalloc(c, (void**)&c->d_probe, sizeof(int));
     rc = rc ? rc : dalloc(c, (void**)&c->d_src_kind, sizeof(int) * S);
     rc = rc ? rc : dalloc(c, (void**)&c->d_src_ip, sizeof(long long) * S);
@@ -607,7 +607,9 @@ static int build_launch_config(qvti_ctx* c)
     sz.blk_stride = c->Nb;
     sz.dyb = c->bufB;
     sz.g1 = c->coef;
-    sz.g2 = g.vti ? c->coef + (long long)kG1 * c->Nb : nullptr;
+    sz.gs = c->coef + (long long)kG1 * c->Nb;
+    sz.g2 = g.vti ? c->coef + (long long)(kG1 + kGS) * c->Nb : nullptr;
+    sz.wab = c->d_wab;
     for (int k = 0; k < 6; ++k) sz.sig[k] = sg[k];
     for (int k = 0; k < 3; ++k) sz.vel[k] = vv[k];
     for (int k = 0; k < 5; ++k) {
@@ -663,7 +665,7 @@ extern "C" int qvti_set_model(qvti_ctx* c, const float* velp, const float* gama_
     if (c->media == QVTI_MEDIA_QCOMP) c->kappa = -c->kappa;
     const double tilt = c->kappa == 0.0 ? 0.0 : 5.0 * 2.0 * M_PI * M_PI * (double)c->g.f0 / (double)c->g.w0;
     c->alpha = exp2(-round(log2(sqrt(1.0 + tilt * tilt))));
-    const float wab[2] = {(float)c->alpha, (float)(c->alpha * c->kappa)};
+    const float wab[3] = {(float)c->alpha, (float)(c->alpha * c->kappa), c->media == QVTI_MEDIA_DISPERSION ? 0.f : 1.f};
     int rc = QVTI_OK;
     if (hipMemcpyAsync(c->d_wab, wab, sizeof wab, hipMemcpyHostToDevice, c->stream) != hipSuccess)
         rc = qvti_fail(QVTI_E_DEVICE, "model upload failed");
@@ -682,14 +684,16 @@ extern "C" int qvti_set_model(qvti_ctx* c, const float* velp, const float* gama_
         ca.eps = c->g.vti ? tmp + 5 * N : nullptr;
         ca.del = c->g.vti ? tmp + 6 * N : nullptr;
         ca.g1 = c->coef;
-        ca.g2 = c->g.vti ? c->coef + (long long)kG1 * c->Nb : nullptr;
+        ca.g2 = c->g.vti ? c->coef + (long long)(kG1 + kGS) * c->Nb : nullptr;
+        ca.s = tmp + 7 * N;  // free after the averages
         const unsigned nb = (unsigned)std::min<long long>((N + kThreads - 1) / kThreads, 65535LL * 4);
         hipLaunchKernelGGL(k_coefficients, dim3(nb), dim3(kThreads), 0, c->stream, ca);
         AvgArgs aa;
         aa.nx = c->g.nx; aa.ny = c->g.ny; aa.nz = c->g.nz;
         aa.sx = (long long)c->g.ny * c->g.nz; aa.sy = c->g.nz; aa.N = N;
         aa.dt = c->g.dt;
-        aa.g1 = c->coef;
+        aa.s = ca.s;
+        aa.gs = c->coef + (long long)kG1 * c->Nb;
         aa.rho = tmp + 4 * N;
         aa.buoy = c->buoy;
         hipLaunchKernelGGL(k_averages, dim3(nb), dim3(kThreads), 0, c->stream, aa);
@@ -1732,7 +1736,7 @@ extern "C" int qvti_kernel_bytes(qvti_ctx* c, int max_classes, double* bytes)
     const double N = (double)c->N * std::max(1, c->nshots), f = 4.0 * N;
     const double slab = (double)std::max(1, c->nshots) * 4.0;
     const double sx = c->slab[0] * slab, sy = c->slab[1] * slab, sz = c->slab[2] * slab;
-    const int ncoef = kG1 + (c->g.vti ? kG2 : 0);
+    const int ncoef = kG1 + kGS + (c->g.vti ? kG2 : 0);
     double b[KC_COUNT] = {};
     b[KC_TICK] = 8;
     b[KC_VEL_X] = 6 * f + 3 * 2 * sx;

@@ -23,7 +23,9 @@ __host__ __device__ __forceinline__ long long blk_index(long long ip, int nf, in
 // A2 w} whose derivatives the stress update weighs with the Q coefficients
 // (k_coefficients in qvti_aux.h).
 constexpr int kFam = 4;
-// coefficient groups: G1 = {P 0-3, S 4-7, S-bar 8-11}, G2 = {H 0-3, D 4-7} (VTI)
-constexpr int kG1 = 3 * kFam, kG2 = 2 * kFam;
+// coefficient groups: G1 = {P: o0, o1; S: o0, o1; r}, the 8-corner averages GS
+// = {S-bar: o0..o3}, G2 = {H: o0, o1; D: o0, o1} (VTI).  The stress update
+// derives o2 and o3 of the sets P, S, H and D (set_coeffs in qvti_aux.h).
+constexpr int kG1 = 5, kGS = kFam, kG2 = 4;
 
 }  // namespace qvti

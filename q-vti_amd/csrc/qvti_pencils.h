@@ -28,11 +28,13 @@
 //    everywhere (q_coeffs in qvti_aux.h), so only A1 w and A3 v need the full
 //    3-D transform - three forward and four inverse complex transforms.  With
 //    five fields {A1 v, v, A3 v, A1 dv, dv} per component it was three and
-//    five, and 248 floats per cell and step through HBM instead of 211 (VTI).
+//    five, and 248 floats per cell and step through HBM instead of 204 (VTI,
+//    with the coefficients of set_coeffs).
 //    Fields that share a complex transform are scaled (alpha and the length
 //    scale of A1 and A3, powers of two) so that the FP32 rounding of one does
 //    not swamp the other where it matters (q_coeffs).
 #pragma once
+#include "qvti_aux.h"
 #include "qvti_fft2l.h"
 #include "qvti_layout.h"
 
@@ -887,8 +889,9 @@ struct StressZArgs {
     const float *dxb, *dyb;
     long long dx_group;
     long long blk_stride;  // per-shot field length of the blocked groups (N rounded up to 64)
-    // coefficient groups G1 {P, S, S-bar} and G2 {H, D} (VTI; else null)
-    const float *g1, *g2;
+    // coefficient groups G1, GS and G2 (VTI; else null)
+    const float *g1, *gs, *g2;
+    const float* wab;  // {alpha, alpha kappa, s4}
     float* sig[6];  // pxx pyy pzz pxy pxz pyz
     float* phx[5];
     float* phy[5];
@@ -991,6 +994,7 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
     const float* st = reinterpret_cast<const float*>(lds);
     const int pml = a.pml;
     const float dt = a.dt;
+    const float alpha = a.wab[0], s4 = a.wab[2];
     const int it = *a.it;
     const int kind = a.src_kind[shot];
     const long long sip = a.src_ip[shot];
@@ -1023,7 +1027,18 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
             const float* __restrict__ dxp = dxs + (blk * (kBlk * kFam) + in);
             const float* __restrict__ dyp = dys + (blk * (kBlk * kDY) + in);
             const float* __restrict__ g1p = a.g1 + (blk * (kBlk * kG1) + in);
+            const float* __restrict__ gsp = a.gs + (blk * (kBlk * kGS) + in);
             const float* __restrict__ g2p = vti ? a.g2 + (blk * (kBlk * kG2) + in) : nullptr;
+            float oP[kFam], oS[kFam], oH[kFam], oD[kFam];
+            {
+                const float r = g1p[4 * kBlk];
+                set_coeffs(oP, g1p[0], g1p[kBlk], r, alpha, s4);
+                set_coeffs(oS, g1p[2 * kBlk], g1p[3 * kBlk], r, alpha, s4);
+                if (vti) {
+                    set_coeffs(oH, g2p[0], g2p[kBlk], r, alpha, s4);
+                    set_coeffs(oD, g2p[2 * kBlk], g2p[3 * kBlk], r, alpha, s4);
+                }
+            }
             float A[14];
 #pragma unroll
             for (int k = 0; k < 14; ++k) A[k] = 0.f;
@@ -1032,12 +1047,8 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
                 const float ez = S(fz[jf]), gz = S(fgx[jf]), hz = S(fhy[jf]);
                 const float ex = dxp[jf * kBlk], gx = dxp[a.dx_group + jf * kBlk], hx = dxp[2 * a.dx_group + jf * kBlk];
                 const float ey = dyp[jf * kBlk], gy = dyp[(kFam + jf) * kBlk], hy = dyp[(2 * kFam + jf) * kBlk];
-                const float c33 = g1p[jf * kBlk], cs = g1p[(kFam + jf) * kBlk], csb = g1p[(2 * kFam + jf) * kBlk];
-                float c11 = c33, c13 = c33;
-                if (vti) {
-                    c11 = g2p[jf * kBlk];
-                    c13 = g2p[(kFam + jf) * kBlk];
-                }
+                const float c33 = oP[jf], cs = oS[jf], csb = gsp[jf * kBlk];
+                const float c11 = vti ? oH[jf] : c33, c13 = vti ? oD[jf] : c33;
                 const float c12 = c11 - 2 * cs, c13d = c13 - 2 * cs;
                 A[0] += c11 * ex;   // s11x
                 A[1] += c12 * ex;   // s12x

@@ -166,7 +166,7 @@ def measured_traffic(name, kernel):
 # name each dispatch carries in a rocprofv3 trace, and the class it times.
 STEP_SIGNATURE = (("k2_deriv_strided", "vel_x"), ("k2_deriv_strided", "vel_y"), ("k2_vel_z", "vel_z_fwd"),
                   ("k2_cfft_strided", "y_fwd"), ("k2_xpass", "xpass"), ("k2_cfft_strided", "y_inv"),
-                  ("k2_zrows", "z_inv"), ("k2_deriv_strided", "str_x"), ("k2_deriv_strided", "str_y"),
+                  ("k2_zrows", "z_inv"), ("k2_stress_xy", "str_x"), ("k2_stress_xy", "str_y"),
                   ("k2_stress_z", "str_z"), ("k_record", "record"))
 
 

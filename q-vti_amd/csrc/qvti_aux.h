@@ -184,7 +184,7 @@ struct AvgArgs {
     long long sx, sy, N;
     float dt;
     const float* s;  // [kFam][N]: the S set
-    float* gs;       // blocked [N/64][kGS][64]: S-bar
+    float* gs;       // [kGS][N]: S-bar
     const float* rho;
     float* buoy;     // [3][N]
 };
@@ -205,7 +205,7 @@ static __global__ __launch_bounds__(256) void k_averages(AvgArgs a)
                                + c(ip + a.sx + a.sy) + c(ip + a.sx + 1 + a.sy);
                 v = 0.125f * s8;
             }
-            a.gs[blk_index(ip, kGS, j)] = v;
+            a.gs[j * a.N + ip] = v;
         }
         // rho + rho' is an FP32 sum in the reference, the rest FP64
         const float r = a.rho[ip];

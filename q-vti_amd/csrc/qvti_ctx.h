@@ -83,7 +83,8 @@ struct qvti_ctx {
     long long kc_launches[KC_COUNT] = {};
     double kc_ms[KC_COUNT] = {};
     // launch configuration
-    StridedArgs a_vx{}, a_vy{}, a_sx{}, a_sy{};
+    StridedArgs a_vx{}, a_vy{};
+    StressXYArgs a_sx{}, a_sy{};
     VelZArgs a_vz{};
     ZRowsArgs a_zi{};
     CStridedArgs a_yf{}, a_yi{};
@@ -105,7 +106,8 @@ struct qvti_ctx {
     // opt-in k-space correction / wavenumber filter (off: the reference scheme)
     bool ks = false;
     float ks_vref = 0.f, ks_fcut = 0.f, ks_vmax = 0.f, ks_taper = 0.f;
-    float* H2 = nullptr;  // [A2 v x,y,z][A2 w x,y,z], allocated on first use
+    // [A2 v x,y,z][A2 w x,y,z], then their three complex spectra; allocated on first use
+    float* H2 = nullptr;
     long long bytes = 0;
     std::vector<void*> allocs;
 };

@@ -190,11 +190,12 @@ static void release(qvti_ctx* c)
 }
 
 // ------------------------------------------------------- sizes / memory --
-// Fields per shot of each scratch buffer (bufA, bufB): the 12 derivatives of
-// the stress family along x and y; the spectra they held before take 8 and
-// 6 (12 in k-space mode).
-constexpr int kBufFields = 3 * kFam;
-static long long state_fields() { return 3 + 6 + 3 + 6 + kBufFields + kBufFields; }
+// Fields per shot of the scratch buffers.  bufA: velocity accumulators (3),
+// then the four Q spectra (8), then the x-derivatives (kDer).  bufB: the three
+// P spectra (6), then the y-derivatives (kDer).
+constexpr int kFieldsA = 8, kFieldsB = 6;
+static_assert(kDer <= kFieldsA && kDer <= kFieldsB, "derivatives fit the scratch buffers");
+static long long state_fields() { return 3 + 6 + 3 + 6 + kFieldsA + kFieldsB; }
 
 extern "C" long long qvti_estimate_bytes(const qvti_grid* g, int max_shots)
 {
@@ -335,8 +336,8 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
     rc = rc ? rc : dalloc(c, (void**)&c->sig, sizeof(float) * 6 * S * N);
     rc = rc ? rc : dalloc(c, (void**)&c->w, sizeof(float) * 3 * S * N);
     rc = rc ? rc : dalloc(c, (void**)&c->H, sizeof(float) * 6 * S * N);
-    rc = rc ? rc : dalloc(c, (void**)&c->bufA, sizeof(float) * kBufFields * S * Nb);
-    rc = rc ? rc : dalloc(c, (void**)&c->bufB, sizeof(float) * kBufFields * S * Nb);
+    rc = rc ? rc : dalloc(c, (void**)&c->bufA, sizeof(float) * kFieldsA * S * Nb);
+    rc = rc ? rc : dalloc(c, (void**)&c->bufB, sizeof(float) * kFieldsB * S * Nb);
     for (int a = 0; a < 3 && !rc; ++a) {
         rc = dalloc(c, (void**)&c->phiv[a], sizeof(float) * 3 * S * c->slab[a]);
         rc = rc ? rc : dalloc(c, (void**)&c->phis[a], sizeof(float) * c->nphis[a] * S * c->slab[a]);
@@ -497,15 +498,14 @@ static int build_launch_config(qvti_ctx* c)
     for (int k = 0; k < 3; ++k) xp.P[k] = P[k];
     xp.Q1[0] = Q[0]; xp.Q1[1] = Q[1]; xp.Q1[2] = nullptr;
     xp.Q3[0] = nullptr; xp.Q3[1] = Q[2]; xp.Q3[2] = Q[3];
-    // k-space mode: A2 F P_c -> Q2_c in bufB fields 6-11 (free once the
-    // x-pass has read P; the y-derivatives overwrite them after z_inv)
+    // k-space mode: A2 F P_c -> Q2_c, after the six real fields of H2
     float2* Q2[3] = {nullptr, nullptr, nullptr};
     float* H2v[3] = {nullptr, nullptr, nullptr};
     float* H2w[3] = {nullptr, nullptr, nullptr};
     xp.ks_vh = xp.ks_k0 = xp.ks_kc = xp.ks_pw = 0.f;
     if (c->ks) {
         for (int k = 0; k < 3; ++k) {
-            Q2[k] = reinterpret_cast<float2*>(fld(c->bufB, 6 + 2 * k, c));
+            Q2[k] = reinterpret_cast<float2*>(fld(c->H2, 6 + 2 * k, c));
             H2v[k] = fld(c->H2, k, c);
             H2w[k] = fld(c->H2, 3 + k, c);
             xp.Q2[k] = Q2[k];
@@ -554,40 +554,41 @@ static int build_launch_config(qvti_ctx* c)
         fam[k][0] = H1w[k]; fam[k][1] = vv[k]; fam[k][2] = H3v[k]; fam[k][3] = ww[k];
         if (c->ks) { fam[k][1] = H2v[k]; fam[k][3] = H2w[k]; }
     }
-    // x/y derivatives of the stress step: blocked groups in bufA (x) and bufB
-    // (y); job k writes field k of the group.
-    // x-derivatives: three blocked groups of 4 (ex, gx, hx), each [shot][N/64][4][64];
-    // y-derivatives: one blocked group of 12
-    float* DX[3 * kFam];
-    float* DY[3 * kFam];
-    for (int k = 0; k < 3 * kFam; ++k) {
-        DX[k] = c->bufA + (long long)(k / kFam) * kFam * c->S * c->Nb + (long long)(k % kFam) * kBlk;
-        DY[k] = c->bufB + (long long)k * kBlk;
-    }
-    StridedArgs& sxa = c->a_sx;
-    strided_common(sxa, 0, Px);
-    sxa.mode = MODE_STORE;
-    sxa.njobs = 3 * kFam;
-    sxa.bnf = kFam;
-    sxa.blk_stride = c->Nb;
-    for (int j = 0; j < kFam; ++j) {
-        const int g = kFam + j, h = 2 * kFam + j;
-        sxa.job[j] = job(fam[0][j], DX[j], nullptr, nullptr, 0, 0);  // ex: dx vx-family, D+
-        sxa.job[g] = job(fam[2][j], DX[g], nullptr, nullptr, 1, 0);  // gx: dx vz-family, D-
-        sxa.job[h] = job(fam[1][j], DX[h], nullptr, nullptr, 1, 0);  // hx: dx vy-family, D-
-    }
-    StridedArgs& sya = c->a_sy;
-    strided_common(sya, 1, Py);
-    sya.mode = MODE_STORE;
-    sya.njobs = 3 * kFam;
-    sya.bnf = 3 * kFam;
-    sya.blk_stride = c->Nb;
-    for (int j = 0; j < kFam; ++j) {
-        const int g = kFam + j, h = 2 * kFam + j;
-        sya.job[j] = job(fam[1][j], DY[j], nullptr, nullptr, 0, 0);  // ey: dy vy-family, D+
-        sya.job[g] = job(fam[2][j], DY[g], nullptr, nullptr, 1, 0);  // gy: dy vz-family, D-
-        sya.job[h] = job(fam[0][j], DY[h], nullptr, nullptr, 1, 0);  // hy: dy vx-family, D-
-    }
+    // x derivatives -> bufA, y derivatives -> bufB; the jobs of two passes
+    // first, they take longest
+    auto stress_xy = [&](StressXYArgs& a, int axis, int P, float* out) {
+        a.nz = nz;
+        a.sx = sx; a.sy = sy;
+        a.axis = axis;
+        a.ztiles = (nz + P - 1) / P;
+        a.nplanes = axis == 0 ? ny : nx;
+        a.run = 1;
+        a.shot_stride = N;
+        a.tw = c->ax[axis].tw;
+        a.sym[0] = c->ax[axis].dp;
+        a.sym[1] = c->ax[axis].dm;
+        a.gs = c->coef + (long long)kG1 * c->Nb;
+        a.N = N;
+        a.out = out;
+        a.blk_stride = c->Nb;
+        a.njobs = 4;
+        const int shear[2] = {2, 1 - axis};  // components of the two sums, D-
+        for (int k = 0; k < 4; ++k) {
+            SJob& J = a.job[k];
+            const int comp = k < 2 ? shear[k] : axis;  // the axis' own component: D+, stored
+            J.n = k < 2 ? 2 : 1;
+            J.sym = k < 2 ? 1 : 0;
+            for (int f = 0; f < J.n; ++f) {  // pairs (A1 w, A2 w), (A2 v, A3 v)
+                const int q = k < 2 ? f : k - 2;
+                J.re[f] = fam[comp][q];
+                J.im[f] = fam[comp][kFam - 1 - q];
+            }
+            J.out[0] = k < 2 ? kFam + k : k - 2;
+            J.out[1] = kFam - 1 - J.out[0];
+        }
+    };
+    stress_xy(c->a_sx, 0, Px, c->bufA);
+    stress_xy(c->a_sy, 1, Py, c->bufB);
 
     // ---- stress z + update
     StressZArgs& sz = c->a_sz;
@@ -603,12 +604,12 @@ static int build_launch_config(qvti_ctx* c)
     for (int k = 0; k < 3; ++k)
         for (int j = 0; j < kFam; ++j) sz.fam[k][j] = fam[k][j];
     sz.dxb = c->bufA;
-    sz.dx_group = (long long)kFam * c->S * c->Nb;
     sz.blk_stride = c->Nb;
     sz.dyb = c->bufB;
     sz.g1 = c->coef;
     sz.gs = c->coef + (long long)kG1 * c->Nb;
     sz.g2 = g.vti ? c->coef + (long long)(kG1 + kGS) * c->Nb : nullptr;
+    sz.N = N;
     sz.wab = c->d_wab;
     for (int k = 0; k < 6; ++k) sz.sig[k] = sg[k];
     for (int k = 0; k < 3; ++k) sz.vel[k] = vv[k];
@@ -647,9 +648,10 @@ extern "C" int qvti_set_model(qvti_ctx* c, const float* velp, const float* gama_
     HIPCHK(hipSetDevice(c->device));
     const long long N = c->N;
     const size_t B = sizeof(float) * N;
-    // The model is staged in the spectral scratch buffer (kBufFields per shot,
-    // free between runs and ordered on the context's stream), so setting a
-    // model allocates nothing and never waits for other contexts' work.
+    // The model is staged in the spectral scratch buffers (7 fields in bufA,
+    // the S set in bufB: free between runs and ordered on the context's
+    // stream), so setting a model allocates nothing and never waits for other
+    // contexts' work.
     float* tmp = c->bufA;
     const int nin = c->g.vti ? 7 : 5;
     const float* srcs[7] = {velp, gama_p, vels, gama_s, rho, eps, delta};
@@ -685,7 +687,7 @@ extern "C" int qvti_set_model(qvti_ctx* c, const float* velp, const float* gama_
         ca.del = c->g.vti ? tmp + 6 * N : nullptr;
         ca.g1 = c->coef;
         ca.g2 = c->g.vti ? c->coef + (long long)(kG1 + kGS) * c->Nb : nullptr;
-        ca.s = tmp + 7 * N;  // free after the averages
+        ca.s = c->bufB;  // kFam fields, free after the averages
         const unsigned nb = (unsigned)std::min<long long>((N + kThreads - 1) / kThreads, 65535LL * 4);
         hipLaunchKernelGGL(k_coefficients, dim3(nb), dim3(kThreads), 0, c->stream, ca);
         AvgArgs aa;
@@ -759,10 +761,10 @@ static void launch_class(qvti_ctx* c, int cls)
         break;
     }
     case KC_STR_X:
-        X.deriv[MODE_STORE][pw_index(X, c->pw[cls])](strided(c->g_sx), st, c->a_sx);
+        X.stress_xy[pw_index(X, c->pw[cls])](strided(c->g_sx), st, c->a_sx);
         break;
     case KC_STR_Y:
-        Y.deriv[MODE_STORE][pw_index(Y, c->pw[cls])](strided(c->g_sy), st, c->a_sy);
+        Y.stress_xy[pw_index(Y, c->pw[cls])](strided(c->g_sy), st, c->a_sy);
         break;
     case KC_STR_Z:
         Z.stress_z[c->g.vti ? 1 : 0](dim3(xcd_grid(c->a_sz.ntiles, S, c->a_sz.run)), st, c->a_sz);
@@ -806,9 +808,9 @@ static void apply_tiles(qvti_ctx* c)
     const int rp = c->run_planes;
     c->a_vx.run = c->a_sx.run = c->a_vy.run = c->a_sy.run = c->a_yf.run = c->a_yi.run = c->a_xp.run = rp;
     c->a_vx.ztiles = zt(0, KC_VEL_X, 2); c->g_vx = grid(ny, c->a_vx.ztiles, rp);
-    c->a_sx.ztiles = zt(0, KC_STR_X, 2); c->g_sx = grid(ny, c->a_sx.ztiles, rp);
+    c->a_sx.ztiles = zt(0, KC_STR_X, 1); c->g_sx = grid(ny, c->a_sx.ztiles, rp);
     c->a_vy.ztiles = zt(1, KC_VEL_Y, 2); c->g_vy = grid(nx, c->a_vy.ztiles, rp);
-    c->a_sy.ztiles = zt(1, KC_STR_Y, 2); c->g_sy = grid(nx, c->a_sy.ztiles, rp);
+    c->a_sy.ztiles = zt(1, KC_STR_Y, 1); c->g_sy = grid(nx, c->a_sy.ztiles, rp);
     c->a_yf.ztiles = zt(1, KC_Y_FWD, 1); c->g_cy = grid(nx, c->a_yf.ztiles, rp);
     c->a_yi.ztiles = zt(1, KC_Y_INV, 1); c->g_yi = grid(nx, c->a_yi.ztiles, rp);
     c->a_xp.ztiles = zt(0, KC_XPASS, 1); c->g_xp = grid(ny, c->a_xp.ztiles, rp);
@@ -821,7 +823,7 @@ static int class_fields(const qvti_ctx* c, int cls)
     switch (cls) {
     case KC_VEL_X: case KC_VEL_Y: case KC_Y_FWD: case KC_XPASS: return 3;
     case KC_Y_INV: return c->a_yi.nfields;  // 4, or 7 in k-space mode
-    case KC_STR_X: case KC_STR_Y: return 3 * kFam;
+    case KC_STR_X: case KC_STR_Y: return 4;
     default: return 1;
     }
 }
@@ -1648,7 +1650,7 @@ extern "C" int qvti_set_kspace(qvti_ctx* c, float vref, float fcut, float vmax, 
     c->begun = 0;
     const bool on = vref > 0.f || fcut > 0.f;
     if (on && !c->H2) {
-        const int rc = dalloc(c, (void**)&c->H2, sizeof(float) * 6 * c->S * c->N);
+        const int rc = dalloc(c, (void**)&c->H2, sizeof(float) * 12 * c->S * c->N);
         if (rc) return rc;
     }
     c->ks = on;
@@ -1748,9 +1750,8 @@ extern "C" int qvti_kernel_bytes(qvti_ctx* c, int max_classes, double* bytes)
     b[KC_XPASS] = 6 * f + (c->ks ? 14 : 8) * f;
     b[KC_Y_INV] = (c->ks ? 28 : 16) * f;
     b[KC_Z_INV] = c->ks ? 14 * f + 12 * f : 8 * f + 6 * f;
-    b[KC_STR_X] = 24 * f;
-    b[KC_STR_Y] = 24 * f;
-    b[KC_STR_Z] = (12 + 24 + 12) * f + ncoef * 4.0 * c->N + 2 * (5 * sx + 5 * sy + 4 * sz);
+    b[KC_STR_X] = b[KC_STR_Y] = (3 * kFam + kDer) * f + kGS * 4.0 * c->N;
+    b[KC_STR_Z] = (12 + 2 * kDer + 12) * f + ncoef * 4.0 * c->N + 2 * (5 * sx + 5 * sy + 4 * sz);
     b[KC_RECORD] = 6.0 * 4 * c->total_rec;
     const int n = std::min(max_classes, (int)KC_COUNT);
     for (int k = 0; k < n; ++k) bytes[k] = b[k];

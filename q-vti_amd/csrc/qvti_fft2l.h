@@ -289,7 +289,7 @@ __host__ __device__ __forceinline__ void inv_la(float2 (&b)[G::N2], float2* pen,
     for (int ja = 0; ja < G::N2; ++ja) {
         float2 w = tw[ja * G::N1 + k1];
         w.y = -w.y;
-        pen[ja * G::ZS + k1] = (ja && k1) ? c_mul(b[ja], w) : b[ja];
+        pen[ja * G::ZS + k1] = ja ? c_mul(b[ja], w) : b[ja];  // (w = 1 exactly for k1 = 0)
     }
 }
 

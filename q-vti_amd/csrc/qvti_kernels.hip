@@ -15,6 +15,11 @@ void l_deriv(dim3 grid, hipStream_t st, const StridedArgs& a)
 {
     hipLaunchKernelGGL((k2_deriv_strided<G, MODE>), grid, dim3(G::T), 0, st, a);
 }
+template <class G>
+void l_stress_xy(dim3 grid, hipStream_t st, const StressXYArgs& a)
+{
+    hipLaunchKernelGGL(k2_stress_xy<G>, grid, dim3(G::T), 0, st, a);
+}
 template <class G, int DIR>
 void l_cfft(dim3 grid, hipStream_t st, const CStridedArgs& a)
 {
@@ -55,6 +60,7 @@ constexpr bool pw_ok()
 }
 
 using DerivFn = void (*)(dim3, hipStream_t, const StridedArgs&);
+using StressXYFn = void (*)(dim3, hipStream_t, const StressXYArgs&);
 using CfftFn = void (*)(dim3, hipStream_t, const CStridedArgs&);
 using XpassFn = void (*)(dim3, hipStream_t, const XPassArgs&);
 
@@ -62,6 +68,12 @@ template <int A, int B, int PW, int MODE>
 DerivFn deriv_fn()
 {
     if constexpr (pw_ok<A, B, PW>()) return &l_deriv<L2<A, B, PW>, MODE>;
+    else return nullptr;
+}
+template <int A, int B, int PW>
+StressXYFn stress_xy_fn()
+{
+    if constexpr (pw_ok<A, B, PW>()) return &l_stress_xy<L2<A, B, PW>>;
     else return nullptr;
 }
 template <int A, int B, int PW, int DIR>
@@ -96,10 +108,11 @@ LenOps make_ops()
         A * B, A, B, G::P, StressTile<G>::R,
         {pencils<A, B, kW0>(), pencils<A, B, kW1>(), pencils<A, B, kW2>()},
         {L2<A, B, kW0>::T, L2<A, B, kW1>::T, L2<A, B, kW2>::T},
-        {{deriv_fn<A, B, kW0, MODE_STORE>(), deriv_fn<A, B, kW1, MODE_STORE>(), deriv_fn<A, B, kW2, MODE_STORE>()},
+        {{deriv_fn<A, B, kW0, MODE_STORE>(), nullptr, nullptr},
          {deriv_fn<A, B, kW0, MODE_VEL_FIRST>(), deriv_fn<A, B, kW1, MODE_VEL_FIRST>(),
           deriv_fn<A, B, kW2, MODE_VEL_FIRST>()},
          {deriv_fn<A, B, kW0, MODE_VEL_ACC>(), deriv_fn<A, B, kW1, MODE_VEL_ACC>(), deriv_fn<A, B, kW2, MODE_VEL_ACC>()}},
+        {stress_xy_fn<A, B, kW0>(), stress_xy_fn<A, B, kW1>(), stress_xy_fn<A, B, kW2>()},
         {{cfft_fn<A, B, kW0, -1>(), cfft_fn<A, B, kW1, -1>(), cfft_fn<A, B, kW2, -1>()},
          {cfft_fn<A, B, kW0, 1>(), cfft_fn<A, B, kW1, 1>(), cfft_fn<A, B, kW2, 1>()}},
         {{xpass_fn<A, B, kW0, false>(), xpass_fn<A, B, kW1, false>(), xpass_fn<A, B, kW2, false>()},

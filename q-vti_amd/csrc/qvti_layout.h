@@ -27,5 +27,56 @@ constexpr int kFam = 4;
 // = {S-bar: o0..o3}, G2 = {H: o0, o1; D: o0, o1} (VTI).  The stress update
 // derives o2 and o3 of the sets P, S, H and D (set_coeffs in qvti_aux.h).
 constexpr int kG1 = 5, kGS = kFam, kG2 = 4;
+// x- (y-) derivatives that the stress update reads: the four of the family
+// whose component is the axis, and the two S-bar-weighted shear sums
+constexpr int kDer = kFam + 2;
+
+// Global memory through a uniform row pointer and a per-lane byte offset.  The
+// empty asm keeps the row's address a value of its own in SGPRs, so that the
+// access is one instruction with one 32-bit offset register shared by all rows
+// (global_load v, v, s[:]; imm, a compile-time byte offset, rides along).  Without it the compiler folds the lane offset into
+// the base and keeps a 64-bit address register pair, made by a 64-bit add, for
+// every row.  Offsets stay below 4 GiB: within one shot's field (512^3
+// floats) or blocked group of kDer fields.
+typedef __attribute__((address_space(1))) char gchar;
+typedef float vfloat2 __attribute__((ext_vector_type(2)));
+struct Row {
+    gchar* p;
+};
+template <class T>
+__device__ __forceinline__ Row row_at(const T* base, long long elem)
+{
+    unsigned long long u = reinterpret_cast<unsigned long long>(base + elem);
+    asm("" : "+s"(u));
+    return Row{(gchar*)u};
+}
+// The lane offset, made opaque where it is used: the 32-to-64-bit extension
+// then sits next to the accesses and folds into them, instead of being hoisted
+// out of loops into a register pair.
+__device__ __forceinline__ unsigned lane_off(unsigned off)
+{
+    asm volatile("" : "+v"(off));
+    return off;
+}
+__device__ __forceinline__ float ld1(Row r, unsigned off, int imm = 0)
+{
+    return *(__attribute__((address_space(1))) const float*)(r.p + off + imm);
+}
+__device__ __forceinline__ float2 ld2(Row r, unsigned off, int imm = 0)
+{
+    const vfloat2 v = *(__attribute__((address_space(1))) const vfloat2*)(r.p + off + imm);
+    return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ void st1(Row r, unsigned off, float v, int imm = 0)
+{
+    *(__attribute__((address_space(1))) float*)(r.p + off + imm) = v;
+}
+__device__ __forceinline__ void st2(Row r, unsigned off, float2 v, int imm = 0)
+{
+    vfloat2 w;
+    w.x = v.x;
+    w.y = v.y;
+    *(__attribute__((address_space(1))) vfloat2*)(r.p + off + imm) = w;
+}
 
 }  // namespace qvti

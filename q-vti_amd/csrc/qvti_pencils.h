@@ -8,7 +8,7 @@
 //                        -> k2_deriv_strided(y, VEL_ACC)
 //                        -> k2_vel_z (z-derivatives, velocity update, forward z-FFTs of v and w)
 //   stress half-step     k2_cfft_strided(y, fwd) -> k2_xpass -> k2_cfft_strided(y, inv)
-//                        -> k2_zrows (inverse z) -> k2_deriv_strided(x, STORE) -> k2_deriv_strided(y, STORE)
+//                        -> k2_zrows (inverse z) -> k2_stress_xy(x) -> k2_stress_xy(y)
 //                        -> k2_stress_z (z-derivatives, stress update, source injection)
 //   receivers            k_record
 //
@@ -28,8 +28,8 @@
 //    everywhere (q_coeffs in qvti_aux.h), so only A1 w and A3 v need the full
 //    3-D transform - three forward and four inverse complex transforms.  With
 //    five fields {A1 v, v, A3 v, A1 dv, dv} per component it was three and
-//    five, and 248 floats per cell and step through HBM instead of 204 (VTI,
-//    with the coefficients of set_coeffs).
+//    five, and 248 floats per cell and step through HBM instead of 188 (VTI,
+//    with the coefficients of set_coeffs and the shear sums of k2_stress_xy).
 //    Fields that share a complex transform are scaled (alpha and the length
 //    scale of A1 and A3, powers of two) so that the FP32 rounding of one does
 //    not swamp the other where it matters (q_coeffs).
@@ -123,7 +123,7 @@ __device__ __forceinline__ void load_twiddles(float2* tws, const float2* tw)
 // 1-D shift-derivatives of real fields along a strided axis (x or y).  Tile:
 // G::P complex pencils = 2*G::P adjacent real z-columns at one value of the
 // other in-plane index, loaded as float2 (two real pencils per complex one).
-// Modes: STORE out = d; VEL_FIRST out = d + phi; VEL_ACC out = acc + d + phi,
+// Modes: STORE out = d (standalone derivative); VEL_FIRST out = d + phi; VEL_ACC out = acc + d + phi,
 // with the velocity C-PML memory variable phi updated on the axis' face slabs
 // (cuviscoelas_3D.cu:1049-1074).
 struct DJob {
@@ -147,16 +147,9 @@ struct StridedArgs {
     const float2* sym[2];
     const float *pa, *pb, *pah, *pbh;
     int njobs;
-    // STORE mode output layout: 0 = natural [shot][N] per job; nf > 0 =
-    // blocked group of nf fields per shot ([shot][N/64][nf][64], see
-    // blk_index), each job's out pointing at its field (group base + f*64)
-    int bnf;
-    // per-shot length of a blocked group's field: N rounded up to whole
-    // 64-cell blocks (shot s of an nf-field group starts at s * nf * blk_stride)
-    long long blk_stride;
     // step counter advanced by this launch (the first kernel of a step), or null
     int* tick;
-    DJob job[3 * kFam];
+    DJob job[3];
 };
 
 template <class G, int MODE>
@@ -216,22 +209,10 @@ void k2_deriv_strided(StridedArgs a)
             if (act1 && zok) {
                 float2 d[G::N1];
                 inv_lb<G>(d, pen, jj);
-                if (a.bnf) {
-                    // blocked group: (ip, ip+1) share a 64-cell block (ip even)
-                    float* ob = J.out + (long long)shot * a.bnf * a.blk_stride;
-                    const unsigned ip0 = (unsigned)(poff + jj * astride + zc);
-                    const unsigned bs = (unsigned)(kBlk * a.bnf);
 #pragma unroll
-                    for (int j1 = 0; j1 < G::N1; ++j1) {
-                        const unsigned ip = ip0 + (unsigned)(G::N2 * j1 * astride);
-                        *reinterpret_cast<float2*>(ob + ((ip >> 6) * bs + (ip & 63u))) = d[j1];
-                    }
-                } else {
-#pragma unroll
-                    for (int j1 = 0; j1 < G::N1; ++j1) {
-                        const long long urow = ubase + (long long)(G::N2 * j1) * astride;
-                        *reinterpret_cast<float2*>(J.out + urow + voff) = d[j1];
-                    }
+                for (int j1 = 0; j1 < G::N1; ++j1) {
+                    const long long urow = ubase + (long long)(G::N2 * j1) * astride;
+                    *reinterpret_cast<float2*>(J.out + urow + voff) = d[j1];
                 }
             }
         } else {
@@ -295,6 +276,151 @@ void k2_deriv_strided(StridedArgs a)
                     }
                     asm volatile("" ::: "memory");  // the next chunk's loads stay after this chunk
                 }
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------
+// Stress half-step: derivatives of the family fields along a strided axis.
+// Tile: G::P adjacent z-columns at one value of the other in-plane index, one
+// complex pencil per column: a pass transforms two fields of one component,
+// (A1 w + i A2 w) or (A2 v + i A3 v).  A job of one pass stores the two
+// derivatives; a job of two passes stores the one real field
+//   sum_j S-bar_j D(in_j)
+// of the component's four derivatives, the only form in which the stress
+// update uses the shear derivatives: six fields per axis go to HBM and back
+// instead of twelve, for four coefficient reads (24 -> 22 floats per cell here,
+// 61 -> 49 in the stress update).  Pairing fields, and not two columns of one
+// field as k2_deriv_strided does, halves the passes of a sum and the
+// accumulators that live through the transforms (N1 instead of 2 N1 registers).
+struct SJob {
+    const float* re[2];
+    const float* im[2];
+    int n;    // passes: 1 or 2
+    int sym;  // 0: D+, 1: D-
+    int out[2];  // n = 1: fields of the output group; n = 2: out[0] the sum's field
+};
+
+struct StressXYArgs {
+    int nz;
+    long long sx, sy;
+    int axis;  // 0: x (stride sx), 1: y (stride sy)
+    int ztiles, nplanes, run;  // workgroup placement: plane_tile()
+    long long shot_stride;
+    const float2* tw;
+    const float2* sym[2];
+    const float* gs;  // S-bar coefficients [kGS][N]
+    long long N;
+    float* out;       // blocked group [shot][N/64][kDer][64]
+    // per-shot length of a blocked group's field: N rounded up to whole 64-cell blocks
+    long long blk_stride;
+    int njobs;
+    SJob job[4];
+};
+
+template <class G>
+// What bounds it at 256^3: 26 floats per cell (each sum reads S-bar) in 370 us
+// along x, 4.7 TB/s, with the VALU busy for about half of that time; 2, 3 and
+// 4 waves per SIMD measure the same there (370-375 us), at 400x400x200 3 waves
+// are best (985 us; 1045 us with 2), hence the bounds.
+__global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(G::NMAX <= 16 ? 4 : 3)))
+void k2_stress_xy(StressXYArgs a)
+{
+    __shared__ float2 lds[G::P * G::PS];
+    __shared__ float2 tws[G::TWN];
+    const int tid = threadIdx.x, shot = blockIdx.y;
+    const PlaneTile pt = plane_tile(a.ztiles, a.nplanes, a.run);
+    if (pt.plane < 0) return;
+    const int other = pt.plane;
+    const int p = tid % G::P, jj = tid / G::P;
+    const int zc = pt.zt * G::P + p;
+    const int nz = a.nz;
+    const bool zok = zc < nz;
+    // columns past nz (last tile of a ragged z) load a valid column and are
+    // never stored, so the loads need no branch
+    const int zl = zok ? zc : nz - 1;
+    const bool act1 = jj < G::N2, act2 = jj < G::N1;
+    const int astride = (int)(a.axis == 0 ? a.sx : a.sy);
+    const long long poff = a.axis == 0 ? (long long)other * a.sy : (long long)other * a.sx;
+    const long long ubase = (long long)shot * a.shot_stride + poff;
+    const unsigned lvoff = 4u * (unsigned)(jj * astride + zl);  // lane byte offset from a uniform row
+    float2* pen = lds + p * G::PS;
+    load_twiddles<G>(tws, a.tw);
+    for (int jb = blockIdx.z; jb < a.njobs; jb += gridDim.z) {
+        const int np = a.job[jb].n;
+        float acc[G::N1];
+#pragma unroll
+        for (int j1 = 0; j1 < G::N1; ++j1) acc[j1] = 0.f;
+#pragma unroll 1
+        for (int f = 0; f < np; ++f) {
+            const float* re = a.job[jb].re[f] + ubase;
+            const float* im = a.job[jb].im[f] + ubase;
+            __syncthreads();
+            if (act1) {
+                float2 v[G::N1];
+                const unsigned o = lane_off(lvoff);
+#pragma unroll
+                for (int j1 = 0; j1 < G::N1; ++j1) {
+                    const long long row = (long long)(j1 * G::N2) * astride;
+                    v[j1] = make_float2(ld1(row_at(re, row), o), ld1(row_at(im, row), o));
+                }
+                fwd_l1<G>(v, pen, tws, jj);
+            }
+            __syncthreads();
+            float2 b[G::N2];
+            if (act2) {
+                fwd_l2<G>(b, pen, jj);
+                const Row S = row_at(a.sym[a.job[jb].sym], 0);
+                const unsigned o = lane_off(8u * jj);
+#pragma unroll
+                for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = c_mul(b[k2], ld2(S, o, 8 * G::N1 * k2));
+            }
+            __syncthreads();
+            if (act2) inv_la<G>(b, pen, tws + G::T2OFF, jj);
+            // The S-bar values of a sum are loaded here, ahead of the last
+            // exchange: their round trip overlaps the barrier and the inverse
+            // transform.  Fields of the pass: (0, 3) for (A1 w, A2 w), (1, 2)
+            // for (A2 v, A3 v).
+            float2 c[G::N1];
+            if (np > 1 && act1) {
+                const float* g0 = a.gs + f * a.N + poff;
+                const float* g1 = a.gs + (kFam - 1 - f) * a.N + poff;
+                const unsigned o = lane_off(lvoff);
+#pragma unroll
+                for (int j1 = 0; j1 < G::N1; ++j1) {
+                    const long long row = (long long)(j1 * G::N2) * astride;
+                    c[j1] = make_float2(ld1(row_at(g0, row), o), ld1(row_at(g1, row), o));
+                }
+            }
+            __syncthreads();
+            if (act1 && zok) {
+                float2 d[G::N1];
+                inv_lb<G>(d, pen, jj);
+                if (np == 1) {
+                    const Row ore = row_at(a.out, (long long)shot * kDer * a.blk_stride + a.job[jb].out[0] * kBlk);
+                    const Row oim = row_at(a.out, (long long)shot * kDer * a.blk_stride + a.job[jb].out[1] * kBlk);
+                    const unsigned ip0 = lane_off((unsigned)(poff + jj * astride + zc));
+#pragma unroll
+                    for (int j1 = 0; j1 < G::N1; ++j1) {
+                        const unsigned ip = ip0 + (unsigned)(G::N2 * j1 * astride);
+                        const unsigned o = 4u * ((ip >> 6) * (unsigned)(kBlk * kDer) + (ip & 63u));
+                        st1(ore, o, d[j1].x);
+                        st1(oim, o, d[j1].y);
+                    }
+                } else {
+#pragma unroll
+                    for (int j1 = 0; j1 < G::N1; ++j1) acc[j1] += c[j1].x * d[j1].x + c[j1].y * d[j1].y;
+                }
+            }
+        }
+        if (np > 1 && act1 && zok) {
+            const Row ob = row_at(a.out, (long long)shot * kDer * a.blk_stride + a.job[jb].out[0] * kBlk);
+            const unsigned ip0 = lane_off((unsigned)(poff + jj * astride + zc));
+#pragma unroll
+            for (int j1 = 0; j1 < G::N1; ++j1) {
+                const unsigned ip = ip0 + (unsigned)(G::N2 * j1 * astride);
+                st1(ob, 4u * ((ip >> 6) * (unsigned)(kBlk * kDer) + (ip & 63u)), acc[j1]);
             }
         }
     }
@@ -881,16 +1007,14 @@ struct StressZArgs {
     // themselves) unless the k-space correction is on
     const float* fam[3][kFam];
     float* vel[3];  // vx vy vz: force sources are added here
-    // x- and y-derivatives in blocked groups:
-    //   dxb: three groups of 4, dx_group floats apart: ex (dx vx-family),
-    //        gx (dx vz-family), hx (dx vy-family), each [shot][N/64][4][64]
-    //   dyb: one group of 12 per shot: ey 0-3 (dy vy-family), gy 4-7 (dy
-    //        vz-family), hy 8-11 (dy vx-family)
+    // x- and y-derivatives, blocked groups [shot][N/64][kDer][64]:
+    //   dxb: ex 0-3 (dx vx-family), sum_j S-bar_j dx of the vz family 4, of the vy family 5
+    //   dyb: ey 0-3 (dy vy-family), sum_j S-bar_j dy of the vz family 4, of the vx family 5
     const float *dxb, *dyb;
-    long long dx_group;
     long long blk_stride;  // per-shot field length of the blocked groups (N rounded up to 64)
     // coefficient groups G1, GS and G2 (VTI; else null)
     const float *g1, *gs, *g2;
+    long long N;
     const float* wab;  // {alpha, alpha kappa, s4}
     float* sig[6];  // pxx pyy pzz pxy pxz pyz
     float* phx[5];
@@ -1001,9 +1125,8 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
     // uniform block bases; per-cell offsets below are unsigned 32-bit
     const long long cbase = r0 * n;          // flat index of the tile's first cell
     const long long fbase = soff + cbase;    // per-shot natural fields
-    constexpr int kDY = 3 * kFam;  // y-derivatives per cell
-    const float* __restrict__ dxs = a.dxb + (long long)shot * kFam * a.blk_stride;
-    const float* __restrict__ dys = a.dyb + (long long)shot * kDY * a.blk_stride;
+    const float* __restrict__ dxs = a.dxb + (long long)shot * kDer * a.blk_stride;
+    const float* __restrict__ dys = a.dyb + (long long)shot * kDer * a.blk_stride;
     constexpr bool vti = VTI;  // G2 (H, D sets) present: a compile-time choice keeps the loads branch-free
     const long long sxb = (long long)shot * a.slabx_stride, syb = (long long)shot * a.slaby_stride,
                     szb = (long long)shot * a.slabz_stride;
@@ -1024,10 +1147,10 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
             // fields at immediate offsets f*64 floats
             const unsigned ip = (unsigned)cbase + o;
             const unsigned blk = ip >> 6, in = ip & 63u;
-            const float* __restrict__ dxp = dxs + (blk * (kBlk * kFam) + in);
-            const float* __restrict__ dyp = dys + (blk * (kBlk * kDY) + in);
+            const float* __restrict__ dxp = dxs + (blk * (kBlk * kDer) + in);
+            const float* __restrict__ dyp = dys + (blk * (kBlk * kDer) + in);
             const float* __restrict__ g1p = a.g1 + (blk * (kBlk * kG1) + in);
-            const float* __restrict__ gsp = a.gs + (blk * (kBlk * kGS) + in);
+            const float* __restrict__ gsp = a.gs + ip;
             const float* __restrict__ g2p = vti ? a.g2 + (blk * (kBlk * kG2) + in) : nullptr;
             float oP[kFam], oS[kFam], oH[kFam], oD[kFam];
             {
@@ -1042,12 +1165,15 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
             float A[14];
 #pragma unroll
             for (int k = 0; k < 14; ++k) A[k] = 0.f;
+            A[9] = dxp[kFam * kBlk];         // sb_zx  (dx vz)
+            A[11] = dxp[(kFam + 1) * kBlk];  // sb_yx  (dx vy)
+            A[13] = dyp[kFam * kBlk];        // sb_zy  (dy vz)
+            A[10] = dyp[(kFam + 1) * kBlk];  // sb_xy  (dy vx)
 #pragma unroll
             for (int jf = 0; jf < kFam; ++jf) {
                 const float ez = S(fz[jf]), gz = S(fgx[jf]), hz = S(fhy[jf]);
-                const float ex = dxp[jf * kBlk], gx = dxp[a.dx_group + jf * kBlk], hx = dxp[2 * a.dx_group + jf * kBlk];
-                const float ey = dyp[jf * kBlk], gy = dyp[(kFam + jf) * kBlk], hy = dyp[(2 * kFam + jf) * kBlk];
-                const float c33 = oP[jf], cs = oS[jf], csb = gsp[jf * kBlk];
+                const float ex = dxp[jf * kBlk], ey = dyp[jf * kBlk];
+                const float c33 = oP[jf], cs = oS[jf], csb = gsp[jf * a.N];
                 const float c11 = vti ? oH[jf] : c33, c13 = vti ? oD[jf] : c33;
                 const float c12 = c11 - 2 * cs, c13d = c13 - 2 * cs;
                 A[0] += c11 * ex;   // s11x
@@ -1059,11 +1185,7 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
                 A[6] += c13d * ez;  // s13z
                 A[7] += c33 * ez;   // s33z
                 A[8] += csb * gz;   // sb_xz  (dz vx)
-                A[9] += csb * gx;   // sb_zx  (dx vz)
-                A[10] += csb * hy;  // sb_xy  (dy vx)
-                A[11] += csb * hx;  // sb_yx  (dx vy)
                 A[12] += csb * hz;  // sb_yz  (dz vy)
-                A[13] += csb * gy;  // sb_zy  (dy vz)
             }
             // Every load of the cell is issued before its first store: the
             // stress and C-PML arrays are distinct, but the compiler cannot

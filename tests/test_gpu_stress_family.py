@@ -54,3 +54,35 @@ def test_stress_family_matches_the_oracle(nx, ny, nz, vti, media, ratio):
           % (nx, ny, nz, media, ratio, rel_l2(st, ref["state"]), max(errs)))
     assert rel_l2(st[:3], ref["state"][:3]) < TOL
     assert rel_l2(st[3:], ref["state"][3:]) < TOL
+
+
+# strided lengths next to row lengths that leave a partial last tile at every
+# tile width, and every pencil count per workgroup (8 to 64 columns)
+STRIDED = [(16, 24, 18), (64, 18, 50), (18, 90, 30), (128, 16, 54), (20, 200, 18), (250, 16, 20), (16, 400, 36),
+           (486, 18, 16), (18, 512, 30)]
+
+
+@pytest.mark.parametrize("nx,ny,nz", STRIDED)
+def test_strided_stress_derivatives_match_the_oracle(nx, ny, nz):
+    """Shear sums and stored derivatives along x and y (two shots, so that the
+    per-shot offsets count): within the bound at the narrowest tiles, and the
+    same bits at every tile width and split."""
+    shot, model = small_case(nx, ny, nz, 4, 8, O.SRC_EXPLOSIVE, True, seed=nx + ny)
+    ref = O.run(shot, model, "f64", state=True)
+    got = []
+    for mode in (0, 2, 4, 16, 18, 20):
+        with qvti.Engine(nx, ny, nz, shot["pml"], shot["dx"], shot["dy"], shot["dz"], shot["dt"], shot["f0"],
+                         shot["w0"], vti=True, max_shots=2) as e:
+            e.set_autotune(mode)
+            e.set_model_dict(model)
+            one = [qvti.make_shot(shot["src_kind"], (shot["sx"] + d, shot["sy"], shot["sz"]), shot["rx"], shot["ry"],
+                                  shot["rz"]) for d in (1, 0)]
+            e.begin(shot["nt"], shot["rik"], one)
+            e.step(shot["nt"])
+            e.finish()
+            got.append(e.state(1))
+    err = rel_l2(got[0], ref["state"])
+    print("%dx%dx%d: state vs FP64 oracle %.2e" % (nx, ny, nz, err))
+    assert err < TOL
+    for st in got[1:]:
+        assert np.array_equal(st, got[0])

@@ -316,8 +316,9 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
         axis_symbols(A.n, A.d, dp, dm, kf);
         pml_profile(A.n, g->pml, A.d, g->f0, pa, pb, pah, pbh);
         rc = rc ? rc : upload(c, &A.tw, tw);
+        dp.insert(dp.end(), dm.begin(), dm.end());  // D+ then D-, one allocation
         rc = rc ? rc : upload(c, &A.dp, dp);
-        rc = rc ? rc : upload(c, &A.dm, dm);
+        A.dm = rc ? nullptr : A.dp + A.n;
         rc = rc ? rc : upload(c, &A.kf, kf);
         rc = rc ? rc : upload(c, &A.a, pa);
         rc = rc ? rc : upload(c, &A.b, pb);
@@ -597,7 +598,7 @@ static int build_launch_config(qvti_ctx* c)
     sz.dt = g.dt;
     sz.shot_stride = N;
     sz.slabx_stride = c->slab[0]; sz.slaby_stride = c->slab[1]; sz.slabz_stride = c->slab[2];
-    sz.tw = Z.tw; sz.symp = Z.dp; sz.symm = Z.dm;
+    sz.tw = Z.tw; sz.symp = Z.dp; sz.symm_off = (unsigned)sizeof(float2) * Z.n;
     sz.pax = X.a; sz.pbx = X.b; sz.paxh = X.ah; sz.pbxh = X.bh;
     sz.pay = Y.a; sz.pby = Y.b; sz.payh = Y.ah; sz.pbyh = Y.bh;
     sz.paz = Z.a; sz.pbz = Z.b; sz.pazh = Z.ah; sz.pbzh = Z.bh;

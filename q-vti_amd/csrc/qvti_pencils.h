@@ -177,6 +177,7 @@ void k2_deriv_strided(StridedArgs a)
     const int astride = (int)(a.axis == 0 ? a.sx : a.sy);
     const long long poff = a.axis == 0 ? (long long)other * a.sy : (long long)other * a.sx;  // plane offset in the shot
     const long long ubase = (long long)shot * a.shot_stride + poff;
+    const unsigned lvoff = 4u * (unsigned)(jj * astride + zl);  // lane byte offset from a uniform row
     float2* pen = lds + p * G::PS;
     load_twiddles<G>(tws, a.tw);
     for (int jb = blockIdx.z; jb < a.njobs; jb += gridDim.z) {
@@ -184,36 +185,32 @@ void k2_deriv_strided(StridedArgs a)
         __syncthreads();
         if (act1) {
             float2 v[G::N1];
-            // uniform row pointer (SGPRs) + one unsigned 32-bit lane offset
-            const unsigned voff = (unsigned)(jj * astride + zl);
+            const unsigned o = lane_off(lvoff);
 #pragma unroll
-            for (int j1 = 0; j1 < G::N1; ++j1) {
-                const float* __restrict__ rp = J.in + ubase + (long long)(j1 * G::N2) * astride;
-                v[j1] = *reinterpret_cast<const float2*>(rp + voff);
-            }
+            for (int j1 = 0; j1 < G::N1; ++j1)
+                v[j1] = ld2(row_at(J.in, ubase + (long long)(j1 * G::N2) * astride), o);
             fwd_l1<G>(v, pen, tws, jj);
         }
         __syncthreads();
         float2 b[G::N2];
         if (act2) {
             fwd_l2<G>(b, pen, jj);
-            const float2* __restrict__ S = a.sym[J.sym];
+            const Row S = row_at(a.sym[J.sym], 0);
+            const unsigned o = lane_off(8u * jj);
 #pragma unroll
-            for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = c_mul(b[k2], S[jj + G::N1 * k2]);
+            for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = c_mul(b[k2], ld2(S, o, 8 * G::N1 * k2));
         }
         __syncthreads();
         if (act2) inv_la<G>(b, pen, tws + G::T2OFF, jj);
         __syncthreads();
-        const unsigned voff = (unsigned)(jj * astride + zc);
         if (MODE == MODE_STORE) {
             if (act1 && zok) {
                 float2 d[G::N1];
                 inv_lb<G>(d, pen, jj);
+                const unsigned o = lane_off(lvoff);
 #pragma unroll
-                for (int j1 = 0; j1 < G::N1; ++j1) {
-                    const long long urow = ubase + (long long)(G::N2 * j1) * astride;
-                    *reinterpret_cast<float2*>(J.out + urow + voff) = d[j1];
-                }
+                for (int j1 = 0; j1 < G::N1; ++j1)
+                    st2(row_at(J.out, ubase + (long long)(G::N2 * j1) * astride), o, d[j1]);
             }
         } else {
             // The C-PML branch differs per element: park the pencil's result in
@@ -231,9 +228,9 @@ void k2_deriv_strided(StridedArgs a)
                 // being hoisted (and held in registers through the FFTs)
                 int jl = jj;
                 asm volatile("" : "+v"(jl));
-                const float* __restrict__ pa = J.half ? a.pah : a.pa;
-                const float* __restrict__ pb = J.half ? a.pbh : a.pb;
-                float2* __restrict__ phs = reinterpret_cast<float2*>(J.phi + (long long)shot * a.slab_stride);
+                const unsigned o = lane_off(lvoff);  // (zok: zl == zc)
+                const Row pa = row_at(J.half ? a.pah : a.pa, 0), pb = row_at(J.half ? a.pbh : a.pb, 0);
+                const Row phs = row_at(J.phi, (long long)shot * a.slab_stride);
                 // Chunks of CH elements: every load of a chunk (unconditional
                 // and in bounds - a non-slab element reads slab plane 0) before
                 // its stores, so the chunk's memory round trips overlap.
@@ -241,7 +238,7 @@ void k2_deriv_strided(StridedArgs a)
 #pragma unroll
                 for (int c0 = 0; c0 < G::N1; c0 += CH) {
                     float2 rr[CH], q[CH];
-                    int sidx[CH];
+                    unsigned sidx[CH];
                     bool upd[CH];
 #pragma unroll
                     for (int jc = 0; jc < CH; ++jc) {
@@ -253,16 +250,16 @@ void k2_deriv_strided(StridedArgs a)
                         const int iy = a.axis == 0 ? other : i;
                         upd[jc] = (i < pml || i >= n - pml) && ix < a.nx - 1 && iy < a.ny - 1;
                         const int si = i < pml ? i : (i >= n - pml ? i - (n - 2 * pml) : 0);
-                        sidx[jc] = (a.axis == 0 ? (si * a.ny + iy) * nz + zc : (ix * 2 * pml + si) * nz + zc) / 2;
-                        const float2 q0 = phs[sidx[jc]];
-                        const float A = pa[i], B = pb[i];
+                        sidx[jc] = 4u * (unsigned)((a.axis == 0 ? si * a.ny + iy : ix * 2 * pml + si) * nz + zc);
+                        const float2 q0 = ld2(phs, sidx[jc]);
+                        const float A = ld1(pa, 4u * jl, 4 * G::N2 * j1), B = ld1(pb, 4u * jl, 4 * G::N2 * j1);
                         q[jc] = q0;
                         if (upd[jc]) {
                             if (zc < nz - 1) { q[jc].x = q0.x + a.dt * (-A * q0.x - B * r.x); r.x = r.x + q[jc].x; }
                             if (zc + 1 < nz - 1) { q[jc].y = q0.y + a.dt * (-A * q0.y - B * r.y); r.y = r.y + q[jc].y; }
                         }
                         if (MODE == MODE_VEL_ACC) {
-                            const float2 ac = *reinterpret_cast<const float2*>(J.acc + urow + voff);
+                            const float2 ac = ld2(row_at(J.acc, urow), o);
                             r = make_float2(ac.x + r.x, ac.y + r.y);
                         }
                         rr[jc] = r;
@@ -271,8 +268,8 @@ void k2_deriv_strided(StridedArgs a)
                     for (int jc = 0; jc < CH; ++jc) {
                         const int j1 = c0 + jc;
                         const long long urow = ubase + (long long)(G::N2 * j1) * astride;
-                        if (upd[jc]) phs[sidx[jc]] = q[jc];
-                        *reinterpret_cast<float2*>(J.out + urow + voff) = rr[jc];
+                        if (upd[jc]) st2(phs, sidx[jc], q[jc]);
+                        st2(row_at(J.out, urow), o, rr[jc]);
                     }
                     asm volatile("" ::: "memory");  // the next chunk's loads stay after this chunk
                 }
@@ -468,21 +465,21 @@ struct VelZArgs {
 // C-PML memory variable on the z-slab, v += b * (acc + dz + phi), dv = v_new
 // - v_old (+ the previous step's source at the injection cell), w = wa v +
 // wb dv.  Writes v and w (rows with rowdom / ok1 only), returns (v_new, w).
-// The pointers are row bases (v, w, acc, bu: the row; ph: the row's z-slab of 2*pml values)
-// and never alias, which lets the compiler issue the loads of later elements
-// before the stores of earlier ones.
+// v, w, acc, bu, inj: uniform tile bases, `row` the byte offset of the lane's
+// row in them; ph: the shot's z-slabs, phrow the byte offset of the row's
+// 2*pml values.
 template <class G, bool INJ>
 __device__ __forceinline__ void vz_component(float2 (&out)[G::N1], const float2 (&d)[G::N1], const bool imag,
-                                             float* __restrict__ v, float* __restrict__ w, const float wa, const float wb,
-                                             const float* __restrict__ acc, const float* __restrict__ bu,
-                                             float* __restrict__ ph, const float* __restrict__ pa,
-                                             const float* __restrict__ pb, const int j, const int pml,
+                                             const Row v, const Row w, const float wa, const float wb, const Row acc,
+                                             const Row bu, const Row ph, const unsigned phrow, const Row pa,
+                                             const Row pb, const unsigned row, const int j, const int pml,
                                              const float dt, const bool rowdom, const bool ok1, const int src_iz,
-                                             const float sprev, const float* __restrict__ inj)
+                                             const float sprev, const Row inj)
 {
     constexpr int n = G::N;
-    int jl = j;  // opaque per call: nothing is shared (and held) across components
-    asm volatile("" : "+v"(jl));
+    // opaque per call: nothing is shared (and held) across components
+    const int jl = (int)lane_off((unsigned)j);
+    const unsigned o = lane_off(row + 4u * j);
     // all loads and arithmetic first (every load unconditional and in bounds:
     // ph is a valid slab row even where it is not used), all stores after, so
     // no load waits behind a store or a branch
@@ -493,12 +490,12 @@ __device__ __forceinline__ void vz_component(float2 (&out)[G::N1], const float2 
     float qn[CH];
 #pragma unroll
     for (int jc = 0; jc < CH; ++jc) {
-        const int j1 = c0 + jc;
+        const int j1 = c0 + jc, im = 4 * G::N2 * j1;
         const int iz = jl + G::N2 * j1;
-        const float vold = v[iz], bb = bu[iz], ac = acc[iz];
+        const float vold = ld1(v, o, im), bb = ld1(bu, o, im), ac = ld1(acc, o, im);
         const bool slab = iz < pml || iz >= n - pml;
         const int si = iz < pml ? iz : (iz >= n - pml ? iz - (n - 2 * pml) : 0);
-        const float q0 = ph[si], A = pa[iz], B = pb[iz];
+        const float q0 = ld1(ph, phrow + 4u * si), A = ld1(pa, 4u * jl, im), B = ld1(pb, 4u * jl, im);
         const bool upd = rowdom && iz < n - 1;
         float dz = imag ? d[j1].y : d[j1].x;
         qn[jc] = q0 + dt * (-A * q0 - B * dz);
@@ -506,17 +503,17 @@ __device__ __forceinline__ void vz_component(float2 (&out)[G::N1], const float2 
         const float vnew = upd ? vold + bb * (ac + dz) : vold;
         float dvv = vnew - vold;
         if (iz == src_iz) dvv += sprev;
-        if constexpr (INJ) dvv += inj[iz];
+        if constexpr (INJ) dvv += ld1(inj, o, im);
         out[j1] = make_float2(vnew, wa * vnew + wb * dvv);
     }
 #pragma unroll
     for (int jc = 0; jc < CH; ++jc) {
-        const int j1 = c0 + jc;
+        const int j1 = c0 + jc, im = 4 * G::N2 * j1;
         const int iz = jl + G::N2 * j1;
         const bool upd = rowdom && iz < n - 1;
-        if (upd && (iz < pml || iz >= n - pml)) ph[iz < pml ? iz : iz - (n - 2 * pml)] = qn[jc];
-        if (upd) v[iz] = out[j1].x;
-        if (ok1) w[iz] = out[j1].y;
+        if (upd && (iz < pml || iz >= n - pml)) st1(ph, phrow + 4u * (iz < pml ? iz : iz - (n - 2 * pml)), qn[jc]);
+        if (upd) st1(v, o, out[j1].x, im);
+        if (ok1) st1(w, o, out[j1].y, im);
     }
     asm volatile("" ::: "memory");  // the next chunk's loads stay after this chunk
     }
@@ -541,7 +538,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
     // uniform block base (shot + first row) and unsigned 32-bit lane offsets;
     // rows past the end (ragged last block) read row r0 and store nothing
     const long long ubase = (long long)shot * a.shot_stride + r0 * n;
-    const unsigned lrow1 = ok1 ? (unsigned)(p1 * n) : 0u;
+    const unsigned lrow1 = ok1 ? 4u * (unsigned)(p1 * n) : 0u;
     float2* pen1 = lds + p1 * G::PS;
     float2* pen2 = lds + p2 * G::PS;
     load_twiddles<G>(tws, a.tw);
@@ -551,19 +548,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
         __syncthreads();
         if (act1) {
             float2 v[G::N1];
+            const unsigned o = lane_off(lrow1 + 4u * j);
+            const Row ra = row_at(fa, ubase), rb = row_at(fb ? fb : fa, ubase);
 #pragma unroll
-            for (int j1 = 0; j1 < G::N1; ++j1) {
-                const unsigned o = lrow1 + j1 * G::N2 + j;
-                v[j1] = make_float2(fa[ubase + o], fb ? fb[ubase + o] : 0.f);
-            }
+            for (int j1 = 0; j1 < G::N1; ++j1)
+                v[j1] = make_float2(ld1(ra, o, 4 * G::N2 * j1), fb ? ld1(rb, o, 4 * G::N2 * j1) : 0.f);
             fwd_l1<G>(v, pen1, tws, j);
         }
         __syncthreads();
         float2 b[G::N2];
         if (act2) {
             fwd_l2<G>(b, pen2, k1);
+            const Row sy = row_at(S, 0);
+            const unsigned o = lane_off(8u * k1);
 #pragma unroll
-            for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = c_mul(b[k2], S[k1 + G::N1 * k2]);
+            for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = c_mul(b[k2], ld2(sy, o, 8 * G::N1 * k2));
         }
         __syncthreads();
         if (act2) inv_la<G>(b, pen2, tws + G::T2OFF, k1);
@@ -578,18 +577,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
     const float wa = a.wab[0], wb = a.wab[1];
     const int ix = (int)(r1 / a.ny), iy = (int)(r1 - (long long)ix * a.ny);
     const bool rowdom = ok1 && ix < a.nx - 1 && iy < a.ny - 1;
-    const long long slab_row = (long long)shot * a.slab_stride + r1 * 2 * a.pml;
+    const unsigned slab_row = ok1 ? (unsigned)(r1 * 2 * a.pml) * 4u : 0u;
 
     // component c on this thread's elements of its row
     auto update = [&](float2 (&out)[G::N1], const float2 (&d)[G::N1], int c, bool imag) {
-        const long long rb = ubase + lrow1;  // row base of this thread's row in the shot's fields
         const int src_iz = (kind == c && sip >= r1 * n && sip < (r1 + 1) * n) ? (int)(sip - r1 * n) : -1;
         const bool h = c == 2;
-        vz_component<G, INJ>(out, d, imag, a.v[c] + rb, a.w[c] + rb, wa, wb, a.acc[c] + rb,
-                        a.buoy[c] + (rb - (long long)shot * a.shot_stride),
-                        a.phi[c] + (ok1 ? slab_row : (long long)shot * a.slab_stride),
-                        h ? a.pah : a.pa, h ? a.pbh : a.pb, j, a.pml, a.dt, rowdom, ok1, src_iz, sprev,
-                        INJ ? a.inj[c] + rb : nullptr);
+        const Row v = row_at(a.v[c], ubase);
+        vz_component<G, INJ>(out, d, imag, v, row_at(a.w[c], ubase), wa, wb, row_at(a.acc[c], ubase),
+                        row_at(a.buoy[c], r0 * n), row_at(a.phi[c], (long long)shot * a.slab_stride), slab_row,
+                        row_at(h ? a.pah : a.pa, 0), row_at(h ? a.pbh : a.pb, 0), lrow1, j, a.pml, a.dt, rowdom, ok1,
+                        src_iz, sprev, INJ ? row_at(a.inj[c], ubase) : v);
     };
     // forward z-FFT of x (first pass of the 3-D transform) into dst
     auto fft_store = [&](float2 (&x)[G::N1], float2* dstp) {
@@ -599,9 +597,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
         if (ok2) {
             float2 b[G::N2];
             fwd_l2<G>(b, pen2, k1);
-            float2* dst = dstp + ubase + (unsigned)(p2 * n);
+            const Row dst = row_at(dstp, ubase);
+            const unsigned o = lane_off(8u * (unsigned)(p2 * n + k1));
 #pragma unroll
-            for (int k2 = 0; k2 < G::N2; ++k2) dst[k1 + G::N1 * k2] = b[k2];
+            for (int k2 = 0; k2 < G::N2; ++k2) st2(dst, o, b[k2], 8 * G::N1 * k2);
         }
     };
 
@@ -674,17 +673,18 @@ __global__ __launch_bounds__(G::T) void k2_cfft_strided(CStridedArgs a)
     const long long tbase = (long long)shot * a.shot_stride +
                             (a.axis == 0 ? (long long)other * a.sy : (long long)other * a.sx) +
                             (long long)pt.zt * G::P;
-    const unsigned voff = (unsigned)(jj * astride + p);
+    const unsigned voff = 8u * (unsigned)(jj * astride + p);
     float2* pen = lds + p * G::PS;
     load_twiddles<G>(tws, a.tw);
     for (int f = blockIdx.z; f < a.nfields; f += gridDim.z) {
         float2* const fb = a.f[f] + tbase;
+        const unsigned o = lane_off(voff);
         __syncthreads();
         if (DIR < 0) {
             if (act1) {
                 float2 v[G::N1];
 #pragma unroll
-                for (int j1 = 0; j1 < G::N1; ++j1) v[j1] = (fb + (long long)(j1 * G::N2) * astride)[voff];
+                for (int j1 = 0; j1 < G::N1; ++j1) v[j1] = ld2(row_at(fb, (long long)(j1 * G::N2) * astride), o);
                 fwd_l1<G>(v, pen, tws, jj);
             }
             __syncthreads();
@@ -692,13 +692,13 @@ __global__ __launch_bounds__(G::T) void k2_cfft_strided(CStridedArgs a)
                 float2 b[G::N2];
                 fwd_l2<G>(b, pen, jj);
 #pragma unroll
-                for (int k2 = 0; k2 < G::N2; ++k2) (fb + (long long)(G::N1 * k2) * astride)[voff] = b[k2];
+                for (int k2 = 0; k2 < G::N2; ++k2) st2(row_at(fb, (long long)(G::N1 * k2) * astride), lane_off(voff), b[k2]);
             }
         } else {
             if (act2) {
                 float2 b[G::N2];
 #pragma unroll
-                for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = (fb + (long long)(G::N1 * k2) * astride)[voff];
+                for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = ld2(row_at(fb, (long long)(G::N1 * k2) * astride), o);
                 inv_la<G>(b, pen, tws + G::T2OFF, jj);
             }
             __syncthreads();
@@ -706,7 +706,7 @@ __global__ __launch_bounds__(G::T) void k2_cfft_strided(CStridedArgs a)
                 float2 d[G::N1];
                 inv_lb<G>(d, pen, jj);
 #pragma unroll
-                for (int j1 = 0; j1 < G::N1; ++j1) (fb + (long long)(G::N2 * j1) * astride)[voff] = d[j1];
+                for (int j1 = 0; j1 < G::N1; ++j1) st2(row_at(fb, (long long)(G::N2 * j1) * astride), lane_off(voff), d[j1]);
             }
         }
     }
@@ -779,7 +779,7 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
     const long long tbase = (long long)shot * a.shot_stride + (long long)iy * a.sy +
                             (long long)pt.zt * G::P;
     const int sxi = (int)a.sx;
-    const unsigned voff = (unsigned)(jj * sxi + p);
+    const unsigned voff = 8u * (unsigned)(jj * sxi + p);
     float2* pen = lds + p * G::PS;
     load_twiddles<G>(tws, a.tw);
     const double ky = a.kfy[iy];
@@ -790,8 +790,9 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
         __syncthreads();
         if (act1) {
             float2 v[G::N1];
+            const unsigned o = lane_off(voff);
 #pragma unroll
-            for (int j1 = 0; j1 < G::N1; ++j1) v[j1] = (src + (long long)(j1 * G::N2) * sxi)[voff];
+            for (int j1 = 0; j1 < G::N1; ++j1) v[j1] = ld2(row_at(src, (long long)(j1 * G::N2) * sxi), o);
             fwd_l1<G>(v, pen, tws, jj);
         }
         __syncthreads();
@@ -843,8 +844,9 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
                 float2 d[G::N1];
                 inv_lb<G>(d, pen, jj);
                 float2* const dst = q + tbase;
+                const unsigned o = lane_off(voff);
 #pragma unroll
-                for (int j1 = 0; j1 < G::N1; ++j1) (dst + (long long)(G::N2 * j1) * sxi)[voff] = d[j1];
+                for (int j1 = 0; j1 < G::N1; ++j1) st2(row_at(dst, (long long)(G::N2 * j1) * sxi), o, d[j1]);
             }
         }
     }
@@ -874,7 +876,7 @@ __global__ __launch_bounds__(kThreads) void k2_zrows(ZRowsArgs a)
     const int tid = threadIdx.x, shot = blockIdx.y;
     const int j = tid % G::N2, p1 = tid / G::N2;
     const int k1 = tid % G::N1, p2 = tid / G::N1;
-    const long long r1 = (long long)blockIdx.x * G::P + p1, r2 = (long long)blockIdx.x * G::P + p2;
+    const long long r0 = (long long)blockIdx.x * G::P, r1 = r0 + p1, r2 = r0 + p2;
     const bool ok1 = p1 < G::P && r1 < a.nrows, ok2 = p2 < G::P && r2 < a.nrows;
     const long long soff = (long long)shot * a.shot_stride;
     float2* pen1 = lds + p1 * G::PS;
@@ -885,25 +887,28 @@ __global__ __launch_bounds__(kThreads) void k2_zrows(ZRowsArgs a)
         if (a.mode == 2 && a.dir < 0) {
             if (ok1) {
                 float2 v[G::N1];
-                const float2* src = a.cin[f] + soff + r1 * n;
+                const Row src = row_at(a.cin[f], soff + r0 * n);
+                const unsigned o = lane_off(8u * (unsigned)(p1 * n + j));
 #pragma unroll
-                for (int j1 = 0; j1 < G::N1; ++j1) v[j1] = src[j1 * G::N2 + j];
+                for (int j1 = 0; j1 < G::N1; ++j1) v[j1] = ld2(src, o, 8 * G::N2 * j1);
                 fwd_l1<G>(v, pen1, tws, j);
             }
             __syncthreads();
             if (ok2) {
                 float2 b[G::N2];
                 fwd_l2<G>(b, pen2, k1);
-                float2* dst = a.cout[f] + soff + r2 * n;
+                const Row dst = row_at(a.cout[f], soff + r0 * n);
+                const unsigned o = lane_off(8u * (unsigned)(p2 * n + k1));
 #pragma unroll
-                for (int k2 = 0; k2 < G::N2; ++k2) dst[k1 + G::N1 * k2] = b[k2];
+                for (int k2 = 0; k2 < G::N2; ++k2) st2(dst, o, b[k2], 8 * G::N1 * k2);
             }
         } else {
             if (ok2) {
                 float2 b[G::N2];
-                const float2* src = a.cin[f] + soff + r2 * n;
+                const Row src = row_at(a.cin[f], soff + r0 * n);
+                const unsigned o = lane_off(8u * (unsigned)(p2 * n + k1));
 #pragma unroll
-                for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = src[k1 + G::N1 * k2];
+                for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = ld2(src, o, 8 * G::N1 * k2);
                 inv_la<G>(b, pen2, tws + G::T2OFF, k1);
             }
             __syncthreads();
@@ -911,16 +916,21 @@ __global__ __launch_bounds__(kThreads) void k2_zrows(ZRowsArgs a)
                 float2 d[G::N1];
                 inv_lb<G>(d, pen1, j);
                 if (a.mode == 2) {
-                    float2* dst = a.cout[f] + soff + r1 * n;
+                    const Row dst = row_at(a.cout[f], soff + r0 * n);
+                    const unsigned o = lane_off(8u * (unsigned)(p1 * n + j));
 #pragma unroll
-                    for (int j1 = 0; j1 < G::N1; ++j1) dst[j + G::N2 * j1] = d[j1];
+                    for (int j1 = 0; j1 < G::N1; ++j1) st2(dst, o, d[j1], 8 * G::N2 * j1);
                 } else {
-                    float* re = a.re_out[f] ? a.re_out[f] + soff + r1 * n : nullptr;
-                    float* im = a.im_out[f] ? a.im_out[f] + soff + r1 * n : nullptr;
+                    const unsigned o = lane_off(4u * (unsigned)(p1 * n + j));
+                    if (a.re_out[f]) {
+                        const Row re = row_at(a.re_out[f], soff + r0 * n);
 #pragma unroll
-                    for (int j1 = 0; j1 < G::N1; ++j1) {
-                        if (re) re[j + G::N2 * j1] = d[j1].x;
-                        if (im) im[j + G::N2 * j1] = d[j1].y;
+                        for (int j1 = 0; j1 < G::N1; ++j1) st1(re, o, d[j1].x, 4 * G::N2 * j1);
+                    }
+                    if (a.im_out[f]) {
+                        const Row im = row_at(a.im_out[f], soff + r0 * n);
+#pragma unroll
+                        for (int j1 = 0; j1 < G::N1; ++j1) st1(im, o, d[j1].y, 4 * G::N2 * j1);
                     }
                 }
             }
@@ -999,7 +1009,8 @@ struct StressZArgs {
     float dt;
     long long shot_stride, slabx_stride, slaby_stride, slabz_stride;
     const float2* tw;
-    const float2 *symp, *symm;
+    const float2* symp;  // D+ symbols; the D- ones follow symm_off bytes on
+    unsigned symm_off;
     const float *pax, *pbx, *paxh, *pbxh;
     const float *pay, *pby, *payh, *pbyh;
     const float *paz, *pbz, *pazh, *pbzh;
@@ -1077,13 +1088,14 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
             const long long row1 = r0 + rr1;
             const bool ok1 = row1 < a.nrows;
             const int c = kind1 < 3 ? kind1 : kind1 - 3;
-            const float* fre = a.fam[c][kind1 < 3 ? 0 : 1];
-            const float* fim = a.fam[c][kind1 < 3 ? 3 : 2];
+            // rows past the end (last tile) read the tile's first row and are not used
+            const long long g = soff + (ok1 ? row1 : r0) * n + j;
+            const float* fre = a.fam[c][kind1 < 3 ? 0 : 1] + g;
+            const float* fim = a.fam[c][kind1 < 3 ? 3 : 2] + g;
             float2 v[G::N1];
 #pragma unroll
             for (int j1 = 0; j1 < G::N1; ++j1) {
-                const long long g = soff + row1 * n + j1 * G::N2 + j;
-                v[j1] = ok1 ? make_float2(fre[g], fim[g]) : make_float2(0.f, 0.f);
+                v[j1] = make_float2(fre[j1 * G::N2], fim[j1 * G::N2]);
             }
             fwd_l1<G>(v, pen1, tws, j);
         }
@@ -1092,9 +1104,11 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
         if (act2) {
             fwd_l2<G>(b, pen2, k1);
             const int kind2 = q2 % 6;
-            const float2* S = kind2 == 2 || kind2 == 5 ? a.symp : a.symm;
+            // both symbol tables sit in one allocation: a per-lane offset picks one
+            const Row S = row_at(a.symp, 0);
+            const unsigned o = lane_off(8u * k1 + (kind2 == 2 || kind2 == 5 ? 0u : a.symm_off));
 #pragma unroll
-            for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = c_mul(b[k2], S[k1 + G::N1 * k2]);
+            for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = c_mul(b[k2], ld2(S, o, 8 * G::N1 * k2));
         }
         __syncthreads();
         if (act2) inv_la<G>(b, pen2, tws + G::T2OFF, k1);
@@ -1125,8 +1139,14 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
     // uniform block bases; per-cell offsets below are unsigned 32-bit
     const long long cbase = r0 * n;          // flat index of the tile's first cell
     const long long fbase = soff + cbase;    // per-shot natural fields
-    const float* __restrict__ dxs = a.dxb + (long long)shot * kDer * a.blk_stride;
-    const float* __restrict__ dys = a.dyb + (long long)shot * kDer * a.blk_stride;
+    const Row dxr = row_at(a.dxb, (long long)shot * kDer * a.blk_stride);
+    const Row dyr = row_at(a.dyb, (long long)shot * kDer * a.blk_stride);
+    const Row g1r = row_at(a.g1, 0), g2r = row_at(VTI ? a.g2 : a.g1, 0);
+    Row gsr[kFam], sgr[6];
+#pragma unroll
+    for (int k = 0; k < kFam; ++k) gsr[k] = row_at(a.gs + k * a.N, cbase);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) sgr[k] = row_at(a.sig[k], fbase);
     constexpr bool vti = VTI;  // G2 (H, D sets) present: a compile-time choice keeps the loads branch-free
     const long long sxb = (long long)shot * a.slabx_stride, syb = (long long)shot * a.slaby_stride,
                     szb = (long long)shot * a.slabz_stride;
@@ -1143,37 +1163,37 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
             const int fz[kFam] = {4, 10, 11, 5};   // vz family (D+): normal dz vz
             const int fgx[kFam] = {0, 6, 7, 1};    // vx family (D-): dz vx for pxz
             const int fhy[kFam] = {2, 8, 9, 3};    // vy family (D-): dz vy for pyz
-            // blocked addresses of the cell: one pointer per group, the
+            // blocked addresses of the cell: one offset per group, the
             // fields at immediate offsets f*64 floats
             const unsigned ip = (unsigned)cbase + o;
             const unsigned blk = ip >> 6, in = ip & 63u;
-            const float* __restrict__ dxp = dxs + (blk * (kBlk * kDer) + in);
-            const float* __restrict__ dyp = dys + (blk * (kBlk * kDer) + in);
-            const float* __restrict__ g1p = a.g1 + (blk * (kBlk * kG1) + in);
-            const float* __restrict__ gsp = a.gs + ip;
-            const float* __restrict__ g2p = vti ? a.g2 + (blk * (kBlk * kG2) + in) : nullptr;
+            const unsigned od = lane_off(4u * (blk * (kBlk * kDer) + in));
+            const unsigned o1 = lane_off(4u * (blk * (kBlk * kG1) + in));
+            const unsigned o2 = lane_off(4u * (blk * (kBlk * kG2) + in));
+            const unsigned oc = lane_off(4u * o);
+            constexpr int FB = 4 * kBlk;  // bytes between the fields of a block
             float oP[kFam], oS[kFam], oH[kFam], oD[kFam];
             {
-                const float r = g1p[4 * kBlk];
-                set_coeffs(oP, g1p[0], g1p[kBlk], r, alpha, s4);
-                set_coeffs(oS, g1p[2 * kBlk], g1p[3 * kBlk], r, alpha, s4);
+                const float r = ld1(g1r, o1, 4 * FB);
+                set_coeffs(oP, ld1(g1r, o1), ld1(g1r, o1, FB), r, alpha, s4);
+                set_coeffs(oS, ld1(g1r, o1, 2 * FB), ld1(g1r, o1, 3 * FB), r, alpha, s4);
                 if (vti) {
-                    set_coeffs(oH, g2p[0], g2p[kBlk], r, alpha, s4);
-                    set_coeffs(oD, g2p[2 * kBlk], g2p[3 * kBlk], r, alpha, s4);
+                    set_coeffs(oH, ld1(g2r, o2), ld1(g2r, o2, FB), r, alpha, s4);
+                    set_coeffs(oD, ld1(g2r, o2, 2 * FB), ld1(g2r, o2, 3 * FB), r, alpha, s4);
                 }
             }
             float A[14];
 #pragma unroll
             for (int k = 0; k < 14; ++k) A[k] = 0.f;
-            A[9] = dxp[kFam * kBlk];         // sb_zx  (dx vz)
-            A[11] = dxp[(kFam + 1) * kBlk];  // sb_yx  (dx vy)
-            A[13] = dyp[kFam * kBlk];        // sb_zy  (dy vz)
-            A[10] = dyp[(kFam + 1) * kBlk];  // sb_xy  (dy vx)
+            A[9] = ld1(dxr, od, kFam * FB);         // sb_zx  (dx vz)
+            A[11] = ld1(dxr, od, (kFam + 1) * FB);  // sb_yx  (dx vy)
+            A[13] = ld1(dyr, od, kFam * FB);        // sb_zy  (dy vz)
+            A[10] = ld1(dyr, od, (kFam + 1) * FB);  // sb_xy  (dy vx)
 #pragma unroll
             for (int jf = 0; jf < kFam; ++jf) {
                 const float ez = S(fz[jf]), gz = S(fgx[jf]), hz = S(fhy[jf]);
-                const float ex = dxp[jf * kBlk], ey = dyp[jf * kBlk];
-                const float c33 = oP[jf], cs = oS[jf], csb = gsp[jf * a.N];
+                const float ex = ld1(dxr, od, jf * FB), ey = ld1(dyr, od, jf * FB);
+                const float c33 = oP[jf], cs = oS[jf], csb = ld1(gsr[jf], oc);
                 const float c11 = vti ? oH[jf] : c33, c13 = vti ? oD[jf] : c33;
                 const float c12 = c11 - 2 * cs, c13d = c13 - 2 * cs;
                 A[0] += c11 * ex;   // s11x
@@ -1192,7 +1212,7 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
             // know it, so loads placed after a store would each wait for it.
             float sg[6];
 #pragma unroll
-            for (int k = 0; k < 6; ++k) sg[k] = a.sig[k][fbase + o];
+            for (int k = 0; k < 6; ++k) sg[k] = ld1(sgr[k], oc);
             const bool xs = ix < pml || ix >= a.nx - pml;
             const bool ys = iy < pml || iy >= a.ny - pml;
             const bool zs = iz < pml || iz >= n - pml;
@@ -1256,12 +1276,12 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
                 a.phz[2][szb + oz] = fxz;
                 a.phz[3][szb + oz] = fyz;
             }
-            a.sig[0][fbase + o] = sg[0] + dt * (A[0] + A[3] + A[6] + (fxx_x + fyx_y + fzx_z));
-            a.sig[1][fbase + o] = sg[1] + dt * (A[1] + A[4] + A[6] + (fxy_x + fyy_y + fzx_z));
-            a.sig[2][fbase + o] = sg[2] + dt * (A[2] + A[5] + A[7] + (fxz_x + fyz_y + fzz_z));
-            a.sig[3][fbase + o] = sg[3] + dt * (A[10] + fxy + A[11] + fyx);
-            a.sig[4][fbase + o] = sg[4] + dt * (A[8] + fxz + A[9] + fzx);
-            a.sig[5][fbase + o] = sg[5] + dt * (A[12] + fyz + A[13] + fzy);
+            st1(sgr[0], oc, sg[0] + dt * (A[0] + A[3] + A[6] + (fxx_x + fyx_y + fzx_z)));
+            st1(sgr[1], oc, sg[1] + dt * (A[1] + A[4] + A[6] + (fxy_x + fyy_y + fzx_z)));
+            st1(sgr[2], oc, sg[2] + dt * (A[2] + A[5] + A[7] + (fxz_x + fyz_y + fzz_z)));
+            st1(sgr[3], oc, sg[3] + dt * (A[10] + fxy + A[11] + fyx));
+            st1(sgr[4], oc, sg[4] + dt * (A[8] + fxz + A[9] + fzx));
+            st1(sgr[5], oc, sg[5] + dt * (A[12] + fyz + A[13] + fzy));
         }
         if (row * n + iz == sip) {
             // source after the stress update; no other workgroup of this

@@ -7,33 +7,41 @@
 
 namespace qvti {
 
-// Receivers: rec[it][r] = v[cell_r] for the three components (after the
-// source injection), cuviscoelas_3D.cu:782-792.  The step counter `it`
-// advances in the first kernel of the next step (k2_deriv_strided's tick).
+// Receivers: rec[it][r] = v[cell_r] for the three components after the
+// source injection, cuviscoelas_3D.cu:782-792.  Runs before the injection
+// (k2_zrows), which adds rik[it] to one cell: a receiver there gets v + rik[it],
+// the value the injection writes.
 struct RecArgs {
     const float *vx, *vy, *vz;
     long long shot_stride;
     const long long* rec_ip;  // all shots' receivers back to back
     const int* rec_off;       // per shot: first receiver, [nshots+1]
     float *rx, *ry, *rz;      // records, per shot offset rec_off[s]*nt
-    int nt;
+    int nt;                   // 0: no receivers
     const int* it;
+    const int* src_kind;
+    const long long* src_ip;
+    const float* rik;
 };
 
-static __global__ __launch_bounds__(256) void k_record(RecArgs a)
+// receivers first, first + stride, ... of one shot
+__device__ __forceinline__ void record_samples(const RecArgs& a, int shot, int first, int stride)
 {
-    const int shot = blockIdx.y;
     const int r0 = a.rec_off[shot], nr = a.rec_off[shot + 1] - r0;
-    const int r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= nr) return;
-    const int it = *a.it;
-    const long long ip = a.rec_ip[r0 + r] + (long long)shot * a.shot_stride;
-    const long long o = (long long)r0 * a.nt + (long long)it * nr + r;
-    a.rx[o] = a.vx[ip];
-    a.ry[o] = a.vy[ip];
-    a.rz[o] = a.vz[ip];
+    if (first >= nr) return;
+    const int it = *a.it, kind = a.src_kind[shot];
+    const long long sip = a.src_ip[shot];
+    const float s = a.rik[it];
+    for (int r = first; r < nr; r += stride) {
+        const long long cell = a.rec_ip[r0 + r], ip = cell + (long long)shot * a.shot_stride;
+        const long long o = (long long)r0 * a.nt + (long long)it * nr + r;
+        const bool src = cell == sip;
+        const float vx = a.vx[ip], vy = a.vy[ip], vz = a.vz[ip];
+        a.rx[o] = src && kind == 0 ? vx + s : vx;
+        a.ry[o] = src && kind == 1 ? vy + s : vy;
+        a.rz[o] = src && kind == 2 ? vz + s : vz;
+    }
 }
-
 
 // Snapshot of one field over the box [lo, hi) (ix slowest) when
 // it % every == 0; snapshot k lands at out[k * W], W the box's cell count.

@@ -90,8 +90,8 @@ struct qvti_ctx {
     CStridedArgs a_yf{}, a_yi{};
     XPassArgs a_xp{};
     StressZArgs a_sz{};
-    RecArgs a_rec{};
-    dim3 g_vx, g_vy, g_vz, g_zr, g_cy, g_xp, g_sz, g_rec, g_sx, g_sy, g_yi;
+    RecArgs a_rec{};  // copied into a_zi.rec (nt = 0: no receivers)
+    dim3 g_vx, g_vy, g_vz, g_zr, g_cy, g_xp, g_sz, g_sx, g_sy, g_yi;
     int P[3] = {0, 0, 0};
     // tile width per kernel class (strided-axis kernels), chosen by the autotuner
     int pw[KC_COUNT] = {};

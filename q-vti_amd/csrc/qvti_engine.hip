@@ -190,7 +190,7 @@ static void release(qvti_ctx* c)
 }
 
 // ------------------------------------------------------- sizes / memory --
-// Fields per shot of the scratch buffers.  bufA: velocity accumulators (3),
+// Fields per shot of the scratch buffers.  bufA: velocity x- and y-derivatives (6),
 // then the four Q spectra (8), then the x-derivatives (kDer).  bufB: the three
 // P spectra (6), then the y-derivatives (kDer).
 constexpr int kFieldsA = 8, kFieldsB = 6;
@@ -382,7 +382,8 @@ static int build_launch_config(qvti_ctx* c)
     c->P[2] = c->ops[2]->Prow;
     const int Px = c->P[0], Py = c->P[1], Pz = c->P[2];
 
-    float* acc[3] = {fld(c->bufA, 0, c), fld(c->bufA, 1, c), fld(c->bufA, 2, c)};
+    float* accx[3] = {fld(c->bufA, 0, c), fld(c->bufA, 1, c), fld(c->bufA, 2, c)};
+    float* accy[3] = {fld(c->bufA, 3, c), fld(c->bufA, 4, c), fld(c->bufA, 5, c)};
     float* vv[3] = {fld(c->v, 0, c), fld(c->v, 1, c), fld(c->v, 2, c)};
     float* ww[3] = {fld(c->w, 0, c), fld(c->w, 1, c), fld(c->w, 2, c)};
     // sig order: pxx pyy pzz pxy pxz pyz
@@ -406,31 +407,33 @@ static int build_launch_config(qvti_ctx* c)
         a.sym[1] = A.dm;
         a.pa = A.a; a.pb = A.b; a.pah = A.ah; a.pbh = A.bh;
     };
-    auto job = [](const float* in, float* out, const float* accp, float* phi, int sym, int half) {
+    auto job = [](const float* in, float* out, float* phi, int sym, int half) {
         DJob j;
-        j.in = in; j.out = out; j.acc = accp; j.phi = phi; j.sym = sym; j.half = half;
+        j.in = in; j.out = out; j.phi = phi; j.sym = sym; j.half = half;
         return j;
     };
-    // ---- velocity x: pxx (D-, half) -> acc_x, pxy (D+) -> acc_y, pxz (D+) -> acc_z
+    // ---- velocity x: pxx (D-, half) -> vx, pxy (D+) -> vy, pxz (D+) -> vz
     StridedArgs& vx = c->a_vx;
     strided_common(vx, 0, Px);
-    vx.mode = MODE_VEL_FIRST;
+    vx.mode = MODE_VEL;
     vx.njobs = 3;
-    vx.job[0] = job(pxx, acc[0], nullptr, nullptr, 1, 1);
-    vx.job[1] = job(pxy, acc[1], nullptr, nullptr, 0, 0);
-    vx.job[2] = job(pxz, acc[2], nullptr, nullptr, 0, 0);
+    vx.job[0] = job(pxx, accx[0], nullptr, 1, 1);
+    vx.job[1] = job(pxy, accx[1], nullptr, 0, 0);
+    vx.job[2] = job(pxz, accx[2], nullptr, 0, 0);
     vx.tick = c->d_it;  // the first kernel of a step advances the step counter
-    for (int k = 0; k < 3; ++k) vx.job[k].phi = c->phiv[0] + (long long)k * c->S * c->slab[0];  // [field][shot][slab]
 
-    // ---- velocity y: pxy (D+) -> acc_x, pyy (D-, half) -> acc_y, pyz (D+) -> acc_z
+    // ---- velocity y: pxy (D+) -> vx, pyy (D-, half) -> vy, pyz (D+) -> vz
     StridedArgs& vy = c->a_vy;
     strided_common(vy, 1, Py);
-    vy.mode = MODE_VEL_ACC;
+    vy.mode = MODE_VEL;
     vy.njobs = 3;
-    vy.job[0] = job(pxy, acc[0], acc[0], nullptr, 0, 0);
-    vy.job[1] = job(pyy, acc[1], acc[1], nullptr, 1, 1);
-    vy.job[2] = job(pyz, acc[2], acc[2], nullptr, 0, 0);
-    for (int k = 0; k < 3; ++k) vy.job[k].phi = c->phiv[1] + (long long)k * c->S * c->slab[1];
+    vy.job[0] = job(pxy, accy[0], nullptr, 0, 0);
+    vy.job[1] = job(pyy, accy[1], nullptr, 1, 1);
+    vy.job[2] = job(pyz, accy[2], nullptr, 0, 0);
+    for (int k = 0; k < 3; ++k) {  // [field][shot][slab]
+        vx.job[k].phi = c->phiv[0] + (long long)k * c->S * c->slab[0];
+        vy.job[k].phi = c->phiv[1] + (long long)k * c->S * c->slab[1];
+    }
 
     // ---- 3-D transform buffers: P (bufB as complex), Q1, Q3 (bufA as complex)
     float2* P[3];
@@ -448,7 +451,8 @@ static int build_launch_config(qvti_ctx* c)
     vz.pa = Z.a; vz.pb = Z.b; vz.pah = Z.ah; vz.pbh = Z.bh;
     vz.pxz = pxz; vz.pyz = pyz; vz.pzz = pzz;
     for (int k = 0; k < 3; ++k) {
-        vz.acc[k] = acc[k];
+        vz.accx[k] = accx[k];
+        vz.accy[k] = accy[k];
         vz.v[k] = vv[k];
         vz.w[k] = ww[k];
         vz.P[k] = P[k];
@@ -633,7 +637,8 @@ static int build_launch_config(qvti_ctx* c)
     rec.shot_stride = N;
     rec.rec_off = c->d_rec_off;
     rec.it = c->d_it;
-    (void)pyy;
+    rec.src_kind = c->d_src_kind;
+    rec.src_ip = c->d_src_ip;
     for (int k = 0; k < KC_COUNT; ++k) c->pw[k] = c->jz[k] = 1;
     apply_tiles(c);
     return QVTI_OK;
@@ -730,6 +735,13 @@ static unsigned xcd_grid(int ntiles, unsigned S, int run)
     return (unsigned)((ntiles + g - 1) / g) * (unsigned)g * S;
 }
 
+// The x and y passes of the velocity and of the stress derivatives each go in
+// one launch (of class vel_x / str_x) when both axes run the same kernel: they
+// are independent (k2_vel_z adds the velocity's), and together they leave no
+// partly filled last round of workgroups between them.  Step with two launches,
+// the second one accumulating / with one: 64^3 85 / 81 us, 128^3 370 / 361 us,
+// 160x160x128 569 / 563 us, 256^3 2.708 / 2.699 ms, 400x400x200 equal.
+static bool merged_xy(const qvti_ctx* c) { return c->ops[0] == c->ops[1]; }
 // Launch one kernel of class cls on the context's stream.
 static void launch_class(qvti_ctx* c, int cls)
 {
@@ -737,13 +749,19 @@ static void launch_class(qvti_ctx* c, int cls)
     const unsigned S = (unsigned)c->nshots;
     const LenOps &X = *c->ops[0], &Y = *c->ops[1], &Z = *c->ops[2];
     auto strided = [&](const dim3& g) { return dim3(g.x, S, (unsigned)c->jz[cls]); };
+    auto pair = [&](const dim3& g) { return dim3(g.x, S, (unsigned)(c->jz[cls] * (merged_xy(c) ? 2 : 1))); };
     switch (cls) {
     case KC_VEL_X:
-        X.deriv[MODE_VEL_FIRST][pw_index(X, c->pw[cls])](strided(c->g_vx), st, c->a_vx);
+    case KC_VEL_Y: {
+        if (cls == KC_VEL_Y && merged_xy(c)) break;
+        StridedPair pr;
+        pr.a[0] = cls == KC_VEL_X ? c->a_vx : c->a_vy;
+        pr.a[1] = c->a_vy;
+        pr.jz = c->jz[cls];
+        const LenOps& O = cls == KC_VEL_X ? X : Y;
+        O.deriv[MODE_VEL][pw_index(O, c->pw[cls])](pair(cls == KC_VEL_X ? c->g_vx : c->g_vy), st, pr);
         break;
-    case KC_VEL_Y:
-        Y.deriv[MODE_VEL_ACC][pw_index(Y, c->pw[cls])](strided(c->g_vy), st, c->a_vy);
-        break;
+    }
     case KC_VEL_Z:
         Z.vel_z[c->a_vz.inj[0] ? 1 : 0](dim3(xcd_grid(c->a_vz.ntiles, S, c->a_vz.run)), st, c->a_vz);
         break;
@@ -758,34 +776,39 @@ static void launch_class(qvti_ctx* c, int cls)
         break;
     case KC_Z_INV: {
         const unsigned zs = QVTI_ZINV_SPLIT == 1 ? 1u : (unsigned)c->a_zi.nfields;
-        Z.zrows(dim3(c->g_zr.x, S, zs), st, c->a_zi);
+        c->a_zi.rec = c->a_rec;
+        if (c->total_rec == 0) c->a_zi.rec.nt = 0;
+        Z.zrows(dim3(c->g_zr.x, S, zs + (c->a_zi.rec.nt > 0 ? 1 : 0)), st, c->a_zi);
         break;
     }
     case KC_STR_X:
-        X.stress_xy[pw_index(X, c->pw[cls])](strided(c->g_sx), st, c->a_sx);
+    case KC_STR_Y: {
+        if (cls == KC_STR_Y && merged_xy(c)) break;
+        StressXYPair pr;
+        pr.a[0] = cls == KC_STR_X ? c->a_sx : c->a_sy;
+        pr.a[1] = c->a_sy;
+        pr.jz = c->jz[cls];
+        const LenOps& O = cls == KC_STR_X ? X : Y;
+        O.stress_xy[pw_index(O, c->pw[cls])](pair(cls == KC_STR_X ? c->g_sx : c->g_sy), st, pr);
         break;
-    case KC_STR_Y:
-        Y.stress_xy[pw_index(Y, c->pw[cls])](strided(c->g_sy), st, c->a_sy);
-        break;
+    }
     case KC_STR_Z:
         Z.stress_z[c->g.vti ? 1 : 0](dim3(xcd_grid(c->a_sz.ntiles, S, c->a_sz.run)), st, c->a_sz);
-        break;
-    case KC_RECORD:
-        hipLaunchKernelGGL(k_record, dim3(c->g_rec.x, S), dim3(kThreads), 0, st, c->a_rec);
         break;
     default:
         break;
     }
 }
 
-// Enqueue one time step (11 launches; vel_x also advances the step counter).
+// Enqueue one time step (8 launches where nx == ny, else 10; the first one
+// also advances the step counter).
 // With timing on, each launch is bracketed by an event pair.
 static void enqueue_step(qvti_ctx* c)
 {
     static const int order[] = {KC_VEL_X, KC_VEL_Y, KC_VEL_Z, KC_Y_FWD, KC_XPASS,
-                                KC_Y_INV, KC_Z_INV, KC_STR_X, KC_STR_Y, KC_STR_Z, KC_RECORD};
+                                KC_Y_INV, KC_Z_INV, KC_STR_X, KC_STR_Y, KC_STR_Z};
     for (int cls : order) {
-        if (cls == KC_RECORD && c->total_rec == 0) continue;
+        if ((cls == KC_VEL_Y || cls == KC_STR_Y) && merged_xy(c)) continue;
         const int e0 = c->timing ? record_event(c, cls) : -1;
         launch_class(c, cls);
         if (e0 >= 0) record_event(c, -1 - cls);
@@ -810,8 +833,10 @@ static void apply_tiles(qvti_ctx* c)
     c->a_vx.run = c->a_sx.run = c->a_vy.run = c->a_sy.run = c->a_yf.run = c->a_yi.run = c->a_xp.run = rp;
     c->a_vx.ztiles = zt(0, KC_VEL_X, 2); c->g_vx = grid(ny, c->a_vx.ztiles, rp);
     c->a_sx.ztiles = zt(0, KC_STR_X, 1); c->g_sx = grid(ny, c->a_sx.ztiles, rp);
-    c->a_vy.ztiles = zt(1, KC_VEL_Y, 2); c->g_vy = grid(nx, c->a_vy.ztiles, rp);
-    c->a_sy.ztiles = zt(1, KC_STR_Y, 1); c->g_sy = grid(nx, c->a_sy.ztiles, rp);
+    // merged launches: the y axis takes the tile width of class x
+    const int vy = merged_xy(c) ? KC_VEL_X : KC_VEL_Y, sy = merged_xy(c) ? KC_STR_X : KC_STR_Y;
+    c->a_vy.ztiles = zt(1, vy, 2); c->g_vy = grid(nx, c->a_vy.ztiles, rp);
+    c->a_sy.ztiles = zt(1, sy, 1); c->g_sy = grid(nx, c->a_sy.ztiles, rp);
     c->a_yf.ztiles = zt(1, KC_Y_FWD, 1); c->g_cy = grid(nx, c->a_yf.ztiles, rp);
     c->a_yi.ztiles = zt(1, KC_Y_INV, 1); c->g_yi = grid(nx, c->a_yi.ztiles, rp);
     c->a_xp.ztiles = zt(0, KC_XPASS, 1); c->g_xp = grid(ny, c->a_xp.ztiles, rp);
@@ -836,7 +861,7 @@ static int class_fields(const qvti_ctx* c, int cls)
 // tuned kernel only writes scratch buffers that a step overwrites first.
 static int autotune_tiles(qvti_ctx* c)
 {
-    static const int classes[] = {KC_VEL_X, KC_VEL_Y, KC_Y_FWD, KC_XPASS, KC_Y_INV, KC_STR_X, KC_STR_Y};
+    static const int classes[] = {KC_VEL_X, KC_VEL_Y, KC_Y_FWD, KC_XPASS, KC_Y_INV, KC_STR_X, KC_STR_Y};  // x before y
     hipEvent_t e0 = nullptr, e1 = nullptr;
     HIPCHK(hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) {
@@ -848,6 +873,11 @@ static int autotune_tiles(qvti_ctx* c)
     c->a_vx.tick = nullptr;
     int rc = QVTI_OK;
     for (int cls : classes) {
+        if ((cls == KC_VEL_Y || cls == KC_STR_Y) && merged_xy(c)) {
+            c->pw[cls] = c->pw[cls == KC_VEL_Y ? KC_VEL_X : KC_STR_X];
+            c->jz[cls] = c->jz[cls == KC_VEL_Y ? KC_VEL_X : KC_STR_X];
+            continue;
+        }
         const LenOps* o = (cls == KC_VEL_X || cls == KC_XPASS || cls == KC_STR_X) ? c->ops[0] : c->ops[1];
         const int nf = class_fields(c, cls);
         int best_pw = 1, best_jz = 1;
@@ -1047,9 +1077,7 @@ extern "C" int qvti_begin(qvti_ctx* c, int nt, const float* rik, const qvti_shot
     c->a_rec.ry = c->d_rec + (long long)c->total_rec * nt;
     c->a_rec.rz = c->d_rec + 2LL * c->total_rec * nt;
     c->a_rec.nt = nt;
-    int maxr = 1;
-    for (int s = 0; s < nshots; ++s) maxr = std::max(maxr, shots[s].nrec);
-    c->g_rec = dim3((unsigned)((maxr + kThreads - 1) / kThreads), 1, 1);
+    c->a_rec.rik = c->d_rik;
     if (c->autotune && c->tuned != nshots) {
         rc = autotune_tiles(c);
         if (rc) return rc;
@@ -1743,8 +1771,8 @@ extern "C" int qvti_kernel_bytes(qvti_ctx* c, int max_classes, double* bytes)
     double b[KC_COUNT] = {};
     b[KC_TICK] = 8;
     b[KC_VEL_X] = 6 * f + 3 * 2 * sx;
-    b[KC_VEL_Y] = 9 * f + 3 * 2 * sy;
-    b[KC_VEL_Z] = (3 + 3 + 3 + 3 + 3 + 6) * f + 3.0 * 4 * c->N + 3 * 2 * sz;  // sig, acc, v r/w, w, P, buoy
+    b[KC_VEL_Y] = 6 * f + 3 * 2 * sy;
+    b[KC_VEL_Z] = (3 + 6 + 3 + 3 + 3 + 6) * f + 3.0 * 4 * c->N + 3 * 2 * sz;  // sig, acc, v r/w, w, P, buoy
     b[KC_Y_FWD] = 12 * f;
     // k-space mode: three more complex spectra through the x-pass, y-inverse
     // and z-inverse, six more real fields out
@@ -1753,7 +1781,12 @@ extern "C" int qvti_kernel_bytes(qvti_ctx* c, int max_classes, double* bytes)
     b[KC_Z_INV] = c->ks ? 14 * f + 12 * f : 8 * f + 6 * f;
     b[KC_STR_X] = b[KC_STR_Y] = (3 * kFam + kDer) * f + kGS * 4.0 * c->N;
     b[KC_STR_Z] = (12 + 2 * kDer + 12) * f + ncoef * 4.0 * c->N + 2 * (5 * sx + 5 * sy + 4 * sz);
-    b[KC_RECORD] = 6.0 * 4 * c->total_rec;
+    b[KC_Z_INV] += 6.0 * 4 * c->total_rec;  // receivers
+    if (merged_xy(c)) {  // both axes in the launch of class x
+        b[KC_VEL_X] += b[KC_VEL_Y];
+        b[KC_STR_X] += b[KC_STR_Y];
+        b[KC_VEL_Y] = b[KC_STR_Y] = 0;
+    }
     const int n = std::min(max_classes, (int)KC_COUNT);
     for (int k = 0; k < n; ++k) bytes[k] = b[k];
     return n;
@@ -1917,17 +1950,19 @@ extern "C" int qvti_deriv1d(int nx, int ny, int nz, float dd, int axis, int sym,
         const LenOps& A = *len_ops(n);
         const int P = A.P[0];
         if (axis < 2) {
-            StridedArgs a{};
+            StridedPair pr{};
+            pr.jz = 1;
+            StridedArgs& a = pr.a[0];
             a.nx = nx; a.ny = ny; a.nz = nz; a.pml = 0;
             a.sx = (long long)ny * nz; a.sy = nz; a.axis = axis;
             a.ztiles = (nz + 2 * P - 1) / (2 * P);
             a.mode = MODE_STORE; a.dt = 0.f; a.shot_stride = N; a.slab_stride = 0;
             a.tw = dtw; a.sym[0] = dsym; a.sym[1] = dsym;
             a.njobs = 1;
-            a.job[0].in = din; a.job[0].out = dout; a.job[0].acc = nullptr; a.job[0].phi = nullptr;
+            a.job[0].in = din; a.job[0].out = dout; a.job[0].phi = nullptr;
             a.job[0].sym = 0; a.job[0].half = 0;
             const int other = axis == 0 ? ny : nx;
-            A.deriv[MODE_STORE][0](dim3((unsigned)(other * a.ztiles), 1), nullptr, a);
+            A.deriv[MODE_STORE][0](dim3((unsigned)(other * a.ztiles), 1), nullptr, pr);
         } else {
             RowDerivArgs r{};
             const long long nrows = (long long)nx * ny;

@@ -11,12 +11,12 @@ namespace qvti {
 namespace {
 
 template <class G, int MODE>
-void l_deriv(dim3 grid, hipStream_t st, const StridedArgs& a)
+void l_deriv(dim3 grid, hipStream_t st, const StridedPair& a)
 {
     hipLaunchKernelGGL((k2_deriv_strided<G, MODE>), grid, dim3(G::T), 0, st, a);
 }
 template <class G>
-void l_stress_xy(dim3 grid, hipStream_t st, const StressXYArgs& a)
+void l_stress_xy(dim3 grid, hipStream_t st, const StressXYPair& a)
 {
     hipLaunchKernelGGL(k2_stress_xy<G>, grid, dim3(G::T), 0, st, a);
 }
@@ -59,8 +59,8 @@ constexpr bool pw_ok()
     else return A * B >= 64 && L2<A, B, PW>::kFits;
 }
 
-using DerivFn = void (*)(dim3, hipStream_t, const StridedArgs&);
-using StressXYFn = void (*)(dim3, hipStream_t, const StressXYArgs&);
+using DerivFn = void (*)(dim3, hipStream_t, const StridedPair&);
+using StressXYFn = void (*)(dim3, hipStream_t, const StressXYPair&);
 using CfftFn = void (*)(dim3, hipStream_t, const CStridedArgs&);
 using XpassFn = void (*)(dim3, hipStream_t, const XPassArgs&);
 
@@ -109,9 +109,7 @@ LenOps make_ops()
         {pencils<A, B, kW0>(), pencils<A, B, kW1>(), pencils<A, B, kW2>()},
         {L2<A, B, kW0>::T, L2<A, B, kW1>::T, L2<A, B, kW2>::T},
         {{deriv_fn<A, B, kW0, MODE_STORE>(), nullptr, nullptr},
-         {deriv_fn<A, B, kW0, MODE_VEL_FIRST>(), deriv_fn<A, B, kW1, MODE_VEL_FIRST>(),
-          deriv_fn<A, B, kW2, MODE_VEL_FIRST>()},
-         {deriv_fn<A, B, kW0, MODE_VEL_ACC>(), deriv_fn<A, B, kW1, MODE_VEL_ACC>(), deriv_fn<A, B, kW2, MODE_VEL_ACC>()}},
+         {deriv_fn<A, B, kW0, MODE_VEL>(), deriv_fn<A, B, kW1, MODE_VEL>(), deriv_fn<A, B, kW2, MODE_VEL>()}},
         {stress_xy_fn<A, B, kW0>(), stress_xy_fn<A, B, kW1>(), stress_xy_fn<A, B, kW2>()},
         {{cfft_fn<A, B, kW0, -1>(), cfft_fn<A, B, kW1, -1>(), cfft_fn<A, B, kW2, -1>()},
          {cfft_fn<A, B, kW0, 1>(), cfft_fn<A, B, kW1, 1>(), cfft_fn<A, B, kW2, 1>()}},

@@ -21,8 +21,8 @@ struct LenOps {
     int P[3];  // pencils per tile of the strided kernels at width index 0, 1, 2 (0: not available)
     int T[3];  // threads per workgroup at width index 0, 1, 2
     // strided-axis kernels, [..][pw index]
-    void (*deriv[3][3])(dim3 grid, hipStream_t st, const StridedArgs& a);  // [MODE_*] (STORE: width index 0 only)
-    void (*stress_xy[3])(dim3 grid, hipStream_t st, const StressXYArgs& a);
+    void (*deriv[2][3])(dim3 grid, hipStream_t st, const StridedPair& a);  // [MODE_*] (STORE: width index 0 only)
+    void (*stress_xy[3])(dim3 grid, hipStream_t st, const StressXYPair& a);
     void (*cfft[2][3])(dim3 grid, hipStream_t st, const CStridedArgs& a);  // [0 forward, 1 inverse]
     void (*xpass[2][3])(dim3 grid, hipStream_t st, const XPassArgs& a);    // [k-space mode off, on]
     // row (z) kernels, 256 threads (stress_z: StressTile)

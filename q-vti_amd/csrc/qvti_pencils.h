@@ -4,13 +4,13 @@
 // (x, y) kernels 256*PW (the tile width the autotuner picks).
 //
 // Per step (reference loop: cuviscoelas_3D.cu:1255-1605):
-//   velocity half-step   k2_deriv_strided(x, VEL_FIRST; advances the step counter)
-//                        -> k2_deriv_strided(y, VEL_ACC)
+//   velocity half-step   k2_deriv_strided (x and y; advances the step counter)
 //                        -> k2_vel_z (z-derivatives, velocity update, forward z-FFTs of v and w)
 //   stress half-step     k2_cfft_strided(y, fwd) -> k2_xpass -> k2_cfft_strided(y, inv)
-//                        -> k2_zrows (inverse z) -> k2_stress_xy(x) -> k2_stress_xy(y)
+//                        -> k2_zrows (inverse z; receivers) -> k2_stress_xy (x and y)
 //                        -> k2_stress_z (z-derivatives, stress update, source injection)
-//   receivers            k_record
+// The x and the y derivatives are independent: one launch takes both where the
+// two axes have one length (and so one kernel), two launches elsewhere.
 //
 // Algebra used (exact in exact arithmetic; only rounding differs from the
 // reference's C2C + `.x / ntp` formulation):
@@ -55,13 +55,14 @@ constexpr int kThreads = 256;
 #ifndef QVTI_STRESSZ_WAVES
 #define QVTI_STRESSZ_WAVES 1
 #endif
-#ifndef QVTI_VZ_CHUNK
-#define QVTI_VZ_CHUNK 4
-#endif
-#ifndef QVTI_VEL_CHUNK
-#define QVTI_VEL_CHUNK 4
-#endif
-enum { MODE_STORE = 0, MODE_VEL_FIRST = 1, MODE_VEL_ACC = 2 };
+enum { MODE_STORE = 0, MODE_VEL = 1 };
+
+// Elements per chunk of the C-PML epilogues: a divisor of the thread's N1
+// elements, about 4 (more would hold more loads in registers than they overlap).
+constexpr int vel_chunk(int n1)
+{
+    return n1 % 4 == 0 ? 4 : (n1 % 5 == 0 ? 5 : (n1 % 3 == 0 ? 3 : 1));
+}
 
 // XCD-aware placement of (row tile, shot) on a 1-D grid of
 // ceil(ntiles / (8 run)) * 8 run * nshots workgroups.  Workgroup ids are dealt
@@ -123,13 +124,14 @@ __device__ __forceinline__ void load_twiddles(float2* tws, const float2* tw)
 // 1-D shift-derivatives of real fields along a strided axis (x or y).  Tile:
 // G::P complex pencils = 2*G::P adjacent real z-columns at one value of the
 // other in-plane index, loaded as float2 (two real pencils per complex one).
-// Modes: STORE out = d (standalone derivative); VEL_FIRST out = d + phi; VEL_ACC out = acc + d + phi,
-// with the velocity C-PML memory variable phi updated on the axis' face slabs
-// (cuviscoelas_3D.cu:1049-1074).
+// Modes: STORE out = d (standalone derivative); VEL out = d + phi, with the
+// velocity C-PML memory variable phi updated on the axis' face slabs
+// (cuviscoelas_3D.cu:1049-1074).  A launch takes one or two axes (of one
+// length), which fill the chip together: at 64^3 an axis' 192 workgroups leave
+// a quarter of the CUs without one.
 struct DJob {
     const float* in;
     float* out;
-    const float* acc;
     float* phi;
     int sym;   // 0: D+, 1: D-
     int half;  // 1: half-cell averaged C-PML a, b
@@ -151,11 +153,17 @@ struct StridedArgs {
     int* tick;
     DJob job[3];
 };
+struct StridedPair {
+    StridedArgs a[2];
+    int jz;  // workgroups per tile and axis; grid z: (axis, job)
+};
 
 template <class G, int MODE>
 __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_STRIDED_WAVES)))
-void k2_deriv_strided(StridedArgs a)
+void k2_deriv_strided(StridedPair pr)
 {
+    const int sel = blockIdx.z / pr.jz, jb0 = blockIdx.z - sel * pr.jz;
+    const StridedArgs& a = pr.a[sel];
     __shared__ float2 lds[G::P * G::PS];
     __shared__ float2 tws[G::TWN];
     const int tid = threadIdx.x, shot = blockIdx.y;
@@ -167,20 +175,23 @@ void k2_deriv_strided(StridedArgs a)
     const int other = pt.plane;
     const int p = tid % G::P, jj = tid / G::P;
     const int zc = pt.zt * 2 * G::P + 2 * p;
-    const int nz = a.nz;
+    // scalars of the chosen axis in registers: read through `a` they would be
+    // loaded again at every use below
+    const int nx = a.nx, ny = a.ny, nz = a.nz, axis = a.axis, pml = a.pml;
+    const float dt = a.dt;
     const bool zok = zc < nz;
     // columns past nz (last tile of a ragged z) load a valid column and are
     // never stored, so the loads need no branch
     const int zl = zok ? zc : nz - 2;
     const bool act1 = jj < G::N2, act2 = jj < G::N1;
     // uniform per-block base (SGPRs) + 32-bit per-thread element offsets
-    const int astride = (int)(a.axis == 0 ? a.sx : a.sy);
-    const long long poff = a.axis == 0 ? (long long)other * a.sy : (long long)other * a.sx;  // plane offset in the shot
+    const int astride = (int)(axis == 0 ? a.sx : a.sy);
+    const long long poff = axis == 0 ? (long long)other * a.sy : (long long)other * a.sx;  // plane offset in the shot
     const long long ubase = (long long)shot * a.shot_stride + poff;
     const unsigned lvoff = 4u * (unsigned)(jj * astride + zl);  // lane byte offset from a uniform row
     float2* pen = lds + p * G::PS;
     load_twiddles<G>(tws, a.tw);
-    for (int jb = blockIdx.z; jb < a.njobs; jb += gridDim.z) {
+    for (int jb = jb0; jb < a.njobs; jb += pr.jz) {
         const DJob J = a.job[jb];
         __syncthreads();
         if (act1) {
@@ -222,7 +233,7 @@ void k2_deriv_strided(StridedArgs a)
             if (act1 && zok) {
 #pragma unroll
                 for (int j1 = 0; j1 < G::N1; ++j1) pen[jj + G::N2 * j1] = d[j1];
-                const int pml = a.pml, n = G::N;
+                constexpr int n = G::N;
                 // an opaque copy of the lane's row index: keeps the per-element
                 // C-PML indices and table loads inside the job loop instead of
                 // being hoisted (and held in registers through the FFTs)
@@ -234,7 +245,7 @@ void k2_deriv_strided(StridedArgs a)
                 // Chunks of CH elements: every load of a chunk (unconditional
                 // and in bounds - a non-slab element reads slab plane 0) before
                 // its stores, so the chunk's memory round trips overlap.
-                constexpr int CH = G::N1 % QVTI_VEL_CHUNK == 0 ? QVTI_VEL_CHUNK : 1;
+                constexpr int CH = vel_chunk(G::N1);
 #pragma unroll
                 for (int c0 = 0; c0 < G::N1; c0 += CH) {
                     float2 rr[CH], q[CH];
@@ -244,23 +255,18 @@ void k2_deriv_strided(StridedArgs a)
                     for (int jc = 0; jc < CH; ++jc) {
                         const int j1 = c0 + jc;
                         const int i = jl + G::N2 * j1;
-                        const long long urow = ubase + (long long)(G::N2 * j1) * astride;
                         float2 r = pen[i];
-                        const int ix = a.axis == 0 ? i : other;
-                        const int iy = a.axis == 0 ? other : i;
-                        upd[jc] = (i < pml || i >= n - pml) && ix < a.nx - 1 && iy < a.ny - 1;
+                        const int ix = axis == 0 ? i : other;
+                        const int iy = axis == 0 ? other : i;
+                        upd[jc] = (i < pml || i >= n - pml) && ix < nx - 1 && iy < ny - 1;
                         const int si = i < pml ? i : (i >= n - pml ? i - (n - 2 * pml) : 0);
-                        sidx[jc] = 4u * (unsigned)((a.axis == 0 ? si * a.ny + iy : ix * 2 * pml + si) * nz + zc);
+                        sidx[jc] = 4u * (unsigned)((axis == 0 ? si * ny + iy : ix * 2 * pml + si) * nz + zc);
                         const float2 q0 = ld2(phs, sidx[jc]);
                         const float A = ld1(pa, 4u * jl, 4 * G::N2 * j1), B = ld1(pb, 4u * jl, 4 * G::N2 * j1);
                         q[jc] = q0;
                         if (upd[jc]) {
-                            if (zc < nz - 1) { q[jc].x = q0.x + a.dt * (-A * q0.x - B * r.x); r.x = r.x + q[jc].x; }
-                            if (zc + 1 < nz - 1) { q[jc].y = q0.y + a.dt * (-A * q0.y - B * r.y); r.y = r.y + q[jc].y; }
-                        }
-                        if (MODE == MODE_VEL_ACC) {
-                            const float2 ac = ld2(row_at(J.acc, urow), o);
-                            r = make_float2(ac.x + r.x, ac.y + r.y);
+                            if (zc < nz - 1) { q[jc].x = q0.x + dt * (-A * q0.x - B * r.x); r.x = r.x + q[jc].x; }
+                            if (zc + 1 < nz - 1) { q[jc].y = q0.y + dt * (-A * q0.y - B * r.y); r.y = r.y + q[jc].y; }
                         }
                         rr[jc] = r;
                     }
@@ -315,6 +321,10 @@ struct StressXYArgs {
     int njobs;
     SJob job[4];
 };
+struct StressXYPair {
+    StressXYArgs a[2];  // one or two axes of one length
+    int jz;             // workgroups per tile and axis; grid z: (axis, job)
+};
 
 template <class G>
 // What bounds it at 256^3: 26 floats per cell (each sum reads S-bar) in 370 us
@@ -322,8 +332,10 @@ template <class G>
 // 4 waves per SIMD measure the same there (370-375 us), at 400x400x200 3 waves
 // are best (985 us; 1045 us with 2), hence the bounds.
 __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(G::NMAX <= 16 ? 4 : 3)))
-void k2_stress_xy(StressXYArgs a)
+void k2_stress_xy(StressXYPair pr)
 {
+    const int sel = blockIdx.z / pr.jz, jb0 = blockIdx.z - sel * pr.jz;
+    const StressXYArgs& a = pr.a[sel];
     __shared__ float2 lds[G::P * G::PS];
     __shared__ float2 tws[G::TWN];
     const int tid = threadIdx.x, shot = blockIdx.y;
@@ -344,7 +356,7 @@ void k2_stress_xy(StressXYArgs a)
     const unsigned lvoff = 4u * (unsigned)(jj * astride + zl);  // lane byte offset from a uniform row
     float2* pen = lds + p * G::PS;
     load_twiddles<G>(tws, a.tw);
-    for (int jb = blockIdx.z; jb < a.njobs; jb += gridDim.z) {
+    for (int jb = jb0; jb < a.njobs; jb += pr.jz) {
         const int np = a.job[jb].n;
         float acc[G::N1];
 #pragma unroll
@@ -442,7 +454,7 @@ struct VelZArgs {
     const float2 *symp, *symm;
     const float *pa, *pb, *pah, *pbh;
     const float *pxz, *pyz, *pzz;
-    const float* acc[3];
+    const float *accx[3], *accy[3];  // x and y derivatives (+ phi)
     float* v[3];
     float* w[3];
     const float* wab;  // {alpha, alpha kappa}
@@ -465,13 +477,13 @@ struct VelZArgs {
 // C-PML memory variable on the z-slab, v += b * (acc + dz + phi), dv = v_new
 // - v_old (+ the previous step's source at the injection cell), w = wa v +
 // wb dv.  Writes v and w (rows with rowdom / ok1 only), returns (v_new, w).
-// v, w, acc, bu, inj: uniform tile bases, `row` the byte offset of the lane's
+// v, w, accx, accy, bu, inj: uniform tile bases, `row` the byte offset of the lane's
 // row in them; ph: the shot's z-slabs, phrow the byte offset of the row's
 // 2*pml values.
 template <class G, bool INJ>
 __device__ __forceinline__ void vz_component(float2 (&out)[G::N1], const float2 (&d)[G::N1], const bool imag,
-                                             const Row v, const Row w, const float wa, const float wb, const Row acc,
-                                             const Row bu, const Row ph, const unsigned phrow, const Row pa,
+                                             const Row v, const Row w, const float wa, const float wb, const Row accx,
+                                             const Row accy, const Row bu, const Row ph, const unsigned phrow, const Row pa,
                                              const Row pb, const unsigned row, const int j, const int pml,
                                              const float dt, const bool rowdom, const bool ok1, const int src_iz,
                                              const float sprev, const Row inj)
@@ -483,8 +495,10 @@ __device__ __forceinline__ void vz_component(float2 (&out)[G::N1], const float2 
     // all loads and arithmetic first (every load unconditional and in bounds:
     // ph is a valid slab row even where it is not used), all stores after, so
     // no load waits behind a store or a branch
-    // (in chunks of QVTI_VZ_CHUNK elements, to bound the registers in flight)
-    constexpr int CH = G::N1 % QVTI_VZ_CHUNK == 0 ? QVTI_VZ_CHUNK : G::N1;
+    // (in chunks, to bound the registers in flight: up to 10 elements at once
+    // - n = 128: 53 -> 51 us at 128^3 against chunks of 4 - else as vel_chunk,
+    // 355 us at 256^3 against 368 us with all 16 at once)
+    constexpr int CH = G::N1 <= 10 ? G::N1 : vel_chunk(G::N1);
 #pragma unroll
     for (int c0 = 0; c0 < G::N1; c0 += CH) {
     float qn[CH];
@@ -492,7 +506,8 @@ __device__ __forceinline__ void vz_component(float2 (&out)[G::N1], const float2 
     for (int jc = 0; jc < CH; ++jc) {
         const int j1 = c0 + jc, im = 4 * G::N2 * j1;
         const int iz = jl + G::N2 * j1;
-        const float vold = ld1(v, o, im), bb = ld1(bu, o, im), ac = ld1(acc, o, im);
+        const float vold = ld1(v, o, im), bb = ld1(bu, o, im);
+        const float ac = ld1(accx, o, im) + ld1(accy, o, im);
         const bool slab = iz < pml || iz >= n - pml;
         const int si = iz < pml ? iz : (iz >= n - pml ? iz - (n - 2 * pml) : 0);
         const float q0 = ld1(ph, phrow + 4u * si), A = ld1(pa, 4u * jl, im), B = ld1(pb, 4u * jl, im);
@@ -519,7 +534,7 @@ __device__ __forceinline__ void vz_component(float2 (&out)[G::N1], const float2 
     }
 }
 
-template <class G, bool INJ = false>
+template <class G, bool INJ>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_VELZ_WAVES))) void k2_vel_z(VelZArgs a)
 {
     __shared__ float2 lds[G::P * G::PS];
@@ -584,7 +599,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
         const int src_iz = (kind == c && sip >= r1 * n && sip < (r1 + 1) * n) ? (int)(sip - r1 * n) : -1;
         const bool h = c == 2;
         const Row v = row_at(a.v[c], ubase);
-        vz_component<G, INJ>(out, d, imag, v, row_at(a.w[c], ubase), wa, wb, row_at(a.acc[c], ubase),
+        vz_component<G, INJ>(out, d, imag, v, row_at(a.w[c], ubase), wa, wb, row_at(a.accx[c], ubase),
+                        row_at(a.accy[c], ubase),
                         row_at(a.buoy[c], r0 * n), row_at(a.phi[c], (long long)shot * a.slab_stride), slab_row,
                         row_at(h ? a.pah : a.pa, 0), row_at(h ? a.pbh : a.pb, 0), lrow1, j, a.pml, a.dt, rowdom, ok1,
                         src_iz, sprev, INJ ? row_at(a.inj[c], ubase) : v);
@@ -856,6 +872,10 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
 // z-direction complex transforms on rows.
 //  mode 1 (inverse, stress step end): re_out + i im_out = IFFT_z(cin)   (either may be null)
 //  mode 2 (plain, standalone transforms): cout = FFT_z^DIR(cin), in place allowed
+// A last grid-z slice (rec.nt > 0) takes the receivers of the step: the
+// velocities are final since k2_vel_z except for the source, whose sample the
+// stress update adds to its cell after this kernel and record_sample adds here
+// (the same FP32 sum).  A launch of its own cost 3.9 us a step.
 struct ZRowsArgs {
     long long nrows;
     long long shot_stride;
@@ -865,6 +885,7 @@ struct ZRowsArgs {
     float2* cout[8];
     float* re_out[8];
     float* im_out[8];
+    RecArgs rec;
 };
 
 template <class G>
@@ -874,6 +895,11 @@ __global__ __launch_bounds__(kThreads) void k2_zrows(ZRowsArgs a)
     __shared__ float2 tws[G::TWN];
     constexpr int n = G::N;
     const int tid = threadIdx.x, shot = blockIdx.y;
+    if (a.rec.nt > 0 && blockIdx.z == gridDim.z - 1) {
+        record_samples(a.rec, shot, blockIdx.x * kThreads + tid, gridDim.x * kThreads);
+        return;
+    }
+    const int fz = a.rec.nt > 0 ? gridDim.z - 1 : gridDim.z;  // grid-z slices of the transforms
     const int j = tid % G::N2, p1 = tid / G::N2;
     const int k1 = tid % G::N1, p2 = tid / G::N1;
     const long long r0 = (long long)blockIdx.x * G::P, r1 = r0 + p1, r2 = r0 + p2;
@@ -882,7 +908,7 @@ __global__ __launch_bounds__(kThreads) void k2_zrows(ZRowsArgs a)
     float2* pen1 = lds + p1 * G::PS;
     float2* pen2 = lds + p2 * G::PS;
     load_twiddles<G>(tws, a.tw);
-    for (int f = blockIdx.z; f < a.nfields; f += gridDim.z) {
+    for (int f = blockIdx.z; f < a.nfields; f += fz) {
         __syncthreads();
         if (a.mode == 2 && a.dir < 0) {
             if (ok1) {

@@ -86,3 +86,29 @@ def test_strided_stress_derivatives_match_the_oracle(nx, ny, nz):
     assert err < TOL
     for st in got[1:]:
         assert np.array_equal(st, got[0])
+
+
+@pytest.mark.parametrize("kind", [O.SRC_FX, O.SRC_FY, O.SRC_FZ, O.SRC_EXPLOSIVE])
+def test_records_are_the_wavefield_after_the_source(kind):
+    """Receivers are sampled before the stress update adds the source to its
+    cell; the records must still be, bit for bit, the velocities that the
+    step leaves behind - at the source cell, beside it, and for shots with
+    more receivers than threads and with none."""
+    shot, model = small_case(18, 18, 20, 4, 6, kind, True)
+    src = (shot["sx"], shot["sy"], shot["sz"])
+    near = [src, (src[0], src[1], src[2] + 1), (0, 0, 0), (17, 17, 19)]
+    full = [(x, y, 7) for x in range(18) for y in range(18)] + near
+    sets = [near, full, []]
+    with qvti.Engine(18, 18, 20, shot["pml"], shot["dx"], shot["dy"], shot["dz"], shot["dt"], shot["f0"], shot["w0"],
+                     vti=True, max_shots=3) as e:
+        e.set_model_dict(model)
+        rs = [np.array(r, np.int32).reshape(-1, 3) for r in sets]
+        e.begin(shot["nt"], shot["rik"], [qvti.make_shot(kind, src, r[:, 0], r[:, 1], r[:, 2]) for r in rs])
+        want = []
+        for _ in range(shot["nt"]):
+            e.step(1)
+            want.append([e.state(k)[:3] for k in range(3)])
+        rec = e.finish()
+    for k, r in enumerate(rs):
+        for t in range(shot["nt"]):
+            assert np.array_equal(rec[k][:, t], want[t][k][:, r[:, 0], r[:, 1], r[:, 2]]), (k, t)

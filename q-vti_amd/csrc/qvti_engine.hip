@@ -742,12 +742,31 @@ static unsigned xcd_grid(int ntiles, unsigned S, int run)
 // the second one accumulating / with one: 64^3 85 / 81 us, 128^3 370 / 361 us,
 // 160x160x128 569 / 563 us, 256^3 2.708 / 2.699 ms, 400x400x200 equal.
 static bool merged_xy(const qvti_ctx* c) { return c->ops[0] == c->ops[1]; }
+// Non-temporal access for a launch of class cls whose tiles are `cols` floats
+// wide: only where the fields that pass from kernel to kernel outgrow the
+// Infinity Cache - the spectra (14 fields) for the velocity and transform
+// kernels, all of a step's fields for the stress kernels - and tiles and rows
+// are whole 128-byte lines.  Step with / without: 256^3 2.53 / 2.70 ms, 32
+// shots of 160x160x128 15.8 / 16.1 ms, 32 shots of 64^3 1.19 / 1.25 ms; at
+// 160x160x128 (spectra 184 MB) xpass, y_inv and z_inv take 44, 39 and 41 us
+// with, 41, 35 and 34 without, str_x and str_z 133 and 144 with, 146 and 156
+// without; 64^3 alone 82.8 / 81.4 us; 400x400x200 (rows end mid-line) 7.9 /
+// 6.8 ms.
+static bool stream_nt(const qvti_ctx* c, int cls, int cols)
+{
+    const bool stress = cls == KC_STR_X || cls == KC_STR_Y || cls == KC_STR_Z;
+    const long long bytes = 4 * (stress ? state_fields() : kFieldsA + kFieldsB) * c->N * c->nshots;
+    return bytes >= kStreamBytes && c->g.nz % 32 == 0 && cols % 32 == 0;
+}
+
 // Launch one kernel of class cls on the context's stream.
 static void launch_class(qvti_ctx* c, int cls)
 {
     hipStream_t st = c->stream;
     const unsigned S = (unsigned)c->nshots;
     const LenOps &X = *c->ops[0], &Y = *c->ops[1], &Z = *c->ops[2];
+    // width of a strided class's tiles in floats: cols per pencil
+    auto nt = [&](const LenOps& o, int cols) { return stream_nt(c, cls, o.P[pw_index(o, c->pw[cls])] * cols) ? 1 : 0; };
     auto strided = [&](const dim3& g) { return dim3(g.x, S, (unsigned)c->jz[cls]); };
     auto pair = [&](const dim3& g) { return dim3(g.x, S, (unsigned)(c->jz[cls] * (merged_xy(c) ? 2 : 1))); };
     switch (cls) {
@@ -759,26 +778,26 @@ static void launch_class(qvti_ctx* c, int cls)
         pr.a[1] = c->a_vy;
         pr.jz = c->jz[cls];
         const LenOps& O = cls == KC_VEL_X ? X : Y;
-        O.deriv[MODE_VEL][pw_index(O, c->pw[cls])](pair(cls == KC_VEL_X ? c->g_vx : c->g_vy), st, pr);
+        O.deriv[nt(O, 2)][pw_index(O, c->pw[cls])](pair(cls == KC_VEL_X ? c->g_vx : c->g_vy), st, pr);
         break;
     }
     case KC_VEL_Z:
         Z.vel_z[c->a_vz.inj[0] ? 1 : 0](dim3(xcd_grid(c->a_vz.ntiles, S, c->a_vz.run)), st, c->a_vz);
         break;
     case KC_Y_FWD:
-        Y.cfft[0][pw_index(Y, c->pw[cls])](strided(c->g_cy), st, c->a_yf);
+        Y.cfft[0][nt(Y, 2)][pw_index(Y, c->pw[cls])](strided(c->g_cy), st, c->a_yf);
         break;
     case KC_XPASS:
-        X.xpass[c->ks ? 1 : 0][pw_index(X, c->pw[cls])](strided(c->g_xp), st, c->a_xp);
+        X.xpass[c->ks ? 1 : 0][nt(X, 2)][pw_index(X, c->pw[cls])](strided(c->g_xp), st, c->a_xp);
         break;
     case KC_Y_INV:
-        Y.cfft[1][pw_index(Y, c->pw[cls])](strided(c->g_yi), st, c->a_yi);
+        Y.cfft[1][nt(Y, 2)][pw_index(Y, c->pw[cls])](strided(c->g_yi), st, c->a_yi);
         break;
     case KC_Z_INV: {
         const unsigned zs = QVTI_ZINV_SPLIT == 1 ? 1u : (unsigned)c->a_zi.nfields;
         c->a_zi.rec = c->a_rec;
         if (c->total_rec == 0) c->a_zi.rec.nt = 0;
-        Z.zrows(dim3(c->g_zr.x, S, zs + (c->a_zi.rec.nt > 0 ? 1 : 0)), st, c->a_zi);
+        Z.zrows[stream_nt(c, cls, 32) ? 1 : 0](dim3(c->g_zr.x, S, zs + (c->a_zi.rec.nt > 0 ? 1 : 0)), st, c->a_zi);
         break;
     }
     case KC_STR_X:
@@ -789,11 +808,11 @@ static void launch_class(qvti_ctx* c, int cls)
         pr.a[1] = c->a_sy;
         pr.jz = c->jz[cls];
         const LenOps& O = cls == KC_STR_X ? X : Y;
-        O.stress_xy[pw_index(O, c->pw[cls])](pair(cls == KC_STR_X ? c->g_sx : c->g_sy), st, pr);
+        O.stress_xy[nt(O, 1)][pw_index(O, c->pw[cls])](pair(cls == KC_STR_X ? c->g_sx : c->g_sy), st, pr);
         break;
     }
     case KC_STR_Z:
-        Z.stress_z[c->g.vti ? 1 : 0](dim3(xcd_grid(c->a_sz.ntiles, S, c->a_sz.run)), st, c->a_sz);
+        Z.stress_z[c->g.vti ? 1 : 0][!stream_nt(c, cls, 32) ? 0 : (S > 1 ? 1 : 2)](dim3(xcd_grid(c->a_sz.ntiles, S, c->a_sz.run)), st, c->a_sz);
         break;
     default:
         break;
@@ -1812,14 +1831,14 @@ static void enqueue_fft3d(int nx, int ny, int nz, int sign, float2* d, const flo
     ZRowsArgs z{};
     z.nrows = nrows; z.shot_stride = N; z.tw = tw[2]; z.mode = 2; z.dir = sign; z.nfields = 1;
     z.cin[0] = d; z.cout[0] = d;
-    Z.zrows(dim3((unsigned)((nrows + Z.Prow - 1) / Z.Prow), 1), st, z);
+    Z.zrows[0](dim3((unsigned)((nrows + Z.Prow - 1) / Z.Prow), 1), st, z);
     for (int axis = 1; axis >= 0; --axis) {
         const LenOps& A = *len_ops(dims[axis]);
         CStridedArgs y{};
         y.nz = nz; y.sx = (long long)ny * nz; y.sy = nz; y.axis = axis;
         y.ztiles = (nz + A.P[0] - 1) / A.P[0]; y.shot_stride = N; y.tw = tw[axis]; y.nfields = 1; y.f[0] = d;
         const int other = axis ? nx : ny;
-        A.cfft[sign < 0 ? 0 : 1][0](dim3((unsigned)(other * y.ztiles), 1), st, y);
+        A.cfft[sign < 0 ? 0 : 1][0][0](dim3((unsigned)(other * y.ztiles), 1), st, y);
     }
 }
 
@@ -1962,7 +1981,7 @@ extern "C" int qvti_deriv1d(int nx, int ny, int nz, float dd, int axis, int sym,
             a.job[0].in = din; a.job[0].out = dout; a.job[0].phi = nullptr;
             a.job[0].sym = 0; a.job[0].half = 0;
             const int other = axis == 0 ? ny : nx;
-            A.deriv[MODE_STORE][0](dim3((unsigned)(other * a.ztiles), 1), nullptr, pr);
+            A.deriv1d(dim3((unsigned)(other * a.ztiles), 1), nullptr, pr);
         } else {
             RowDerivArgs r{};
             const long long nrows = (long long)nx * ny;

@@ -10,40 +10,40 @@
 namespace qvti {
 namespace {
 
-template <class G, int MODE>
+template <class G, int MODE, bool NT>
 void l_deriv(dim3 grid, hipStream_t st, const StridedPair& a)
 {
-    hipLaunchKernelGGL((k2_deriv_strided<G, MODE>), grid, dim3(G::T), 0, st, a);
+    hipLaunchKernelGGL((k2_deriv_strided<G, MODE, NT>), grid, dim3(G::T), 0, st, a);
 }
-template <class G>
+template <class G, bool NT>
 void l_stress_xy(dim3 grid, hipStream_t st, const StressXYPair& a)
 {
-    hipLaunchKernelGGL(k2_stress_xy<G>, grid, dim3(G::T), 0, st, a);
+    hipLaunchKernelGGL((k2_stress_xy<G, NT>), grid, dim3(G::T), 0, st, a);
 }
-template <class G, int DIR>
+template <class G, int DIR, bool NT>
 void l_cfft(dim3 grid, hipStream_t st, const CStridedArgs& a)
 {
-    hipLaunchKernelGGL((k2_cfft_strided<G, DIR>), grid, dim3(G::T), 0, st, a);
+    hipLaunchKernelGGL((k2_cfft_strided<G, DIR, NT>), grid, dim3(G::T), 0, st, a);
 }
-template <class G, bool KS>
+template <class G, bool KS, bool NT>
 void l_xpass(dim3 grid, hipStream_t st, const XPassArgs& a)
 {
-    hipLaunchKernelGGL((k2_xpass<G, KS>), grid, dim3(G::T), 0, st, a);
+    hipLaunchKernelGGL((k2_xpass<G, KS, NT>), grid, dim3(G::T), 0, st, a);
 }
 template <class G, bool INJ>
 void l_vel_z(dim3 grid, hipStream_t st, const VelZArgs& a)
 {
     hipLaunchKernelGGL((k2_vel_z<G, INJ>), grid, dim3(kThreads), 0, st, a);
 }
-template <class G>
+template <class G, bool NT>
 void l_zrows(dim3 grid, hipStream_t st, const ZRowsArgs& a)
 {
-    hipLaunchKernelGGL(k2_zrows<G>, grid, dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL((k2_zrows<G, NT>), grid, dim3(kThreads), 0, st, a);
 }
-template <class G, bool VTI>
+template <class G, bool VTI, int NT>
 void l_stress_z(dim3 grid, hipStream_t st, const StressZArgs& a)
 {
-    hipLaunchKernelGGL((k2_stress_z<G, VTI>), grid, dim3(StressTile<G>::T), 0, st, a);
+    hipLaunchKernelGGL((k2_stress_z<G, VTI, NT>), grid, dim3(StressTile<G>::T), 0, st, a);
 }
 template <class G>
 void l_deriv_rows(dim3 grid, hipStream_t st, const RowDerivArgs& a)
@@ -59,33 +59,41 @@ constexpr bool pw_ok()
     else return A * B >= 64 && L2<A, B, PW>::kFits;
 }
 
+// A non-temporal variant exists where the tile is made of whole 128-byte
+// lines, `cols` floats per pencil; elsewhere its entry is the plain kernel.
+template <int A, int B, int PW, int COLS>
+constexpr bool lines()
+{
+    return L2<A, B, PW>::P * COLS % 32 == 0;
+}
+
 using DerivFn = void (*)(dim3, hipStream_t, const StridedPair&);
 using StressXYFn = void (*)(dim3, hipStream_t, const StressXYPair&);
 using CfftFn = void (*)(dim3, hipStream_t, const CStridedArgs&);
 using XpassFn = void (*)(dim3, hipStream_t, const XPassArgs&);
 
-template <int A, int B, int PW, int MODE>
+template <int A, int B, int PW, int MODE, bool NT>
 DerivFn deriv_fn()
 {
-    if constexpr (pw_ok<A, B, PW>()) return &l_deriv<L2<A, B, PW>, MODE>;
+    if constexpr (pw_ok<A, B, PW>()) return &l_deriv<L2<A, B, PW>, MODE, NT && lines<A, B, PW, 2>()>;
     else return nullptr;
 }
-template <int A, int B, int PW>
+template <int A, int B, int PW, bool NT>
 StressXYFn stress_xy_fn()
 {
-    if constexpr (pw_ok<A, B, PW>()) return &l_stress_xy<L2<A, B, PW>>;
+    if constexpr (pw_ok<A, B, PW>()) return &l_stress_xy<L2<A, B, PW>, NT && lines<A, B, PW, 1>()>;
     else return nullptr;
 }
-template <int A, int B, int PW, int DIR>
+template <int A, int B, int PW, int DIR, bool NT>
 CfftFn cfft_fn()
 {
-    if constexpr (pw_ok<A, B, PW>()) return &l_cfft<L2<A, B, PW>, DIR>;
+    if constexpr (pw_ok<A, B, PW>()) return &l_cfft<L2<A, B, PW>, DIR, NT && lines<A, B, PW, 2>()>;
     else return nullptr;
 }
-template <int A, int B, int PW, bool KS>
+template <int A, int B, int PW, bool KS, bool NT>
 XpassFn xpass_fn()
 {
-    if constexpr (pw_ok<A, B, PW>()) return &l_xpass<L2<A, B, PW>, KS>;
+    if constexpr (pw_ok<A, B, PW>()) return &l_xpass<L2<A, B, PW>, KS, NT && lines<A, B, PW, 2>()>;
     else return nullptr;
 }
 template <int A, int B, int PW>
@@ -104,22 +112,26 @@ template <int A, int B>
 LenOps make_ops()
 {
     using G = L2<A, B, 1>;
+    constexpr int kNt = A * B % 32 == 0 ? 1 : 0;  // rows of whole 128-byte lines
+#define QVTI_WIDTHS(fn, ...) {fn<A, B, kW0, __VA_ARGS__>(), fn<A, B, kW1, __VA_ARGS__>(), fn<A, B, kW2, __VA_ARGS__>()}
+#define QVTI_WIDTHS_NT(fn, ...) {QVTI_WIDTHS(fn, __VA_ARGS__, false), QVTI_WIDTHS(fn, __VA_ARGS__, true)}
     return LenOps{
         A * B, A, B, G::P, StressTile<G>::R,
         {pencils<A, B, kW0>(), pencils<A, B, kW1>(), pencils<A, B, kW2>()},
         {L2<A, B, kW0>::T, L2<A, B, kW1>::T, L2<A, B, kW2>::T},
-        {{deriv_fn<A, B, kW0, MODE_STORE>(), nullptr, nullptr},
-         {deriv_fn<A, B, kW0, MODE_VEL>(), deriv_fn<A, B, kW1, MODE_VEL>(), deriv_fn<A, B, kW2, MODE_VEL>()}},
-        {stress_xy_fn<A, B, kW0>(), stress_xy_fn<A, B, kW1>(), stress_xy_fn<A, B, kW2>()},
-        {{cfft_fn<A, B, kW0, -1>(), cfft_fn<A, B, kW1, -1>(), cfft_fn<A, B, kW2, -1>()},
-         {cfft_fn<A, B, kW0, 1>(), cfft_fn<A, B, kW1, 1>(), cfft_fn<A, B, kW2, 1>()}},
-        {{xpass_fn<A, B, kW0, false>(), xpass_fn<A, B, kW1, false>(), xpass_fn<A, B, kW2, false>()},
-         {xpass_fn<A, B, kW0, true>(), xpass_fn<A, B, kW1, true>(), xpass_fn<A, B, kW2, true>()}},
+        deriv_fn<A, B, kW0, MODE_STORE, false>(),
+        QVTI_WIDTHS_NT(deriv_fn, MODE_VEL),
+        {QVTI_WIDTHS(stress_xy_fn, false), QVTI_WIDTHS(stress_xy_fn, true)},
+        {QVTI_WIDTHS_NT(cfft_fn, -1), QVTI_WIDTHS_NT(cfft_fn, 1)},
+        {QVTI_WIDTHS_NT(xpass_fn, false), QVTI_WIDTHS_NT(xpass_fn, true)},
         {&l_vel_z<G, false>, &l_vel_z<G, true>},
-        &l_zrows<G>,
-        {&l_stress_z<G, false>, &l_stress_z<G, true>},
+        {&l_zrows<G, false>, &l_zrows<G, kNt != 0>},
+        {{&l_stress_z<G, false, 0>, &l_stress_z<G, false, kNt * 1>, &l_stress_z<G, false, kNt * 2>},
+         {&l_stress_z<G, true, 0>, &l_stress_z<G, true, kNt * 1>, &l_stress_z<G, true, kNt * 2>}},
         &l_deriv_rows<G>,
     };
+#undef QVTI_WIDTHS
+#undef QVTI_WIDTHS_NT
 }
 
 }  // namespace

@@ -20,15 +20,16 @@ struct LenOps {
     int Rsz;   // rows per workgroup of the stress update (StressTile)
     int P[3];  // pencils per tile of the strided kernels at width index 0, 1, 2 (0: not available)
     int T[3];  // threads per workgroup at width index 0, 1, 2
-    // strided-axis kernels, [..][pw index]
-    void (*deriv[2][3])(dim3 grid, hipStream_t st, const StridedPair& a);  // [MODE_*] (STORE: width index 0 only)
-    void (*stress_xy[3])(dim3 grid, hipStream_t st, const StressXYPair& a);
-    void (*cfft[2][3])(dim3 grid, hipStream_t st, const CStridedArgs& a);  // [0 forward, 1 inverse]
-    void (*xpass[2][3])(dim3 grid, hipStream_t st, const XPassArgs& a);    // [k-space mode off, on]
+    // strided-axis kernels, [..][non-temporal][pw index]
+    void (*deriv1d)(dim3 grid, hipStream_t st, const StridedPair& a);  // MODE_STORE, width index 0
+    void (*deriv[2][3])(dim3 grid, hipStream_t st, const StridedPair& a);
+    void (*stress_xy[2][3])(dim3 grid, hipStream_t st, const StressXYPair& a);
+    void (*cfft[2][2][3])(dim3 grid, hipStream_t st, const CStridedArgs& a);  // [0 forward, 1 inverse]
+    void (*xpass[2][2][3])(dim3 grid, hipStream_t st, const XPassArgs& a);    // [k-space mode off, on]
     // row (z) kernels, 256 threads (stress_z: StressTile)
     void (*vel_z[2])(dim3 grid, hipStream_t st, const VelZArgs& a);  // [without, with extra point sources]
-    void (*zrows)(dim3 grid, hipStream_t st, const ZRowsArgs& a);
-    void (*stress_z[2])(dim3 grid, hipStream_t st, const StressZArgs& a);  // [isotropic, VTI]
+    void (*zrows[2])(dim3 grid, hipStream_t st, const ZRowsArgs& a);  // [non-temporal]
+    void (*stress_z[2][3])(dim3 grid, hipStream_t st, const StressZArgs& a);  // [isotropic, VTI][NT]
     void (*deriv_rows)(dim3 grid, hipStream_t st, const RowDerivArgs& a);
 };
 

@@ -158,7 +158,8 @@ struct StridedPair {
     int jz;  // workgroups per tile and axis; grid z: (axis, job)
 };
 
-template <class G, int MODE>
+// NT: non-temporal loads and stores (stream_nt)
+template <class G, int MODE, bool NT>
 __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_STRIDED_WAVES)))
 void k2_deriv_strided(StridedPair pr)
 {
@@ -199,7 +200,7 @@ void k2_deriv_strided(StridedPair pr)
             const unsigned o = lane_off(lvoff);
 #pragma unroll
             for (int j1 = 0; j1 < G::N1; ++j1)
-                v[j1] = ld2(row_at(J.in, ubase + (long long)(j1 * G::N2) * astride), o);
+                v[j1] = ld2<NT>(row_at(J.in, ubase + (long long)(j1 * G::N2) * astride), o);
             fwd_l1<G>(v, pen, tws, jj);
         }
         __syncthreads();
@@ -271,12 +272,11 @@ void k2_deriv_strided(StridedPair pr)
                         rr[jc] = r;
                     }
 #pragma unroll
-                    for (int jc = 0; jc < CH; ++jc) {
-                        const int j1 = c0 + jc;
-                        const long long urow = ubase + (long long)(G::N2 * j1) * astride;
+                    for (int jc = 0; jc < CH; ++jc)
                         if (upd[jc]) st2(phs, sidx[jc], q[jc]);
-                        st2(row_at(J.out, urow), o, rr[jc]);
-                    }
+#pragma unroll
+                    for (int jc = 0; jc < CH; ++jc)
+                        st2<NT>(row_at(J.out, ubase + (long long)(G::N2 * (c0 + jc)) * astride), o, rr[jc]);
                     asm volatile("" ::: "memory");  // the next chunk's loads stay after this chunk
                 }
             }
@@ -326,7 +326,8 @@ struct StressXYPair {
     int jz;             // workgroups per tile and axis; grid z: (axis, job)
 };
 
-template <class G>
+// NT: non-temporal field loads and stores (stream_nt)
+template <class G, bool NT>
 // What bounds it at 256^3: 26 floats per cell (each sum reads S-bar) in 370 us
 // along x, 4.7 TB/s, with the VALU busy for about half of that time; 2, 3 and
 // 4 waves per SIMD measure the same there (370-375 us), at 400x400x200 3 waves
@@ -372,7 +373,7 @@ void k2_stress_xy(StressXYPair pr)
 #pragma unroll
                 for (int j1 = 0; j1 < G::N1; ++j1) {
                     const long long row = (long long)(j1 * G::N2) * astride;
-                    v[j1] = make_float2(ld1(row_at(re, row), o), ld1(row_at(im, row), o));
+                    v[j1] = make_float2(ld1<NT>(row_at(re, row), o), ld1<NT>(row_at(im, row), o));
                 }
                 fwd_l1<G>(v, pen, tws, jj);
             }
@@ -414,8 +415,8 @@ void k2_stress_xy(StressXYPair pr)
                     for (int j1 = 0; j1 < G::N1; ++j1) {
                         const unsigned ip = ip0 + (unsigned)(G::N2 * j1 * astride);
                         const unsigned o = 4u * ((ip >> 6) * (unsigned)(kBlk * kDer) + (ip & 63u));
-                        st1(ore, o, d[j1].x);
-                        st1(oim, o, d[j1].y);
+                        st1<NT>(ore, o, d[j1].x);
+                        st1<NT>(oim, o, d[j1].y);
                     }
                 } else {
 #pragma unroll
@@ -429,7 +430,7 @@ void k2_stress_xy(StressXYPair pr)
 #pragma unroll
             for (int j1 = 0; j1 < G::N1; ++j1) {
                 const unsigned ip = ip0 + (unsigned)(G::N2 * j1 * astride);
-                st1(ob, 4u * ((ip >> 6) * (unsigned)(kBlk * kDer) + (ip & 63u)), acc[j1]);
+                st1<NT>(ob, 4u * ((ip >> 6) * (unsigned)(kBlk * kDer) + (ip & 63u)), acc[j1]);
             }
         }
     }
@@ -671,7 +672,8 @@ struct CStridedArgs {
     float2* f[8];
 };
 
-template <class G, int DIR>
+// NT: non-temporal loads (stream_nt); the stores feed the next kernel's rows
+template <class G, int DIR, bool NT>
 __global__ __launch_bounds__(G::T) void k2_cfft_strided(CStridedArgs a)
 {
     __shared__ float2 lds[G::P * G::PS];
@@ -700,7 +702,8 @@ __global__ __launch_bounds__(G::T) void k2_cfft_strided(CStridedArgs a)
             if (act1) {
                 float2 v[G::N1];
 #pragma unroll
-                for (int j1 = 0; j1 < G::N1; ++j1) v[j1] = ld2(row_at(fb, (long long)(j1 * G::N2) * astride), o);
+                for (int j1 = 0; j1 < G::N1; ++j1)
+                    v[j1] = ld2<NT>(row_at(fb, (long long)(j1 * G::N2) * astride), o);
                 fwd_l1<G>(v, pen, tws, jj);
             }
             __syncthreads();
@@ -714,7 +717,8 @@ __global__ __launch_bounds__(G::T) void k2_cfft_strided(CStridedArgs a)
             if (act2) {
                 float2 b[G::N2];
 #pragma unroll
-                for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = ld2(row_at(fb, (long long)(G::N1 * k2) * astride), o);
+                for (int k2 = 0; k2 < G::N2; ++k2)
+                    b[k2] = ld2<NT>(row_at(fb, (long long)(G::N1 * k2) * astride), o);
                 inv_la<G>(b, pen, tws + G::T2OFF, jj);
             }
             __syncthreads();
@@ -778,7 +782,8 @@ __device__ __forceinline__ float kspace_factor(const XPassArgs& a, float k)
     return f;
 }
 
-template <class G, bool KS = false>
+// NT: non-temporal loads and stores (stream_nt)
+template <class G, bool KS, bool NT>
 __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS_WAVES))) void k2_xpass(XPassArgs a)
 {
     __shared__ float2 lds[G::P * G::PS];
@@ -808,7 +813,7 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
             float2 v[G::N1];
             const unsigned o = lane_off(voff);
 #pragma unroll
-            for (int j1 = 0; j1 < G::N1; ++j1) v[j1] = ld2(row_at(src, (long long)(j1 * G::N2) * sxi), o);
+            for (int j1 = 0; j1 < G::N1; ++j1) v[j1] = ld2<NT>(row_at(src, (long long)(j1 * G::N2) * sxi), o);
             fwd_l1<G>(v, pen, tws, jj);
         }
         __syncthreads();
@@ -862,7 +867,7 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
                 float2* const dst = q + tbase;
                 const unsigned o = lane_off(voff);
 #pragma unroll
-                for (int j1 = 0; j1 < G::N1; ++j1) st2(row_at(dst, (long long)(G::N2 * j1) * sxi), o, d[j1]);
+                for (int j1 = 0; j1 < G::N1; ++j1) st2<NT>(row_at(dst, (long long)(G::N2 * j1) * sxi), o, d[j1]);
             }
         }
     }
@@ -888,7 +893,8 @@ struct ZRowsArgs {
     RecArgs rec;
 };
 
-template <class G>
+// NT: non-temporal loads (stream_nt)
+template <class G, bool NT>
 __global__ __launch_bounds__(kThreads) void k2_zrows(ZRowsArgs a)
 {
     __shared__ float2 lds[G::P * G::PS];
@@ -934,7 +940,7 @@ __global__ __launch_bounds__(kThreads) void k2_zrows(ZRowsArgs a)
                 const Row src = row_at(a.cin[f], soff + r0 * n);
                 const unsigned o = lane_off(8u * (unsigned)(p2 * n + k1));
 #pragma unroll
-                for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = ld2(src, o, 8 * G::N1 * k2);
+                for (int k2 = 0; k2 < G::N2; ++k2) b[k2] = ld2<NT>(src, o, 8 * G::N1 * k2);
                 inv_la<G>(b, pen2, tws + G::T2OFF, k1);
             }
             __syncthreads();
@@ -1084,7 +1090,11 @@ struct StressTile {
 // staging field index = 2*kind (+1 for the imaginary part)
 //   c     (0-2): A1 w_c + i A2 w_c    3 + c (3-5): A2 v_c + i A3 v_c
 // (c = 2: D+, else D-)
-template <class G, bool VTI>
+// NT (stream_nt): 1 loads the derivatives non-temporally, 2 (one shot) the
+// coefficients and stresses as well - with several shots the coefficients are
+// read again for the next shot of the tile.  256^3: 714 -> 657 us (2), 32
+// shots of 160x160x128: 4234 -> 4192 us (1; 4260 with 2).
+template <class G, bool VTI, int NT>
 __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_eu(QVTI_STRESSZ_WAVES))) void k2_stress_z(
     StressZArgs a)
 {
@@ -1200,26 +1210,26 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
             constexpr int FB = 4 * kBlk;  // bytes between the fields of a block
             float oP[kFam], oS[kFam], oH[kFam], oD[kFam];
             {
-                const float r = ld1(g1r, o1, 4 * FB);
-                set_coeffs(oP, ld1(g1r, o1), ld1(g1r, o1, FB), r, alpha, s4);
-                set_coeffs(oS, ld1(g1r, o1, 2 * FB), ld1(g1r, o1, 3 * FB), r, alpha, s4);
+                const float r = ld1<(NT > 1)>(g1r, o1, 4 * FB);
+                set_coeffs(oP, ld1<(NT > 1)>(g1r, o1), ld1<(NT > 1)>(g1r, o1, FB), r, alpha, s4);
+                set_coeffs(oS, ld1<(NT > 1)>(g1r, o1, 2 * FB), ld1<(NT > 1)>(g1r, o1, 3 * FB), r, alpha, s4);
                 if (vti) {
-                    set_coeffs(oH, ld1(g2r, o2), ld1(g2r, o2, FB), r, alpha, s4);
-                    set_coeffs(oD, ld1(g2r, o2, 2 * FB), ld1(g2r, o2, 3 * FB), r, alpha, s4);
+                    set_coeffs(oH, ld1<(NT > 1)>(g2r, o2), ld1<(NT > 1)>(g2r, o2, FB), r, alpha, s4);
+                    set_coeffs(oD, ld1<(NT > 1)>(g2r, o2, 2 * FB), ld1<(NT > 1)>(g2r, o2, 3 * FB), r, alpha, s4);
                 }
             }
             float A[14];
 #pragma unroll
             for (int k = 0; k < 14; ++k) A[k] = 0.f;
-            A[9] = ld1(dxr, od, kFam * FB);         // sb_zx  (dx vz)
-            A[11] = ld1(dxr, od, (kFam + 1) * FB);  // sb_yx  (dx vy)
-            A[13] = ld1(dyr, od, kFam * FB);        // sb_zy  (dy vz)
-            A[10] = ld1(dyr, od, (kFam + 1) * FB);  // sb_xy  (dy vx)
+            A[9] = ld1<(NT > 0)>(dxr, od, kFam * FB);         // sb_zx  (dx vz)
+            A[11] = ld1<(NT > 0)>(dxr, od, (kFam + 1) * FB);  // sb_yx  (dx vy)
+            A[13] = ld1<(NT > 0)>(dyr, od, kFam * FB);        // sb_zy  (dy vz)
+            A[10] = ld1<(NT > 0)>(dyr, od, (kFam + 1) * FB);  // sb_xy  (dy vx)
 #pragma unroll
             for (int jf = 0; jf < kFam; ++jf) {
                 const float ez = S(fz[jf]), gz = S(fgx[jf]), hz = S(fhy[jf]);
-                const float ex = ld1(dxr, od, jf * FB), ey = ld1(dyr, od, jf * FB);
-                const float c33 = oP[jf], cs = oS[jf], csb = ld1(gsr[jf], oc);
+                const float ex = ld1<(NT > 0)>(dxr, od, jf * FB), ey = ld1<(NT > 0)>(dyr, od, jf * FB);
+                const float c33 = oP[jf], cs = oS[jf], csb = ld1<(NT > 1)>(gsr[jf], oc);
                 const float c11 = vti ? oH[jf] : c33, c13 = vti ? oD[jf] : c33;
                 const float c12 = c11 - 2 * cs, c13d = c13 - 2 * cs;
                 A[0] += c11 * ex;   // s11x
@@ -1238,7 +1248,7 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
             // know it, so loads placed after a store would each wait for it.
             float sg[6];
 #pragma unroll
-            for (int k = 0; k < 6; ++k) sg[k] = ld1(sgr[k], oc);
+            for (int k = 0; k < 6; ++k) sg[k] = ld1<(NT > 1)>(sgr[k], oc);
             const bool xs = ix < pml || ix >= a.nx - pml;
             const bool ys = iy < pml || iy >= a.ny - pml;
             const bool zs = iz < pml || iz >= n - pml;
@@ -1302,12 +1312,12 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
                 a.phz[2][szb + oz] = fxz;
                 a.phz[3][szb + oz] = fyz;
             }
-            st1(sgr[0], oc, sg[0] + dt * (A[0] + A[3] + A[6] + (fxx_x + fyx_y + fzx_z)));
-            st1(sgr[1], oc, sg[1] + dt * (A[1] + A[4] + A[6] + (fxy_x + fyy_y + fzx_z)));
-            st1(sgr[2], oc, sg[2] + dt * (A[2] + A[5] + A[7] + (fxz_x + fyz_y + fzz_z)));
-            st1(sgr[3], oc, sg[3] + dt * (A[10] + fxy + A[11] + fyx));
-            st1(sgr[4], oc, sg[4] + dt * (A[8] + fxz + A[9] + fzx));
-            st1(sgr[5], oc, sg[5] + dt * (A[12] + fyz + A[13] + fzy));
+            st1<(NT > 1)>(sgr[0], oc, sg[0] + dt * (A[0] + A[3] + A[6] + (fxx_x + fyx_y + fzx_z)));
+            st1<(NT > 1)>(sgr[1], oc, sg[1] + dt * (A[1] + A[4] + A[6] + (fxy_x + fyy_y + fzx_z)));
+            st1<(NT > 1)>(sgr[2], oc, sg[2] + dt * (A[2] + A[5] + A[7] + (fxz_x + fyz_y + fzz_z)));
+            st1<(NT > 1)>(sgr[3], oc, sg[3] + dt * (A[10] + fxy + A[11] + fyx));
+            st1<(NT > 1)>(sgr[4], oc, sg[4] + dt * (A[8] + fxz + A[9] + fzx));
+            st1<(NT > 1)>(sgr[5], oc, sg[5] + dt * (A[12] + fyz + A[13] + fzy));
         }
         if (row * n + iz == sip) {
             // source after the stress update; no other workgroup of this

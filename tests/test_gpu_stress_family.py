@@ -112,3 +112,34 @@ def test_records_are_the_wavefield_after_the_source(kind):
     for k, r in enumerate(rs):
         for t in range(shot["nt"]):
             assert np.array_equal(rec[k][:, t], want[t][k][:, r[:, 0], r[:, 1], r[:, 2]]), (k, t)
+
+
+@pytest.mark.parametrize("nx,ny,nz,shots", [(96, 90, 512, 1), (128, 128, 128, 1), (64, 48, 96, 17), (160, 160, 64, 4)])
+def test_streaming_variants_give_the_same_bits(nx, ny, nz, shots):
+    """Grids beyond the Infinity Cache take non-temporal variants of the
+    kernels (all of them, or the stress kernels only).  Shot 0 of the batch
+    must equal the same shot run alone on a context of one shot, and every
+    tile width must give the same bits (widths differ in which tiles are whole
+    lines); the first case, one shot, is checked against the oracle."""
+    shot, model = small_case(nx, ny, nz, 6, 3, O.SRC_FZ, True, seed=5)
+
+    def run(n, mode):
+        with qvti.Engine(nx, ny, nz, shot["pml"], shot["dx"], shot["dy"], shot["dz"], shot["dt"], shot["f0"],
+                         shot["w0"], vti=True, max_shots=n) as e:
+            e.set_autotune(mode)
+            e.set_model_dict(model)
+            e.begin(shot["nt"], shot["rik"],
+                    [qvti.make_shot(shot["src_kind"], (shot["sx"] + k % 3, shot["sy"], shot["sz"]), shot["rx"],
+                                    shot["ry"], shot["rz"]) for k in range(n)])
+            e.step(shot["nt"])
+            e.finish()
+            return e.state(0)
+
+    ref = run(1, 0)
+    for mode in (0, 2, 4, 16):
+        assert np.array_equal(run(shots, mode), ref), mode
+    if (nx, ny, nz) == (96, 90, 512):
+        want = O.run(shot, model, "f64", state=True)["state"]
+        err = rel_l2(ref, want)
+        print("%dx%dx%d: state vs FP64 oracle %.2e" % (nx, ny, nz, err))
+        assert err < TOL

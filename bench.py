@@ -13,7 +13,7 @@ bandwidth probe - and the CPU baseline.  Prints ONE JSON line.
   python bench.py --summarize-pmc DIR [DIR ...]
 
 value = total cells x K / timed wall seconds / 1e9 (Gcell-steps/s) over K
-steps of the production path (HIP graph per step), bracketed by device
+steps of the production path (HIP graphs of several steps), bracketed by device
 synchronisations.  A second region of K steps launches the same kernels
 directly with every launch bracketed by HIP events on the engine's stream;
 the dominant kernel's average duration there gives the achieved algorithmic
@@ -80,7 +80,7 @@ def engine(g, max_shots=1):
 
 def run_plain(name, steps, warmup, kspace_vref=0.0, tiles=1):
     """Two timed regions of `steps` steps each on one shot, after `warmup`
-    steps: (1) the production path (one HIP graph per step, blow-up probe
+    steps: (1) the production path (graphs of several steps, blow-up probe
     every 50 steps) gives the throughput; (2) the same kernels launched
     directly, each bracketed by HIP events on the engine's stream, gives the
     per-kernel average durations.  kspace_vref > 0 runs the opt-in k-space

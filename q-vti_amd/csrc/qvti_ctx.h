@@ -61,7 +61,7 @@ struct qvti_ctx {
     int* d_rec_off = nullptr;
     int total_rec = 0;
     float* d_rec = nullptr;
-    long long rec_cap = 0;
+    long long rec_cap = 0, rec_ip_cap = 0, rik_cap = 0;  // elements allocated
     int probe_every = 50;
     float probe_limit = 1e30f;
     // snapshot of the box [snap_lo, snap_hi) (default: the interior window)
@@ -74,7 +74,7 @@ struct qvti_ctx {
     long long snap_lim = 0;      // floats this run may write: min(box * snapshots, snap_cap)
     // graphs
     bool use_graphs = true;
-    hipGraphExec_t gexec = nullptr;
+    hipGraphExec_t gexec = nullptr;  // kGraphSteps steps of the current run
     // timing
     bool timing = false;
     int ev_max = 0, ev_used = 0;

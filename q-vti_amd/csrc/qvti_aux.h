@@ -72,9 +72,12 @@ static __global__ __launch_bounds__(256) void k_snapshot(SnapArgs a)
 }
 
 // Blow-up probe: max |v| over a field (bit pattern of a non-negative float
-// orders like an int; NaN sorts above Inf).
+// orders like an int; NaN sorts above Inf).  One atomic per workgroup, and none
+// where the running maximum already covers it: with one per wave, all to one
+// address, 64^3 took 50 us.
 static __global__ __launch_bounds__(256) void k_probe(const float* f, long long N, int* out)
 {
+    __shared__ int wave[4];
     int m = 0;
     for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < N; q += (long long)gridDim.x * 256) {
         const int b = __float_as_int(fabsf(f[q]));
@@ -84,7 +87,11 @@ static __global__ __launch_bounds__(256) void k_probe(const float* f, long long 
         const int o = __shfl_down(m, off);
         m = o > m ? o : m;
     }
-    if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+    if ((threadIdx.x & 63) == 0) wave[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 1; k < 4; ++k) m = wave[k] > m ? wave[k] : m;
+    if (m > *out) atomicMax(out, m);  // (a stale read only costs an atomic: *out never falls during a run)
 }
 
 // ---- setup kernels (once per model) ------------------------------------

@@ -782,7 +782,7 @@ static void launch_class(qvti_ctx* c, int cls)
         break;
     }
     case KC_VEL_Z:
-        Z.vel_z[c->a_vz.inj[0] ? 1 : 0](dim3(xcd_grid(c->a_vz.ntiles, S, c->a_vz.run)), st, c->a_vz);
+        Z.vel_z[c->a_vz.inj[0] ? 1 : 0](dim3(xcd_grid(c->a_vz.ntiles, S, c->a_vz.run), 2), st, c->a_vz);
         break;
     case KC_Y_FWD:
         Y.cfft[0][nt(Y, 2)][pw_index(Y, c->pw[cls])](strided(c->g_cy), st, c->a_yf);
@@ -1142,7 +1142,8 @@ extern "C" int qvti_step(qvti_ctx* c, int nsteps)
         c->steps_done += graph ? kGraphSteps : 1;
         if (c->probe_every > 0 && (c->steps_done % c->probe_every == 0 || c->steps_done == c->nt)) {
             const int e0 = c->timing ? record_event(c, KC_PROBE) : -1;
-            hipLaunchKernelGGL(k_probe, dim3(1024), dim3(kThreads), 0, c->stream, (const float*)c->v, nprobe, c->d_probe);
+            const unsigned pg = (unsigned)std::min<long long>((nprobe + 4095) / 4096, 1024);
+            hipLaunchKernelGGL(k_probe, dim3(pg), dim3(kThreads), 0, c->stream, (const float*)c->v, nprobe, c->d_probe);
             if (e0 >= 0) record_event(c, -1 - KC_PROBE);
         }
     }

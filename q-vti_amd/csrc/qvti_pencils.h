@@ -1,7 +1,7 @@
 // qvti_pencils.h -- pencil kernels of the time step on the two-level register
 // FFT (qvti_fft2l.h).  Every kernel is a template over the split G = L2<N1,N2,PW>
 // of its axis length; the row (z) kernels run 256 threads, the strided-axis
-// (x, y) kernels 256*PW (the tile width the autotuner picks).
+// (x, y) kernels up to 256*PW (the tile width the autotuner picks).
 //
 // Per step (reference loop: cuviscoelas_3D.cu:1255-1605):
 //   velocity half-step   k2_deriv_strided (x and y; advances the step counter)
@@ -442,6 +442,11 @@ void k2_stress_xy(StressXYPair pr)
 //   v += b * (acc_xy + dz sigma + phi_z);  dv = v_new - v_old + src_prev;
 //   w = alpha v + (alpha kappa) dv;
 //   P0 = FFT_z(wx + i wy), P1 = FFT_z(wz + i vz), P2 = FFT_z(vx + i vy)
+// Two workgroups per tile (grid y): vx and vy with P0 and P2, and vz with P1.
+// They share nothing but the twiddles, and the chain of dependent transforms,
+// which bounds the kernel where a grid has few tiles, is a third shorter:
+// 64^3 20 -> 15 us, 160x160x128 78 -> 73 us, 256^3 349 -> 345 us (5.2 TB/s),
+// 400x400x200 751 -> 738 us.
 // dv is the change since the previous step's pre-injection velocity (the
 // reference's V - V_prev, cuviscoelas_3D.cu:517-522, 1124-1131, without 1/dt).
 // Tile: G::P rows (z-pencils).
@@ -624,7 +629,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
     // Packing of the stress step's transforms: P0 = F(wx + i wy),
     // P1 = F(wz + i vz), P2 = F(vx + i vy).  A1 is needed on P0 and P1, A3 on
     // P1 and P2.
-    {
+    if (blockIdx.y == 0) {
         float2 d[G::N1];
         deriv(a.pxz, a.pyz, a.symp, d);  // dz pxz (vx) + i dz pyz (vy), D+
         float2 u[G::N1];
@@ -645,8 +650,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
         }
         fft_store(x0, a.P[0]);
         fft_store(x1, a.P[2]);
-    }
-    {
+    } else {
         float2 d[G::N1];
         deriv(a.pzz, nullptr, a.symm, d);  // dz pzz (vz), D-
         float2 x2[G::N1];
@@ -1116,10 +1120,9 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
     const long long soff = (long long)shot * a.shot_stride;
     float2* pen1 = lds + q1 * G::PS;
     float2* pen2 = lds + q2 * G::PS;
-    for (int t = tid; t < G::TWN; t += T::T) twiddle_entry<G>(tws, a.tw, t);
-    __syncthreads();
     {
         const int kind1 = q1 % 6, rr1 = q1 / 6;
+        float2 v[G::N1];  // on its way while the twiddle tables load (256^3: 665 -> 655 us)
         if (act1) {
             const long long row1 = r0 + rr1;
             const bool ok1 = row1 < a.nrows;
@@ -1128,13 +1131,12 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
             const long long g = soff + (ok1 ? row1 : r0) * n + j;
             const float* fre = a.fam[c][kind1 < 3 ? 0 : 1] + g;
             const float* fim = a.fam[c][kind1 < 3 ? 3 : 2] + g;
-            float2 v[G::N1];
 #pragma unroll
-            for (int j1 = 0; j1 < G::N1; ++j1) {
-                v[j1] = make_float2(fre[j1 * G::N2], fim[j1 * G::N2]);
-            }
-            fwd_l1<G>(v, pen1, tws, j);
+            for (int j1 = 0; j1 < G::N1; ++j1) v[j1] = make_float2(fre[j1 * G::N2], fim[j1 * G::N2]);
         }
+        for (int t = tid; t < G::TWN; t += T::T) twiddle_entry<G>(tws, a.tw, t);
+        __syncthreads();
+        if (act1) fwd_l1<G>(v, pen1, tws, j);
         __syncthreads();
         float2 b[G::N2];
         if (act2) {

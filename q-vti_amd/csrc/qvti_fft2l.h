@@ -219,16 +219,21 @@ __host__ __device__ __forceinline__ void rdft(float2* v)
 }
 
 // Per-length constants of the two-level scheme.  PW widens the tile of the
-// strided-axis kernels: a workgroup of T = 256*PW threads holds P = T/NMAX
-// pencils, so each row of the tile is P (complex) or 2P (real) contiguous
-// z-columns wide.
+// strided-axis kernels: a workgroup of T threads holds P pencils of NMAX
+// threads, so each row of the tile is P (complex) or 2P (real) contiguous
+// z-columns wide: as many as 256 PW threads hold, except that PW = 4 takes a
+// multiple of 32 where NMAX is not a power of two, so that the rows are whole
+// 128-byte lines in every kernel (n = 400: 12, 25 and 32 pencils; it has no
+// LDS for 51).  324x270x128 2118 -> 1969 us a step, 320x180x64 685 -> 637 us,
+// 400x400x200 6.07 -> 5.93 ms.
 template <int N1_, int N2_, int PW_ = 1>
 struct L2 {
     static constexpr int N1 = N1_, N2 = N2_, N = N1_ * N2_;
     static constexpr int NMAX = N1 > N2 ? N1 : N2;
     static constexpr int PW = PW_;
-    static constexpr int T = 256 * PW_;           // threads per workgroup
-    static constexpr int P = T / NMAX;            // pencils per tile
+    static constexpr int P4 = 1024 / NMAX;
+    static constexpr int P = PW < 4 ? 256 * PW / NMAX : ((NMAX & (NMAX - 1)) == 0 || P4 < 32 ? P4 : P4 / 32 * 32);  // pencils per tile
+    static constexpr int T = PW < 4 ? 256 * PW : (P * NMAX + 63) / 64 * 64;  // threads per workgroup
     // LDS layout of one pencil: Y rows k1 of length N2 padded by one, Z rows ja
     // of length N1 padded by one; the pencil stride is odd (bank spread).
     static constexpr int YS = N2 + 1, ZS = N1 + 1;
@@ -241,7 +246,7 @@ struct L2 {
     static constexpr int T2OFF = N1 == N2 ? 0 : N;
     static constexpr int TWN = N + T2OFF;
     // LDS of a strided tile (pencils + twiddles) within the 160 KiB of a CU
-    static constexpr bool kFits = 8L * (P * PS + TWN) <= 160L * 1024;
+    static constexpr bool kFits = T <= 1024 && 8L * (P * PS + TWN) <= 160L * 1024;
 };
 
 // Fill the twiddle tables (G::TWN entries) from tw[m] = W_N^m.

@@ -4,7 +4,7 @@
 // length (qvti_pencils.h).  Each supported length gets one LenOps record of
 // launch functions, defined in the build group of qvti_kernels.hip that the
 // length belongs to (qvti_lengths.h); the groups compile in parallel.  Tile
-// widths PW = 1, 2, 4 (256, 512, 1024 threads) are indexed 0, 1, 2; a width
+// widths PW = 1, 2, 4 (256, 512, up to 1024 threads) are indexed 0, 1, 2; a width
 // that a length does not support (short axes, LDS) has null entries.
 #pragma once
 #include <hip/hip_runtime.h>

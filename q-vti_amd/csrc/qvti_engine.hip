@@ -759,6 +759,12 @@ static bool stream_nt(const qvti_ctx* c, int cls, int cols)
     return bytes >= kStreamBytes && c->g.nz % 32 == 0 && cols % 32 == 0;
 }
 
+// Shots that k2_stress_xy interleaves on grid x.  All of them, where the four
+// S-bar fields are beyond one XCD's 4 MB of L2 (32 shots of 160x160x128: 3615
+// -> 3346 us); else none (32 shots of 64^3, whose S-bar fits: 238 us, 252
+// interleaved).
+static int stress_xy_shots(const qvti_ctx* c) { return 16 * c->N > (4LL << 20) ? c->nshots : 1; }
+
 // Launch one kernel of class cls on the context's stream.
 static void launch_class(qvti_ctx* c, int cls)
 {
@@ -807,8 +813,10 @@ static void launch_class(qvti_ctx* c, int cls)
         pr.a[0] = cls == KC_STR_X ? c->a_sx : c->a_sy;
         pr.a[1] = c->a_sy;
         pr.jz = c->jz[cls];
+        pr.nshots = stress_xy_shots(c);
+        const dim3 g = pair(cls == KC_STR_X ? c->g_sx : c->g_sy);
         const LenOps& O = cls == KC_STR_X ? X : Y;
-        O.stress_xy[nt(O, 1)][pw_index(O, c->pw[cls])](pair(cls == KC_STR_X ? c->g_sx : c->g_sy), st, pr);
+        O.stress_xy[nt(O, 1)][pw_index(O, c->pw[cls])](dim3(g.x * pr.nshots, S / pr.nshots, g.z), st, pr);
         break;
     }
     case KC_STR_Z:

@@ -100,9 +100,8 @@ __device__ __forceinline__ TileShot tile_shot(int ntiles, int nshots, int run)
 struct PlaneTile {
     int plane, zt;
 };
-__device__ __forceinline__ PlaneTile plane_tile(int ztiles, int nplanes, int run)
+__device__ __forceinline__ PlaneTile plane_tile(int ztiles, int nplanes, int run, int id)
 {
-    const int id = blockIdx.x;
     if (!run) {
         const int pl = id / ztiles;
         return {pl, id - pl * ztiles};
@@ -171,7 +170,7 @@ void k2_deriv_strided(StridedPair pr)
     // one thread of the grid advances the step counter; the kernels of the
     // step that read it run after this one
     if (a.tick != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && tid == 0) *a.tick = *a.tick + 1;
-    const PlaneTile pt = plane_tile(a.ztiles, a.nplanes, a.run);
+    const PlaneTile pt = plane_tile(a.ztiles, a.nplanes, a.run, blockIdx.x);
     if (pt.plane < 0) return;
     const int other = pt.plane;
     const int p = tid % G::P, jj = tid / G::P;
@@ -324,6 +323,7 @@ struct StressXYArgs {
 struct StressXYPair {
     StressXYArgs a[2];  // one or two axes of one length
     int jz;             // workgroups per tile and axis; grid z: (axis, job)
+    int nshots;         // shots interleaved on grid x, or 1
 };
 
 // NT: non-temporal field loads and stores (stream_nt)
@@ -339,8 +339,12 @@ void k2_stress_xy(StressXYPair pr)
     const StressXYArgs& a = pr.a[sel];
     __shared__ float2 lds[G::P * G::PS];
     __shared__ float2 tws[G::TWN];
-    const int tid = threadIdx.x, shot = blockIdx.y;
-    const PlaneTile pt = plane_tile(a.ztiles, a.nplanes, a.run);
+    const int tid = threadIdx.x;
+    // pr.nshots > 1: the shots of one tile follow each other on one XCD (as
+    // tile_shot), so the S-bar values are read from its L2 after the first
+    // shot; 1: the shots are on grid y (stress_xy_shots)
+    const int q = (int)(blockIdx.x >> 3) / pr.nshots, shot = (int)blockIdx.y + (int)(blockIdx.x >> 3) - q * pr.nshots;
+    const PlaneTile pt = plane_tile(a.ztiles, a.nplanes, a.run, q * 8 + (int)(blockIdx.x & 7));
     if (pt.plane < 0) return;
     const int other = pt.plane;
     const int p = tid % G::P, jj = tid / G::P;
@@ -683,7 +687,7 @@ __global__ __launch_bounds__(G::T) void k2_cfft_strided(CStridedArgs a)
     __shared__ float2 lds[G::P * G::PS];
     __shared__ float2 tws[G::TWN];
     const int tid = threadIdx.x, shot = blockIdx.y;
-    const PlaneTile pt = plane_tile(a.ztiles, a.nplanes, a.run);
+    const PlaneTile pt = plane_tile(a.ztiles, a.nplanes, a.run, blockIdx.x);
     if (pt.plane < 0) return;
     const int other = pt.plane;
     const int p = tid % G::P, jj = tid / G::P;
@@ -793,7 +797,7 @@ __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(QVTI_XPASS
     __shared__ float2 lds[G::P * G::PS];
     __shared__ float2 tws[G::TWN];
     const int tid = threadIdx.x, shot = blockIdx.y;
-    const PlaneTile pt = plane_tile(a.ztiles, a.ny, a.run);
+    const PlaneTile pt = plane_tile(a.ztiles, a.ny, a.run, blockIdx.x);
     if (pt.plane < 0) return;
     const int iy = pt.plane;
     const int p = tid % G::P, jj = tid / G::P;

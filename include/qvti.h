@@ -246,8 +246,9 @@ int qvti_tile_choice(qvti_ctx *c, int max_classes, int *pencils, int *split);
  *    taper_ratio in [0, 1]).
  *  vref = 0 and fcut = 0: both off.
  * Takes effect at the next qvti_begin; a run in progress must be begun
- * again, as after qvti_set_snapshot.  The first call that switches it on allocates 6 more fields per
- * shot; each step then runs three more complex 3-D inverse transforms. */
+ * again, as after qvti_set_snapshot.  The first call that switches it on allocates 12 more fields per
+ * shot (three complex spectra and the six real fields they become); each step
+ * then runs three more complex 3-D inverse transforms. */
 int qvti_set_kspace(qvti_ctx *c, float vref, float fcut, float vmax, float taper_ratio);
 /* Two-level FFT split of each axis (0: the default N1 x N2 of the length;
  * 1: an alternative for lengths 64 96 100 128 160 200 256 400).  The split

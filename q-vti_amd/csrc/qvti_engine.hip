@@ -291,8 +291,10 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
     // When a z row does not end on a 128-byte line, neighbouring row tiles
     // and neighbouring planes share lines (and 64-cell blocks): run 8 row
     // tiles and 2 planes per XCD so those are fetched once.  Measured at
-    // 400x400x200 (800-byte rows): str_z 2472 -> 2380 us, str_x 1066 ->
-    // 1036 us; at 256^3 (aligned rows) one tile and one plane per XCD is best.
+    // 400x400x200 (800-byte rows), when five fields per component went through
+    // them: str_z 2472 -> 2380 us, str_x 1066 -> 1036 us (1365 us and, with the
+    // y-derivatives, 1790 us since); at 256^3 (aligned rows) one tile and one
+    // plane per XCD is best.
     if ((g->nz * 4) % 128 != 0) {
         c->run_rows = 8;
         c->run_planes = 2;

@@ -328,10 +328,11 @@ struct StressXYPair {
 
 // NT: non-temporal field loads and stores (stream_nt)
 template <class G, bool NT>
-// What bounds it at 256^3: 26 floats per cell (each sum reads S-bar) in 370 us
-// along x, 4.7 TB/s, with the VALU busy for about half of that time; 2, 3 and
-// 4 waves per SIMD measure the same there (370-375 us), at 400x400x200 3 waves
-// are best (985 us; 1045 us with 2), hence the bounds.
+// What bounds it: 52 floats per cell for both axes (each sum reads S-bar).
+// 256^3: 687 us, 5.1 TB/s, the rate of the memory at 20 streams; 400x400x200:
+// 1790 us, 3.7 TB/s, 3 waves per SIMD and rows that end mid-line.  The bounds:
+// one axis at 256^3, before the streaming, took 370-375 us with 2, 3 and 4
+// waves per SIMD; at 400x400x200 3 waves were best (985 us; 1045 us with 2).
 __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(G::NMAX <= 16 ? 4 : 3)))
 void k2_stress_xy(StressXYPair pr)
 {
@@ -449,8 +450,8 @@ void k2_stress_xy(StressXYPair pr)
 // Two workgroups per tile (grid y): vx and vy with P0 and P2, and vz with P1.
 // They share nothing but the twiddles, and the chain of dependent transforms,
 // which bounds the kernel where a grid has few tiles, is a third shorter:
-// 64^3 20 -> 15 us, 160x160x128 78 -> 73 us, 256^3 349 -> 345 us (5.2 TB/s),
-// 400x400x200 751 -> 738 us.
+// 64^3 20 -> 15 us, 160x160x128 78 -> 73 us, 256^3 349 -> 343 us (27 floats per
+// cell, 5.3 TB/s: the memory bounds it there), 400x400x200 751 -> 738 us.
 // dv is the change since the previous step's pre-injection velocity (the
 // reference's V - V_prev, cuviscoelas_3D.cu:517-522, 1124-1131, without 1/dt).
 // Tile: G::P rows (z-pencils).
@@ -1081,11 +1082,14 @@ struct StressZArgs {
 // transform levels take one pass: 6 R NMAX <= T).
 //  * rows that end on a 128-byte line: T = 192 or 256, whichever leaves fewer
 //    threads idle in the transforms (256 = 16 x 16: 12 pencils on 192 threads;
-//    at 256^3 1001 us against 1081 us on 384 and 1269 us on 512 threads: more,
-//    smaller workgroups overlap their load and transform phases better);
+//    at 256^3 1001 us against 1081 us on 384 and 1269 us on 512 threads (646
+//    us since the shear sums left it and with streaming): more, smaller
+//    workgroups overlap their load and transform phases better; 384 threads at
+//    n = 128: 109 us against 91 us at 128^3);
 //  * long rows that end mid-line share their last line and 64-cell block with
 //    the next tile, so fewer, larger tiles: T = 512 (400x400x200: 4 rows,
-//    1980 us, against 2211 us with 2 rows on 256 threads).
+//    1980 us, against 2211 us with 2 rows on 256 threads; 1365 us since the
+//    shear sums left it).
 template <class G>
 struct StressTile {
     static constexpr int R256 = 256 / (6 * G::NMAX), R192 = 192 / (6 * G::NMAX);
@@ -1100,7 +1104,8 @@ struct StressTile {
 // (c = 2: D+, else D-)
 // NT (stream_nt): 1 loads the derivatives non-temporally, 2 (one shot) the
 // coefficients and stresses as well - with several shots the coefficients are
-// read again for the next shot of the tile.  256^3: 714 -> 657 us (2), 32
+// read again for the next shot of the tile.  49 floats per cell bound it: 256^3
+// 714 -> 657 us (2; 646 us, 5.1 TB/s, with the early loads below), 32
 // shots of 160x160x128: 4234 -> 4192 us (1; 4260 with 2).
 template <class G, bool VTI, int NT>
 __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_eu(QVTI_STRESSZ_WAVES))) void k2_stress_z(

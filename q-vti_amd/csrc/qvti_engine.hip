@@ -285,9 +285,12 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
         c->snap_hi[a] = dims[a] - g->pml;
     }
     c->nrows = (long long)g->nx * g->ny;
-    // 1 / |k| of five times the dominant frequency at 3000 m/s, as a power of
-    // two: A3 v = L |k| v stays below v, with which it shares a transform
-    c->L = exp2(round(log2(3000.0 / (5.0 * 2.0 * M_PI * (double)g->f0))));
+    // 1 / |k| at the Nyquist wavenumber of the finest axis, as a power of two:
+    // A3 v = L |k| v stays below v, with which it shares a transform, in any
+    // medium.  (Set from a frequency and 3000 m/s, a 300 m/s medium's A3 v was
+    // ten times v.)  The rounding of v in A3 v enters the stresses times
+    // gamma * cells per wavelength / 2.
+    c->L = exp2(round(log2(std::min({(double)g->dx, (double)g->dy, (double)g->dz}) / M_PI)));
     // When a z row does not end on a 128-byte line, neighbouring row tiles
     // and neighbouring planes share lines (and 64-cell blocks): run 8 row
     // tiles and 2 planes per XCD so those are fetched once.  Measured at

@@ -56,6 +56,30 @@ def test_stress_family_matches_the_oracle(nx, ny, nz, vti, media, ratio):
     assert rel_l2(st[3:], ref["state"][3:]) < TOL
 
 
+@pytest.mark.parametrize("scale", [0.05, 1.0, 20.0])
+def test_field_scales_suit_slow_and_fast_media(scale):
+    """v shares a complex transform with L |k| v; in a slow medium on a fine
+    grid, and in a fast one on a coarse grid, its rounding must stay that of
+    plain FP32: within twice the FP32 oracle's own distance to FP64."""
+    shot, model = small_case(48, 36, 40, 4, 20, O.SRC_FX, True, seed=3)
+    for k in ("dx", "dy", "dz"):
+        shot[k] = float(np.float32(shot[k] * scale))
+    shot["dt"] = float(np.float32(shot["dt"] * min(scale, 1.0)))
+    model = dict(model, vp=model["vp"] * np.float32(scale), vs=model["vs"] * np.float32(scale))
+    ref = O.run(shot, model, "f64", state=True)["state"]
+    floor = rel_l2(O.run(shot, model, "f32", state=True)["state"], ref)
+    with qvti.Engine(48, 36, 40, shot["pml"], shot["dx"], shot["dy"], shot["dz"], shot["dt"], shot["f0"], shot["w0"],
+                     vti=True) as e:
+        e.set_model_dict(model)
+        e.begin(shot["nt"], shot["rik"], [qvti.make_shot(shot["src_kind"], (shot["sx"], shot["sy"], shot["sz"]),
+                                                         shot["rx"], shot["ry"], shot["rz"])])
+        e.step(shot["nt"])
+        e.finish()
+        err = rel_l2(e.state(), ref)
+    print("scale %g: state vs FP64 oracle %.2e, FP32 oracle %.2e" % (scale, err, floor))
+    assert err < 2 * floor
+
+
 # strided lengths next to row lengths that leave a partial last tile at every
 # tile width, and every pencil count per workgroup (8 to 64 columns)
 STRIDED = [(16, 24, 18), (64, 18, 50), (18, 90, 30), (128, 16, 54), (20, 200, 18), (250, 16, 20), (16, 400, 36),

@@ -108,12 +108,12 @@ static __global__ __launch_bounds__(256) void k_probe(const float* f, long long 
 //   o0 A1 v + o3 A1 dv = (o0 / alpha) A1 w,
 //   o1 v + o4 dv       = (o1 - o4 / kappa) v + (o4 / (alpha kappa)) w,
 // o4 / kappa = -M g^2: four terms per moduli set instead of five, exactly,
-// and A1 acts on w alone.  alpha and the length scale L of A1 = 1/(L |k|) and
-// A3 = L |k| are powers of two (they only shift exponents) that keep w below v
-// up to five times the dominant frequency and A3 v at every wavenumber: v,
-// whose coefficient is the largest by far, then takes no rounding from the
-// field that shares a complex transform with it, and the others' coefficients
-// are of order g.
+// and A1 acts on w alone.  alpha (qvti_set_model) and the length scale L of
+// A1 = 1/(L |k|) and A3 = L |k| (qvti_create) are powers of two (they only
+// shift exponents) that keep w and A3 v within a few times v at every
+// frequency and wavenumber: v, whose coefficient is the largest by far, then
+// takes little rounding from the field that shares a complex transform with
+// it, and the others' coefficients are of order g.
 //   o[0] = L o0 / alpha (A1 w), o[1] = M (1 + g^2) (v),
 //   o[2] = o2 / L (A3 v),       o[3] = -M g^2 / alpha (w)
 // o2 and o3 follow from o0, o1 and one field r = alpha / (rho w0^2 L^2):

@@ -666,25 +666,31 @@ extern "C" int qvti_set_model(qvti_ctx* c, const float* velp, const float* gama_
     float* tmp = c->bufA;
     const int nin = c->g.vti ? 7 : 5;
     const float* srcs[7] = {velp, gama_p, vels, gama_s, rho, eps, delta};
-    // w = alpha (v + kappa dv), kappa dv being pi f / f_ref times v at the
-    // frequency f (w0 = 2 pi f_ref).  alpha scales w to the size of v at 5 f0,
-    // the top of a pulse's spectrum: in the transforms that carry both, the
-    // rounding of w then stays below that of v, and w itself enters the
-    // stresses with the small Q coefficients only (measured, 160x160x128,
-    // k-space mode, records against FP64: 3.2e-7 with alpha set at f0)
+    // w = alpha (v + kappa dv).  alpha scales w to the size of v at the angular
+    // frequency 1 / (2 dt), where |dv| = |v| / 2: a stable run has |dv| <= 2 |v|,
+    // so |w| stays below about 5 |v| whatever the wavelet and f0 are (f0 only
+    // shapes the C-PML), and wz, which shares a transform with vz, cannot swamp
+    // it.  The rounding of vz in wz grows with 1 / alpha, but enters with the
+    // small Q coefficients.  Measured, state against FP64, 96x80x64, 160 steps,
+    // scaled at 5 f0 / at omega dt = 1 / at 1/2 / at 1/4:
+    //   k-space mode, f0 = 1 Hz, 80 Hz wavelet  10.8e-6 / 4.9e-6 / 4.9e-6 / 5.1e-6
+    //   k-space mode, f0 = wavelet = 20 Hz       2.0e-6 / 2.0e-6 / 2.0e-6 / 2.0e-6
+    //   the same, 8 times the wavelet            6.2e-6 / 6.2e-6 / 6.2e-6 / 6.4e-6
+    //   f0 = wavelet = 20 Hz, Q 2-15             0.7e-6 / 1.0e-6 / 0.8e-6 / 0.7e-6
+    // (five fields per component, dv itself beside v: 4.9, 2.0, 6.2, 1.0e-6).
     c->kappa = c->media == QVTI_MEDIA_DISPERSION || c->media == QVTI_MEDIA_LOSSLESS
                    ? 0.0
                    : -kRefPi / ((double)c->g.w0 * (double)c->g.dt);
     if (c->media == QVTI_MEDIA_QCOMP) c->kappa = -c->kappa;
-    const double tilt = c->kappa == 0.0 ? 0.0 : 5.0 * 2.0 * M_PI * M_PI * (double)c->g.f0 / (double)c->g.w0;
+    const double tilt = 0.5 * c->kappa;
     c->alpha = exp2(-round(log2(sqrt(1.0 + tilt * tilt))));
     const float wab[3] = {(float)c->alpha, (float)(c->alpha * c->kappa), c->media == QVTI_MEDIA_DISPERSION ? 0.f : 1.f};
     int rc = QVTI_OK;
-    if (hipMemcpyAsync(c->d_wab, wab, sizeof wab, hipMemcpyHostToDevice, c->stream) != hipSuccess)
-        rc = qvti_fail(QVTI_E_DEVICE, "model upload failed");
     for (int k = 0; k < nin && !rc; ++k)
         if (hipMemcpyAsync(tmp + k * N, srcs[k], B, hipMemcpyHostToDevice, c->stream) != hipSuccess)
             rc = qvti_fail(QVTI_E_DEVICE, "model upload failed");
+    if (!rc && hipMemcpyAsync(c->d_wab, wab, sizeof wab, hipMemcpyHostToDevice, c->stream) != hipSuccess)
+        rc = qvti_fail(QVTI_E_DEVICE, "model upload failed");
     if (!rc) {
         CoefArgs ca;
         ca.N = N;

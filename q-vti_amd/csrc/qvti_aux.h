@@ -116,12 +116,12 @@ static __global__ __launch_bounds__(256) void k_probe(const float* f, long long 
 // it, and the others' coefficients are of order g.
 //   o[0] = L o0 / alpha (A1 w), o[1] = M (1 + g^2) (v),
 //   o[2] = o2 / L (A3 v),       o[3] = -M g^2 / alpha (w)
-// o2 and o3 follow from o0, o1 and one field r = alpha / (rho w0^2 L^2):
-//   o3 = -o0^2 r,  o2 = -o0 r M,  M = o1 + alpha o3
-// (set_coeffs).  The stress update forms them per cell in FP32, so that it
-// reads 13 coefficient fields instead of 20 (VTI; 9 instead of 12 isotropic).
-// Their rounding (about 2^-23 relative) enters the stresses times g, of order
-// 1e-2, so below that of o1 v.
+// The sets P, H and D share rho and g, so the stress update reads c of each
+// set, g, rho and forms the four in FP64 per cell, each rounded once
+// (set_coeffs): 9 fields instead of 16 (VTI; 6 instead of 8 isotropic).  c is
+// held as an FP32 value and 16 bits more, exact to 2^-40, so that the four are
+// rounded as from the FP64 c but for about one in 30000, which lies that close
+// to a rounding boundary (with 8 bits it was one in 150).
 // media (qvti_set_media, the reference's media_type, viscoelas_3D.cpp:57-60):
 // 0 viscoelastic (as above); 1 dispersion only (tau terms dropped: kappa = 0,
 // w = v, no fourth term); 2 lossless (gamma = 0); 3 Q-compensating (tau terms
@@ -140,16 +140,24 @@ __device__ __forceinline__ void q_coeffs(double rho, double v, double g, double 
     o[3] = -Mg2 / alpha;
 }
 
-// The four coefficients of one moduli set in the stress update from its
-// stored o0, o1 and the cell's r; s4 = 0 where the medium has no tau terms
-// (dispersion only), else 1.
-__device__ __forceinline__ void set_coeffs(float (&o)[kFam], float o0, float o1, float r, float alpha, float s4)
+// c as an FP32 value and 16 signed bits: c = hi (1 + low 2^-39)
+__device__ __forceinline__ int low_bits(double c, float hi)
 {
-    const float t = o0 * r;
-    o[0] = o0;
-    o[1] = o1;
-    o[3] = -s4 * (o0 * t);
-    o[2] = -t * (o1 + alpha * o[3]);
+    const double x = rint((c - (double)hi) / (double)hi * 0x1p39);
+    return fabs(x) <= 32768.0 ? (int)fmin(x, 32767.0) : 0;  // (0 or not finite: no low bits)
+}
+
+// The four coefficients of one moduli set in the stress update (q_coeffs).
+__device__ __forceinline__ void set_coeffs(float (&o)[kFam], float hi, int low, double g, double rho,
+                                           const MediumConst& k)
+{
+    const double h = hi;
+    const double c = fma(h * 0x1p-39, (double)low, h);
+    const double rc = rho * c, M = rc * c, Mg = M * g, Mg2 = Mg * g;
+    o[0] = (float)(rc * g * k.k0);
+    o[1] = (float)fma(Mg2, k.s4, M);
+    o[2] = (float)(Mg * c * k.k2);
+    o[3] = (float)(Mg2 * k.k3);
 }
 
 // (blocked field groups and coefficient group sizes: qvti_layout.h)
@@ -159,37 +167,43 @@ struct CoefArgs {
     int vti, media;
     double w0, alpha, L;
     const float *vp, *gp, *vs, *gs, *rho, *eps, *del;
-    float* g1;  // blocked [N/64][kG1][64]
-    float* g2;  // blocked [N/64][kG2][64] (VTI only)
-    float* s;   // [kFam][N]: the S set, averaged by k_averages
+    float* gm;   // blocked [N/64][kGM][64]
+    float* low;  // [N]: low bits of H and D (VTI only)
+    float* s;    // [kFam][N]: the coefficients of the set S, averaged by k_averages
 };
 
 static __global__ __launch_bounds__(256) void k_coefficients(CoefArgs a)
 {
     for (long long ip = (long long)blockIdx.x * 256 + threadIdx.x; ip < a.N; ip += (long long)gridDim.x * 256) {
-        double o[kFam];
-        const double r = a.rho[ip];
-        q_coeffs(r, a.vp[ip], a.gp[ip], a.w0, a.alpha, a.L, a.media, o);
-        for (int j = 0; j < 2; ++j) a.g1[blk_index(ip, kG1, j)] = (float)o[j];
-        q_coeffs(r, a.vs[ip], a.gs[ip], a.w0, a.alpha, a.L, a.media, o);
-        for (int j = 0; j < 2; ++j) a.g1[blk_index(ip, kG1, 2 + j)] = (float)o[j];
-        for (int j = 0; j < kFam; ++j) a.s[j * a.N + ip] = (float)o[j];
-        // (rho = 0: every coefficient is 0)
-        a.g1[blk_index(ip, kG1, 4)] = r != 0.0 ? (float)(a.alpha / (r * (a.w0 * a.w0) * (a.L * a.L))) : 0.f;
+        const double r = a.rho[ip], half_pi = 3.1415926 / 2.0;
+        const float gp = a.media == 2 ? 0.f : a.gp[ip], gs = a.media == 2 ? 0.f : a.gs[ip];
+        const int nf = kGM(a.vti);
+        auto put = [&](int f, float v) { a.gm[blk_index(ip, nf, f)] = v; };
+        const double cosp = cos((double)gp * half_pi), coss = cos((double)gs * half_pi);
+        // two speeds and the word of their low bits
+        auto speeds = [&](int f0, double c0, int f1, double c1) {
+            put(f0, (float)c0);
+            put(f1, (float)c1);
+            return __int_as_float((low_bits(c0, (float)c0) & 0xffff) | (low_bits(c1, (float)c1) << 16));
+        };
+        put(GM_LOW, speeds(GM_CP, a.vp[ip] * cosp, GM_CS, a.vs[ip] * coss));
         if (a.vti) {
             const double e = a.eps[ip], dl = a.del[ip], vp = a.vp[ip], vs = a.vs[ip];
             const double vh = e == 0.0 ? vp : vp * sqrt(1.0 + 2.0 * e);
-            q_coeffs(r, vh, a.gp[ip], a.w0, a.alpha, a.L, a.media, o);
-            for (int j = 0; j < 2; ++j) a.g2[blk_index(ip, kG2, j)] = (float)o[j];
             double vd = vp;
             if (dl != 0.0) {
                 const double c33 = r * vp * vp, c44 = r * vs * vs;
                 const double prod = (c33 - c44) * (c33 * (1.0 + 2.0 * dl) - c44);
                 vd = sqrt((sqrt(prod > 0.0 ? prod : 0.0) + c44) / r);
             }
-            q_coeffs(r, vd, a.gp[ip], a.w0, a.alpha, a.L, a.media, o);
-            for (int j = 0; j < 2; ++j) a.g2[blk_index(ip, kG2, 2 + j)] = (float)o[j];
+            a.low[ip] = speeds(GM_CH, vh * cosp, GM_CD, vd * cosp);
         }
+        put(GM_GP, gp);
+        put(GM_GS, gs);
+        put(GM_RHO, a.rho[ip]);
+        double o[kFam];
+        q_coeffs(r, a.vs[ip], a.gs[ip], a.w0, a.alpha, a.L, a.media, o);
+        for (int j = 0; j < kFam; ++j) a.s[j * a.N + ip] = (float)o[j];
     }
 }
 
@@ -200,7 +214,7 @@ struct AvgArgs {
     long long sx, sy, N;
     float dt;
     const float* s;  // [kFam][N]: the S set
-    float* gs;       // [kGS][N]: S-bar
+    float* gs;       // [kFam][N]: S-bar
     const float* rho;
     float* buoy;     // [3][N]
 };

@@ -38,13 +38,13 @@ struct qvti_ctx {
     const LenOps* ops[3] = {nullptr, nullptr, nullptr};  // kernels of the x, y, z lengths
     int split[3] = {0, 0, 0};                            // their split variants (len_ops)
     // model
-    float* coef = nullptr;  // blocked coefficient groups G1 (5 fields), GS (4), G2 (4, VTI)
+    float* coef = nullptr;  // medium fields (a blocked group of kGM, then kGS in natural order)
     float* buoy = nullptr;  // [3][N]
     bool has_model = false;
     int media = 0;  // QVTI_MEDIA_*: applied by the next qvti_set_model
     double alpha = 1.0, kappa = 0.0;  // w = alpha (v + kappa dv) of the current model's medium (q_coeffs)
     double L = 1.0;                   // length scale of A1 and A3
-    float* d_wab = nullptr;           // {alpha, alpha kappa, s4 (set_coeffs)} on the device
+    MediumConst* d_med = nullptr;     // constants of the current model's medium
     // state, field-major [field][shot][N]
     float *v = nullptr, *sig = nullptr, *w = nullptr, *H = nullptr, *bufA = nullptr, *bufB = nullptr;
     float *phiv[3] = {nullptr, nullptr, nullptr}, *phis[3] = {nullptr, nullptr, nullptr};

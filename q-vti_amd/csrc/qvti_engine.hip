@@ -203,7 +203,7 @@ extern "C" long long qvti_estimate_bytes(const qvti_grid* g, int max_shots)
     const long long N = (long long)g->nx * g->ny * g->nz;
     const long long p2 = 2LL * g->pml;
     const long long slabs = 8LL * (p2 * g->ny * g->nz + (long long)g->nx * p2 * g->nz) + 7LL * g->nx * g->ny * p2;
-    const long long model = kG1 + kGS + (g->vti ? kG2 : 0) + 3;
+    const long long model = kGM(g->vti) + kGS(g->vti) + 3;
     return 4LL * (N * (state_fields() * max_shots + model) + slabs * max_shots) + (64LL << 20);
 }
 
@@ -336,7 +336,7 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
     c->slab[1] = (long long)g->nx * p2 * g->nz;
     c->slab[2] = (long long)g->nx * g->ny * p2;
     const long long Nb = c->Nb;
-    rc = rc ? rc : dalloc(c, (void**)&c->coef, sizeof(float) * (kG1 + kGS + (g->vti ? kG2 : 0)) * Nb);
+    rc = rc ? rc : dalloc(c, (void**)&c->coef, sizeof(float) * (kGM(g->vti) + kGS(g->vti)) * Nb);
     rc = rc ? rc : dalloc(c, (void**)&c->buoy, sizeof(float) * 3 * N);
     rc = rc ? rc : dalloc(c, (void**)&c->v, sizeof(float) * 3 * S * N);
     rc = rc ? rc : dalloc(c, (void**)&c->sig, sizeof(float) * 6 * S * N);
@@ -349,7 +349,7 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
         rc = rc ? rc : dalloc(c, (void**)&c->phis[a], sizeof(float) * c->nphis[a] * S * c->slab[a]);
     }
     rc = rc ? rc : dalloc(c, (void**)&c->d_it, sizeof(int));
-    rc = rc ? rc : dalloc(c, (void**)&c->d_wab, 3 * sizeof(float));
+    rc = rc ? rc : dalloc(c, (void**)&c->d_med, sizeof(MediumConst));
     rc = rc ? rc : dalloc(c, (void**)&c->d_probe, sizeof(int));
     rc = rc ? rc : dalloc(c, (void**)&c->d_src_kind, sizeof(int) * S);
     rc = rc ? rc : dalloc(c, (void**)&c->d_src_ip, sizeof(long long) * S);
@@ -464,7 +464,7 @@ static int build_launch_config(qvti_ctx* c)
         vz.buoy[k] = c->buoy + (long long)k * N;
         vz.phi[k] = c->phiv[2] + (long long)k * c->S * c->slab[2];
     }
-    vz.wab = c->d_wab;
+    vz.med = c->d_med;
     vz.src_kind = c->d_src_kind;
     vz.src_ip = c->d_src_ip;
     vz.rik = nullptr;  // set at begin
@@ -577,7 +577,7 @@ static int build_launch_config(qvti_ctx* c)
         a.tw = c->ax[axis].tw;
         a.sym[0] = c->ax[axis].dp;
         a.sym[1] = c->ax[axis].dm;
-        a.gs = c->coef + (long long)kG1 * c->Nb;
+        a.gs = c->coef + (long long)kGM(g.vti) * c->Nb;
         a.N = N;
         a.out = out;
         a.blk_stride = c->Nb;
@@ -616,11 +616,10 @@ static int build_launch_config(qvti_ctx* c)
     sz.dxb = c->bufA;
     sz.blk_stride = c->Nb;
     sz.dyb = c->bufB;
-    sz.g1 = c->coef;
-    sz.gs = c->coef + (long long)kG1 * c->Nb;
-    sz.g2 = g.vti ? c->coef + (long long)(kG1 + kGS) * c->Nb : nullptr;
+    sz.gm = c->coef;
+    sz.gs = c->coef + (long long)kGM(g.vti) * c->Nb;
     sz.N = N;
-    sz.wab = c->d_wab;
+    sz.med = c->d_med;
     for (int k = 0; k < 6; ++k) sz.sig[k] = sg[k];
     for (int k = 0; k < 3; ++k) sz.vel[k] = vv[k];
     for (int k = 0; k < 5; ++k) {
@@ -684,26 +683,28 @@ extern "C" int qvti_set_model(qvti_ctx* c, const float* velp, const float* gama_
     if (c->media == QVTI_MEDIA_QCOMP) c->kappa = -c->kappa;
     const double tilt = 0.5 * c->kappa;
     c->alpha = exp2(-round(log2(sqrt(1.0 + tilt * tilt))));
-    const float wab[3] = {(float)c->alpha, (float)(c->alpha * c->kappa), c->media == QVTI_MEDIA_DISPERSION ? 0.f : 1.f};
+    const double w0 = (double)c->g.w0, s4 = c->media == QVTI_MEDIA_DISPERSION ? 0.0 : 1.0;
+    const MediumConst med = {-w0 * (c->L / c->alpha), 1.0 / (w0 * c->L), -s4 / c->alpha, s4,
+                             (float)c->alpha, (float)(c->alpha * c->kappa)};
     int rc = QVTI_OK;
     for (int k = 0; k < nin && !rc; ++k)
         if (hipMemcpyAsync(tmp + k * N, srcs[k], B, hipMemcpyHostToDevice, c->stream) != hipSuccess)
             rc = qvti_fail(QVTI_E_DEVICE, "model upload failed");
-    if (!rc && hipMemcpyAsync(c->d_wab, wab, sizeof wab, hipMemcpyHostToDevice, c->stream) != hipSuccess)
+    if (!rc && hipMemcpyAsync(c->d_med, &med, sizeof med, hipMemcpyHostToDevice, c->stream) != hipSuccess)
         rc = qvti_fail(QVTI_E_DEVICE, "model upload failed");
     if (!rc) {
         CoefArgs ca;
         ca.N = N;
         ca.vti = c->g.vti;
         ca.media = c->media;
-        ca.w0 = (double)c->g.w0;
+        ca.w0 = w0;
         ca.alpha = c->alpha;
         ca.L = c->L;
         ca.vp = tmp; ca.gp = tmp + N; ca.vs = tmp + 2 * N; ca.gs = tmp + 3 * N; ca.rho = tmp + 4 * N;
         ca.eps = c->g.vti ? tmp + 5 * N : nullptr;
         ca.del = c->g.vti ? tmp + 6 * N : nullptr;
-        ca.g1 = c->coef;
-        ca.g2 = c->g.vti ? c->coef + (long long)(kG1 + kGS) * c->Nb : nullptr;
+        ca.gm = c->coef;
+        ca.low = c->coef + (long long)kGM(c->g.vti) * c->Nb + kFam * N;
         ca.s = c->bufB;  // kFam fields, free after the averages
         const unsigned nb = (unsigned)std::min<long long>((N + kThreads - 1) / kThreads, 65535LL * 4);
         hipLaunchKernelGGL(k_coefficients, dim3(nb), dim3(kThreads), 0, c->stream, ca);
@@ -712,7 +713,7 @@ extern "C" int qvti_set_model(qvti_ctx* c, const float* velp, const float* gama_
         aa.sx = (long long)c->g.ny * c->g.nz; aa.sy = c->g.nz; aa.N = N;
         aa.dt = c->g.dt;
         aa.s = ca.s;
-        aa.gs = c->coef + (long long)kG1 * c->Nb;
+        aa.gs = c->coef + (long long)kGM(c->g.vti) * c->Nb;
         aa.rho = tmp + 4 * N;
         aa.buoy = c->buoy;
         hipLaunchKernelGGL(k_averages, dim3(nb), dim3(kThreads), 0, c->stream, aa);
@@ -1817,7 +1818,7 @@ extern "C" int qvti_kernel_bytes(qvti_ctx* c, int max_classes, double* bytes)
     const double N = (double)c->N * std::max(1, c->nshots), f = 4.0 * N;
     const double slab = (double)std::max(1, c->nshots) * 4.0;
     const double sx = c->slab[0] * slab, sy = c->slab[1] * slab, sz = c->slab[2] * slab;
-    const int ncoef = kG1 + kGS + (c->g.vti ? kG2 : 0);
+    const int ncoef = kGM(c->g.vti) + kGS(c->g.vti);
     double b[KC_COUNT] = {};
     b[KC_TICK] = 8;
     b[KC_VEL_X] = 6 * f + 3 * 2 * sx;
@@ -1829,7 +1830,7 @@ extern "C" int qvti_kernel_bytes(qvti_ctx* c, int max_classes, double* bytes)
     b[KC_XPASS] = 6 * f + (c->ks ? 14 : 8) * f;
     b[KC_Y_INV] = (c->ks ? 28 : 16) * f;
     b[KC_Z_INV] = c->ks ? 14 * f + 12 * f : 8 * f + 6 * f;
-    b[KC_STR_X] = b[KC_STR_Y] = (3 * kFam + kDer) * f + kGS * 4.0 * c->N;
+    b[KC_STR_X] = b[KC_STR_Y] = (3 * kFam + kDer) * f + kFam * 4.0 * c->N;
     b[KC_STR_Z] = (12 + 2 * kDer + 12) * f + ncoef * 4.0 * c->N + 2 * (5 * sx + 5 * sy + 4 * sz);
     b[KC_Z_INV] += 6.0 * 4 * c->total_rec;  // receivers
     if (merged_xy(c)) {  // both axes in the launch of class x

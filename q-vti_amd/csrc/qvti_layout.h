@@ -23,10 +23,20 @@ __host__ __device__ __forceinline__ long long blk_index(long long ip, int nf, in
 // A2 w} whose derivatives the stress update weighs with the Q coefficients
 // (k_coefficients in qvti_aux.h).
 constexpr int kFam = 4;
-// coefficient groups: G1 = {P: o0, o1; S: o0, o1; r}, the 8-corner averages GS
-// = {S-bar: o0..o3}, G2 = {H: o0, o1; D: o0, o1} (VTI).  The stress update
-// derives o2 and o3 of the sets P, S, H and D (set_coeffs in qvti_aux.h).
-constexpr int kG1 = 5, kGS = kFam, kG2 = 4;
+// Medium fields from which the stress update forms the coefficients of the
+// moduli sets P, S, H and D (set_coeffs in qvti_aux.h): the speeds c = v
+// cos(pi g/2), the low bits of two of them, the gammas and the density in one
+// blocked group per cell (the last two: VTI); in natural order the four
+// coefficients of S-bar (8-corner averages) and, VTI, the low bits of the other
+// two speeds (a ninth field in the group would pass 4 GiB at 512^3).
+enum { GM_CP, GM_CS, GM_LOW, GM_GP, GM_GS, GM_RHO, GM_CH, GM_CD };
+constexpr int kGM(bool vti) { return vti ? 8 : 6; }
+constexpr int kGS(bool vti) { return vti ? kFam + 1 : kFam; }
+// constants of the medium and the run (q_coeffs), on the device
+struct MediumConst {
+    double k0, k2, k3, s4;
+    float wa, wb;  // alpha, alpha kappa
+};
 // x- (y-) derivatives that the stress update reads: the four of the family
 // whose component is the axis, and the two S-bar-weighted shear sums
 constexpr int kDer = kFam + 2;
@@ -37,7 +47,7 @@ constexpr int kDer = kFam + 2;
 // (global_load v, v, s[:]; imm, a compile-time byte offset, rides along).  Without it the compiler folds the lane offset into
 // the base and keeps a 64-bit address register pair, made by a 64-bit add, for
 // every row.  Offsets stay below 4 GiB: within one shot's field (512^3
-// floats) or blocked group of kDer fields.
+// floats) or blocked group of at most 8 fields.
 typedef __attribute__((address_space(1))) char gchar;
 typedef float vfloat2 __attribute__((ext_vector_type(2)));
 struct Row {

@@ -48,12 +48,14 @@ constexpr int kThreads = 256;
 #define QVTI_XPASS_WAVES 1
 #endif
 // minimum waves per SIMD the z-row kernels are compiled for (1: no bound on
-// their registers; 4 caps them at 128 VGPRs, the occupancy their LDS allows)
+// their registers; 4 caps them at 128 VGPRs, the occupancy their LDS allows;
+// the stress update takes 137 without at n = 160, 192, 288 and 320, none of its
+// lengths spills with: 160^3 188 -> 174 us, 192^3 287 -> 269 us)
 #ifndef QVTI_VELZ_WAVES
 #define QVTI_VELZ_WAVES 1
 #endif
 #ifndef QVTI_STRESSZ_WAVES
-#define QVTI_STRESSZ_WAVES 1
+#define QVTI_STRESSZ_WAVES 4
 #endif
 enum { MODE_STORE = 0, MODE_VEL = 1 };
 
@@ -312,7 +314,7 @@ struct StressXYArgs {
     long long shot_stride;
     const float2* tw;
     const float2* sym[2];
-    const float* gs;  // S-bar coefficients [kGS][N]
+    const float* gs;  // S-bar coefficients [kFam][N]
     long long N;
     float* out;       // blocked group [shot][N/64][kDer][64]
     // per-shot length of a blocked group's field: N rounded up to whole 64-cell blocks
@@ -468,7 +470,7 @@ struct VelZArgs {
     const float *accx[3], *accy[3];  // x and y derivatives (+ phi)
     float* v[3];
     float* w[3];
-    const float* wab;  // {alpha, alpha kappa}
+    const MediumConst* med;
     float2* P[3];
     const float* buoy[3];
     float* phi[3];  // z-slab: phi_pxz_z (node), phi_pyz_z (node), phi_pzz_z (half)
@@ -600,7 +602,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(QVTI_V
     const int kind = a.src_kind[shot];
     const long long sip = a.src_ip[shot];
     const float sprev = it > 0 ? a.rik[it - 1] : 0.f;
-    const float wa = a.wab[0], wb = a.wab[1];
+    const float wa = a.med->wa, wb = a.med->wb;
     const int ix = (int)(r1 / a.ny), iy = (int)(r1 - (long long)ix * a.ny);
     const bool rowdom = ok1 && ix < a.nx - 1 && iy < a.ny - 1;
     const unsigned slab_row = ok1 ? (unsigned)(r1 * 2 * a.pml) * 4u : 0u;
@@ -1064,10 +1066,9 @@ struct StressZArgs {
     //   dyb: ey 0-3 (dy vy-family), sum_j S-bar_j dy of the vz family 4, of the vx family 5
     const float *dxb, *dyb;
     long long blk_stride;  // per-shot field length of the blocked groups (N rounded up to 64)
-    // coefficient groups G1, GS and G2 (VTI; else null)
-    const float *g1, *gs, *g2;
+    const float *gm, *gs;  // medium fields: the blocked group; in natural order
     long long N;
-    const float* wab;  // {alpha, alpha kappa, s4}
+    const MediumConst* med;
     float* sig[6];  // pxx pyy pzz pxy pxz pyz
     float* phx[5];
     float* phy[5];
@@ -1105,8 +1106,9 @@ struct StressTile {
 // NT (stream_nt): 1 loads the derivatives non-temporally, 2 (one shot) the
 // coefficients and stresses as well - with several shots the coefficients are
 // read again for the next shot of the tile.  49 floats per cell bound it: 256^3
-// 714 -> 657 us (2; 646 us, 5.1 TB/s, with the early loads below), 32
-// shots of 160x160x128: 4234 -> 4192 us (1; 4260 with 2).
+// 714 -> 657 us (2; 654 us, 5.0 TB/s, with the early loads below and the FP64
+// coefficients, 730 us with all 16 of them read), 32 shots of 160x160x128:
+// 4234 -> 4192 us (1; 4260 with 2).
 template <class G, bool VTI, int NT>
 __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_eu(QVTI_STRESSZ_WAVES))) void k2_stress_z(
     StressZArgs a)
@@ -1179,7 +1181,7 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
     const float* st = reinterpret_cast<const float*>(lds);
     const int pml = a.pml;
     const float dt = a.dt;
-    const float alpha = a.wab[0], s4 = a.wab[2];
+    const MediumConst med = *a.med;
     const int it = *a.it;
     const int kind = a.src_kind[shot];
     const long long sip = a.src_ip[shot];
@@ -1188,10 +1190,10 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
     const long long fbase = soff + cbase;    // per-shot natural fields
     const Row dxr = row_at(a.dxb, (long long)shot * kDer * a.blk_stride);
     const Row dyr = row_at(a.dyb, (long long)shot * kDer * a.blk_stride);
-    const Row g1r = row_at(a.g1, 0), g2r = row_at(VTI ? a.g2 : a.g1, 0);
-    Row gsr[kFam], sgr[6];
+    const Row gmr = row_at(a.gm, 0);
+    Row gsr[kGS(VTI)], sgr[6];
 #pragma unroll
-    for (int k = 0; k < kFam; ++k) gsr[k] = row_at(a.gs + k * a.N, cbase);
+    for (int k = 0; k < kGS(VTI); ++k) gsr[k] = row_at(a.gs + k * a.N, cbase);
 #pragma unroll
     for (int k = 0; k < 6; ++k) sgr[k] = row_at(a.sig[k], fbase);
     constexpr bool vti = VTI;  // G2 (H, D sets) present: a compile-time choice keeps the loads branch-free
@@ -1215,18 +1217,20 @@ __global__ __launch_bounds__(StressTile<G>::T) __attribute__((amdgpu_waves_per_e
             const unsigned ip = (unsigned)cbase + o;
             const unsigned blk = ip >> 6, in = ip & 63u;
             const unsigned od = lane_off(4u * (blk * (kBlk * kDer) + in));
-            const unsigned o1 = lane_off(4u * (blk * (kBlk * kG1) + in));
-            const unsigned o2 = lane_off(4u * (blk * (kBlk * kG2) + in));
+            const unsigned om = lane_off(4u * (blk * (kBlk * kGM(VTI)) + in));
             const unsigned oc = lane_off(4u * o);
             constexpr int FB = 4 * kBlk;  // bytes between the fields of a block
             float oP[kFam], oS[kFam], oH[kFam], oD[kFam];
             {
-                const float r = ld1<(NT > 1)>(g1r, o1, 4 * FB);
-                set_coeffs(oP, ld1<(NT > 1)>(g1r, o1), ld1<(NT > 1)>(g1r, o1, FB), r, alpha, s4);
-                set_coeffs(oS, ld1<(NT > 1)>(g1r, o1, 2 * FB), ld1<(NT > 1)>(g1r, o1, 3 * FB), r, alpha, s4);
+                auto gm = [&](int f) { return ld1<(NT > 1)>(gmr, om, f * FB); };
+                const int ps = __float_as_int(gm(GM_LOW));  // (the low half's sign is extended)
+                const double rho = gm(GM_RHO), gp = gm(GM_GP);
+                set_coeffs(oP, gm(GM_CP), (int)(short)ps, gp, rho, med);
+                set_coeffs(oS, gm(GM_CS), ps >> 16, gm(GM_GS), rho, med);
                 if (vti) {
-                    set_coeffs(oH, ld1<(NT > 1)>(g2r, o2), ld1<(NT > 1)>(g2r, o2, FB), r, alpha, s4);
-                    set_coeffs(oD, ld1<(NT > 1)>(g2r, o2, 2 * FB), ld1<(NT > 1)>(g2r, o2, 3 * FB), r, alpha, s4);
+                    const int hd = __float_as_int(ld1<(NT > 1)>(gsr[kFam], oc));
+                    set_coeffs(oH, gm(GM_CH), (int)(short)hd, gp, rho, med);
+                    set_coeffs(oD, gm(GM_CD), hd >> 16, gp, rho, med);
                 }
             }
             float A[14];

@@ -74,7 +74,11 @@ struct qvti_ctx {
     long long snap_lim = 0;      // floats this run may write: min(box * snapshots, snap_cap)
     // graphs
     bool use_graphs = true;
-    hipGraphExec_t gexec = nullptr;  // kGraphSteps steps of the current run
+    hipGraphExec_t gexec = nullptr;   // kGraphSteps steps of the current run
+    hipGraphExec_t gexec1 = nullptr;  // one step of it (qvti_step)
+    // host microseconds: return of the last qvti_step (0: none in this run), waits
+    // for the context since then, a step's direct launches when last measured
+    double host_end = 0.0, host_wait = 0.0, host_step = 0.0;
     // timing
     bool timing = false;
     int ev_max = 0, ev_used = 0;

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -177,10 +178,17 @@ static int upload(qvti_ctx* c, T** dst, const std::vector<T>& src)
     return QVTI_OK;
 }
 
+static void drop_graphs(qvti_ctx* c)
+{
+    for (hipGraphExec_t* g : {&c->gexec, &c->gexec1}) {
+        if (*g) hipGraphExecDestroy(*g);
+        *g = nullptr;
+    }
+}
+
 static void release(qvti_ctx* c)
 {
-    if (c->gexec) hipGraphExecDestroy(c->gexec);
-    c->gexec = nullptr;
+    drop_graphs(c);
     for (auto e : c->ev) hipEventDestroy(e);
     c->ev.clear();
     for (void* p : c->allocs) hipFree(p);
@@ -1004,17 +1012,17 @@ static void enqueue_step_with_snap(qvti_ctx* c)
 // the host's share low (a direct step takes it 20 us) at the direct speed.
 constexpr int kGraphSteps = 10;
 
-static int capture_graph(qvti_ctx* c)
+static int capture_graph(qvti_ctx* c, int steps, hipGraphExec_t* exec)
 {
     hipGraph_t graph = nullptr;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < kGraphSteps; ++k) enqueue_step_with_snap(c);
+    for (int k = 0; k < steps; ++k) enqueue_step_with_snap(c);
     hipError_t e = hipStreamEndCapture(c->stream, &graph);
     if (e != hipSuccess) return qvti_fail(QVTI_E_DEVICE, "graph capture failed: %s", hipGetErrorString(e));
-    e = hipGraphInstantiate(&c->gexec, graph, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
     hipGraphDestroy(graph);
     if (e != hipSuccess) {
-        c->gexec = nullptr;
+        *exec = nullptr;
         return qvti_fail(QVTI_E_DEVICE, "graph instantiate failed: %s", hipGetErrorString(e));
     }
     return QVTI_OK;
@@ -1053,10 +1061,8 @@ extern "C" int qvti_begin(qvti_ctx* c, int nt, const float* rik, const qvti_shot
     // the previous run's kernel arguments).
     c->begun = 0;
     c->steps_done = 0;
-    if (c->gexec) {
-        hipGraphExecDestroy(c->gexec);
-        c->gexec = nullptr;
-    }
+    drop_graphs(c);
+    c->host_end = 0.0;
     // (re)allocate run buffers
     auto realloc_dev = [&](void** p, size_t bytes) -> int {
         if (*p) {
@@ -1142,6 +1148,33 @@ extern "C" int qvti_begin(qvti_ctx* c, int nt, const float* rik, const qvti_shot
     return QVTI_OK;
 }
 
+static double host_us()
+{
+    return std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+
+// Counts a call's duration as a wait for the context (host_sets_pace).
+struct HostWait {
+    qvti_ctx* c;
+    double t0 = host_us();
+    explicit HostWait(qvti_ctx* ctx) : c(ctx) {}
+    ~HostWait() { c->host_wait += host_us() - t0; }
+};
+
+// Whether the host, and not the GPU, sets the pace of single steps: the caller
+// has been away from the context, its own waits aside, for longer than a step
+// takes to launch - it steps other contexts on this thread - and the step is
+// short.  Then the step goes as a graph of its own, which costs the GPU about 5
+// us more and the host 17 us instead of the 25 to 40 of 8 to 10 launches.  us a
+// step, direct / as a graph: eight contexts stepped in turn, 32^3 31 / 20,
+// 50x30x32 37 / 28, 48^3 31 / 28, 60^3 51 / 52, 64^3 46 / 47; one context, 48^3
+// 57 / 61, 64^3 69 / 74.  Same bits either way.
+static bool host_sets_pace(const qvti_ctx* c, double now)
+{
+    return c->host_end > 0.0 && c->host_step > 0.0 && c->N * c->nshots < (3LL << 16) &&
+           now - c->host_end - c->host_wait > c->host_step;
+}
+
 extern "C" int qvti_step(qvti_ctx* c, int nsteps)
 {
     if (!c) return qvti_fail(QVTI_E_ARG, "NULL context");
@@ -1150,6 +1183,16 @@ extern "C" int qvti_step(qvti_ctx* c, int nsteps)
         return qvti_fail(QVTI_E_ARG, "%d steps requested, %d of %d done", nsteps, c->steps_done, c->nt);
     HIPCHK(hipSetDevice(c->device));
     const long long nprobe = 3LL * c->S * c->N;
+    const double t0 = host_us();
+    bool one = c->use_graphs && !c->timing && host_sets_pace(c, t0);
+    if (one && !c->gexec1) {
+        one = c->nt - c->steps_done >= 2 * kGraphSteps;
+        if (one && capture_graph(c, 1, &c->gexec1)) {
+            c->use_graphs = one = false;
+            qvti_clear_error();
+        }
+    }
+    int direct = 0;
     for (const int end = c->steps_done + nsteps; c->steps_done < end;) {
         // steps until the next launch of the blow-up probe
         const int left = c->probe_every > 0 ? std::min(end - c->steps_done, c->probe_every - c->steps_done % c->probe_every)
@@ -1158,15 +1201,17 @@ extern "C" int qvti_step(qvti_ctx* c, int nsteps)
         if (graph && !c->gexec) {
             // worth capturing from the second group of steps on, for two groups or more
             graph = c->steps_done >= kGraphSteps && c->nt - c->steps_done >= 2 * kGraphSteps;
-            if (graph && capture_graph(c)) {
+            if (graph && capture_graph(c, kGraphSteps, &c->gexec)) {
                 c->use_graphs = graph = false;  // fall back to direct launches of the same kernels
                 qvti_clear_error();
             }
         }
-        if (graph)
-            HIPCHK(hipGraphLaunch(c->gexec, c->stream));
-        else
+        if (graph || one) {
+            HIPCHK(hipGraphLaunch(graph ? c->gexec : c->gexec1, c->stream));
+        } else {
             enqueue_step_with_snap(c);
+            ++direct;
+        }
         c->steps_done += graph ? kGraphSteps : 1;
         if (c->probe_every > 0 && (c->steps_done % c->probe_every == 0 || c->steps_done == c->nt)) {
             const int e0 = c->timing ? record_event(c, KC_PROBE) : -1;
@@ -1176,6 +1221,9 @@ extern "C" int qvti_step(qvti_ctx* c, int nsteps)
         }
     }
     HIPCHK(hipGetLastError());
+    c->host_end = host_us();
+    c->host_wait = 0.0;
+    if (nsteps > 0 && direct == nsteps && !c->timing) c->host_step = (c->host_end - t0) / nsteps;
     return QVTI_OK;
 }
 
@@ -1197,6 +1245,7 @@ static void harvest_events(qvti_ctx* c)
 extern "C" int qvti_sync(qvti_ctx* c)
 {
     if (!c) return qvti_fail(QVTI_E_ARG, "NULL context");
+    const HostWait wait(c);
     HIPCHK(hipSetDevice(c->device));
     HIPCHK(hipStreamSynchronize(c->stream));
     if (c->timing) harvest_events(c);
@@ -1294,6 +1343,7 @@ extern "C" int qvti_checkpoint(qvti_ctx* c, void* buf, long long capacity)
 {
     if (!c || !buf) return qvti_fail(QVTI_E_ARG, "NULL argument");
     if (!c->begun) return qvti_fail(QVTI_E_STATE, "no run in progress");
+    const HostWait wait(c);
     HIPCHK(hipSetDevice(c->device));
     HIPCHK(hipStreamSynchronize(c->stream));
     int probe = 0;
@@ -1358,6 +1408,7 @@ extern "C" int qvti_get_state(qvti_ctx* c, int shot, int field, float* out)
 {
     if (!c || !out) return qvti_fail(QVTI_E_ARG, "NULL argument");
     if (shot < 0 || shot >= c->S || field < 0 || field > 8) return qvti_fail(QVTI_E_ARG, "shot/field out of range");
+    const HostWait wait(c);
     HIPCHK(hipSetDevice(c->device));
     HIPCHK(hipStreamSynchronize(c->stream));
     const float* base = field < 3 ? fld(c->v, field, c) : fld(c->sig, field - 3, c);

@@ -43,3 +43,12 @@ def test_more_than_one_gpu_is_refused_before_any_device_work():
                        text=True, timeout=120)
     assert r.returncode == 2
     assert "one GPU" in r.stderr and r.stdout == ""
+
+
+def test_moved_bytes_are_those_of_the_launches():
+    """The step's achieved GB/s counts what its launches move, not the literal
+    scheme's bytes."""
+    kt = {"a": {"launches": 40, "total_ms": 1.0, "bytes_per_launch": 3.0},
+          "b": {"launches": 20, "total_ms": 1.0, "bytes_per_launch": 10.0},
+          "c": {"launches": 0, "total_ms": 0.0, "bytes_per_launch": 7.0}}
+    assert bench.moved_bytes(kt, 20) == 16.0

@@ -13,6 +13,8 @@
 #include "qvti_pencils.h"
 
 namespace qvti {
+// (KC_TICK and KC_RECORD keep the class order of qvti_kernel_times: the first
+// velocity kernel advances the step counter, k2_zrows takes the receivers)
 enum KClass {
     KC_TICK = 0, KC_VEL_X, KC_VEL_Y, KC_VEL_Z, KC_Y_FWD, KC_XPASS, KC_Y_INV, KC_Z_INV,
     KC_STR_X, KC_STR_Y, KC_STR_Z, KC_RECORD, KC_SNAP, KC_PROBE, KC_COUNT

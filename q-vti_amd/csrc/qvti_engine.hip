@@ -293,11 +293,13 @@ extern "C" int qvti_create(qvti_ctx** out, const qvti_grid* g, int max_shots, in
         c->snap_hi[a] = dims[a] - g->pml;
     }
     c->nrows = (long long)g->nx * g->ny;
-    // 1 / |k| at the Nyquist wavenumber of the finest axis, as a power of two:
-    // A3 v = L |k| v stays below v, with which it shares a transform, in any
-    // medium.  (Set from a frequency and 3000 m/s, a 300 m/s medium's A3 v was
-    // ten times v.)  The rounding of v in A3 v enters the stresses times
-    // gamma * cells per wavelength / 2.
+    // 1 / |k| at the Nyquist wavenumber of the finest axis, as the nearest power
+    // of two, in any medium: A3 v = L |k| v is at most sqrt(6) = 2.45 times v,
+    // with which it shares a transform (sqrt(2) from the rounding of L, sqrt(3)
+    // at the corner of the wavenumber cube; below v up to 0.4 of the corner).
+    // Half and a quarter of L gave the same errors.  (Set from a frequency and
+    // 3000 m/s, a 300 m/s medium's A3 v was ten times v.)  The rounding of v in
+    // A3 v enters the stresses times gamma * cells per wavelength / 2.
     c->L = exp2(round(log2(std::min({(double)g->dx, (double)g->dy, (double)g->dz}) / M_PI)));
     // When a z row does not end on a 128-byte line, neighbouring row tiles
     // and neighbouring planes share lines (and 64-cell blocks): run 8 row
@@ -745,7 +747,7 @@ static int record_event(qvti_ctx* c, int cls)
 // Workgroups per row tile of the final inverse z pass: 1 puts all fields in
 // one workgroup, any other value one field per workgroup.
 #ifndef QVTI_ZINV_SPLIT
-#define QVTI_ZINV_SPLIT 5
+#define QVTI_ZINV_SPLIT 4
 #endif
 
 // 1-D grid of the XCD-aware row kernels (tile_shot): ceil(ntiles/(8 run))*8 run*S.

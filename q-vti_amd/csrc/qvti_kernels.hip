@@ -103,11 +103,11 @@ constexpr int pencils()
     else return 0;
 }
 
-// Built at load time (dynamic initialisation), so that every launch function
-// whose address the record holds is instantiated and emitted.
 // tile widths PW of width index 0, 1, 2
 constexpr int kW0 = 1, kW1 = 2, kW2 = 4;
 
+// Built at load time (dynamic initialisation), so that every launch function
+// whose address the record holds is instantiated and emitted.
 template <int A, int B>
 LenOps make_ops()
 {

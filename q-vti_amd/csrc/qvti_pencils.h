@@ -28,8 +28,9 @@
 //    everywhere (q_coeffs in qvti_aux.h), so only A1 w and A3 v need the full
 //    3-D transform - three forward and four inverse complex transforms.  With
 //    five fields {A1 v, v, A3 v, A1 dv, dv} per component it was three and
-//    five, and 248 floats per cell and step through HBM instead of 188 (VTI,
-//    with the coefficients of set_coeffs and the shear sums of k2_stress_xy).
+//    five, and 248 floats per cell and step instead of 188 (VTI, with the
+//    coefficients of set_coeffs and the shear sums of k2_stress_xy, each field
+//    of a launch counted once; 196 with the second reads of S-bar there).
 //    Fields that share a complex transform are scaled (alpha and the length
 //    scale of A1 and A3, powers of two) so that the FP32 rounding of one does
 //    not swamp the other where it matters (q_coeffs).
@@ -294,7 +295,8 @@ void k2_deriv_strided(StridedPair pr)
 //   sum_j S-bar_j D(in_j)
 // of the component's four derivatives, the only form in which the stress
 // update uses the shear derivatives: six fields per axis go to HBM and back
-// instead of twelve, for four coefficient reads (24 -> 22 floats per cell here,
+// instead of twelve, for four coefficient fields that each of the two sums
+// reads (24 -> 26 floats per cell and axis here, 22 with S-bar counted once;
 // 61 -> 49 in the stress update).  Pairing fields, and not two columns of one
 // field as k2_deriv_strided does, halves the passes of a sum and the
 // accumulators that live through the transforms (N1 instead of 2 N1 registers).
@@ -328,13 +330,17 @@ struct StressXYPair {
     int nshots;         // shots interleaved on grid x, or 1
 };
 
-// NT: non-temporal field loads and stores (stream_nt)
-template <class G, bool NT>
+// NT: non-temporal field loads and stores (stream_nt).
 // What bounds it: 52 floats per cell for both axes (each sum reads S-bar).
-// 256^3: 687 us, 5.1 TB/s, the rate of the memory at 20 streams; 400x400x200:
+// 256^3: 680 us, 5.1 TB/s, the rate of the memory at 20 streams; 400x400x200:
 // 1790 us, 3.7 TB/s, 3 waves per SIMD and rows that end mid-line.  The bounds:
 // one axis at 256^3, before the streaming, took 370-375 us with 2, 3 and 4
 // waves per SIMD; at 400x400x200 3 waves were best (985 us; 1045 us with 2).
+// Some splits spill under them: 256 and 240 up to 6 VGPRs, 480 to 512 from 5 to
+// 73 by tile width; other bounds were not timed there.  A whole step of
+// 480x480x32, 500x500x32, 512x512x128 takes 1.39, 1.68, 6.76 ms (1.96, 2.12,
+// 7.77 ms when every derivative was stored).
+template <class G, bool NT>
 __global__ __launch_bounds__(G::T) __attribute__((amdgpu_waves_per_eu(G::NMAX <= 16 ? 4 : 3)))
 void k2_stress_xy(StressXYPair pr)
 {

@@ -81,6 +81,7 @@ struct qvti_ctx {
     // host microseconds: return of the last qvti_step (0: none in this run), waits
     // for the context since then, a step's direct launches when last measured
     double host_end = 0.0, host_wait = 0.0, host_step = 0.0;
+    int host_away = 0;  // calls of qvti_step in a row that host_sets_pace held for
     // timing
     bool timing = false;
     int ev_max = 0, ev_used = 0;

@@ -1065,6 +1065,7 @@ extern "C" int qvti_begin(qvti_ctx* c, int nt, const float* rik, const qvti_shot
     c->steps_done = 0;
     drop_graphs(c);
     c->host_end = 0.0;
+    c->host_away = 0;
     // (re)allocate run buffers
     auto realloc_dev = [&](void** p, size_t bytes) -> int {
         if (*p) {
@@ -1186,7 +1187,9 @@ extern "C" int qvti_step(qvti_ctx* c, int nsteps)
     HIPCHK(hipSetDevice(c->device));
     const long long nprobe = 3LL * c->S * c->N;
     const double t0 = host_us();
-    bool one = c->use_graphs && !c->timing && host_sets_pace(c, t0);
+    // (two calls in a row: a migration is away from its receiver context once a segment)
+    c->host_away = host_sets_pace(c, t0) ? c->host_away + 1 : 0;
+    bool one = c->use_graphs && !c->timing && c->host_away > 1;
     if (one && !c->gexec1) {
         one = c->nt - c->steps_done >= 2 * kGraphSteps;
         if (one && capture_graph(c, 1, &c->gexec1)) {

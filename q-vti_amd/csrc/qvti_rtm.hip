@@ -129,6 +129,15 @@ __global__ __launch_bounds__(256) void k_img_exa(float* img, const float* smax, 
         if (tex[i] == t && fabsf(smax[i]) > thr) img[i] += field_at(r, i) / smax[i];
 }
 
+// One step of a run whose caller launches more on the stream after each: those
+// launches may wait for the GPU, so the time until the next step does not tell
+// that the host sets the pace (qvti_step).
+int step_one(qvti_ctx* c)
+{
+    c->host_end = 0.0;
+    return qvti_step(c, 1);
+}
+
 unsigned grid_for(long long N) { return (unsigned)std::min<long long>((N + 255) / 256, 65535LL * 4); }
 
 }  // namespace
@@ -223,7 +232,7 @@ extern "C" int qvti_rtm(qvti_ctx* cs, qvti_ctx* cr, int nt, const float* rik, co
         }
         if (exa) {
             for (int t = t0; t < t1 && !rc; ++t) {
-                rc = qvti_step(cs, 1);
+                rc = step_one(cs);
                 hipLaunchKernelGGL(k_exa_track, dim3(gN), dim3(256), 0, cs->stream, d_smax, d_tex, fs, t, N);
             }
         } else {
@@ -257,7 +266,7 @@ extern "C" int qvti_rtm(qvti_ctx* cs, qvti_ctx* cr, int nt, const float* rik, co
             if (rc) break;
             RTMCHK(hipStreamWaitEvent(cs->stream, used[b], 0));
             for (int t = t0; t < t1 && !rc; ++t) {
-                rc = qvti_step(cs, 1);
+                rc = step_one(cs);
                 hipLaunchKernelGGL(k_field_copy, dim3(gN), dim3(256), 0, cs->stream, seg + (size_t)(t - t0) * N, fs, N);
             }
             if (rc) break;
@@ -265,7 +274,7 @@ extern "C" int qvti_rtm(qvti_ctx* cs, qvti_ctx* cr, int nt, const float* rik, co
             RTMCHK(hipStreamWaitEvent(cr->stream, ready[b], 0));
         }
         for (int t = t1 - 1; t >= t0 && !rc; --t) {
-            rc = qvti_step(cr, 1);
+            rc = step_one(cr);
             if (rc) break;
             InjArgs ia;
             for (int c = 0; c < 3; ++c) {

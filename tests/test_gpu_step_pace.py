@@ -52,7 +52,7 @@ def test_contexts_stepped_in_turn_give_the_same_bits(n, contexts, read):
     """With several contexts in turn a step goes as a graph of its own, with one
     by direct launches: records and states equal those of direct launches
     (set_graphs(False)) in both, with readbacks between the replays too.  The
-    times are printed only: the host's share differs from box to box (32^3,
+    times are printed only: the host's share differs between machines (32^3,
     eight contexts, direct / graph: 31 / 20 us and 23 / 19.5 us)."""
     direct, want = _run(n, False, contexts, read)
     us, got = _run(n, True, contexts, read)

@@ -10,12 +10,12 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nx,ny,nz", [(400, 400, 50), (500, 500, 32)])
-def test_tuning_costs_at_most_twelve_steps(nx, ny, nz):
+def test_tuning_costs_less_than_a_short_run(nx, ny, nz):
     """Every tile candidate of the strided kernels is launched on the grid
-    itself before the first run.  They take about 0.6 of a step, six candidates
+    itself before the first run.  They take 0.6 to 0.8 of a step, six candidates
     each at these lengths: four launches for the first one and two for the
-    others are 14 x 0.6 = 8.4 steps, four for each were 14.4.  The bound lies
-    between."""
+    others are 14 x 0.6 = 8.4 to 14 x 0.8 = 11.2 steps, four for each 14.4 to
+    19.2.  The bound lies in the gap."""
     f = lambda v: np.full((nx, ny, nz), v, np.float32)  # noqa: E731
     model = dict(vp=f(3000), vs=f(1700), rho=f(2200), gp=f(0.005), gs=f(0.01))
     shot = qvti.make_shot(qvti.SRC_FZ, (nx // 2, ny // 2, nz // 2), [], [], [])
@@ -37,4 +37,4 @@ def test_tuning_costs_at_most_twelve_steps(nx, ny, nz):
             step = (time.perf_counter() - t0) / 20
         ratio.append((t[0] - t[1]) / step)
     print("%dx%dx%d: tuning takes %s steps of %.2f ms" % (nx, ny, nz, ["%.1f" % r for r in ratio], step * 1e3))
-    assert min(ratio[1:]) < 12.0  # (the first context also loads the kernels)
+    assert min(ratio[1:]) < 13.0  # (the first context also loads the kernels)
